@@ -18,7 +18,7 @@
 //   * shell pairs sorted by class (la lb), la >= lb, then by Schwarz bound descending;
 //   * primitive pairs (PrimPair, 96 B AoS) referenced by pair ranges;
 //   * Boys table F_m(T_i) (361 x 25 doubles);
-//   * per call: Cartesian densities (row-major, ncart^2), forward J/K accumulators,
+//   * per call: Cartesian densities (row-major, ncart^2), forward J (pair order) and K accumulators,
 //     (plus transposed-density accumulators used only for a non-symmetric X),
 //     compacted quartet task lists per class pair (uint2 {bra pair, ket pair}).
 //
@@ -482,28 +482,50 @@ __global__ void cart_density_kernel(const double* __restrict__ X, int n, int ld,
   Dc[k] = sk;
 }
 
-// AX_i[mu + nu*ld] += f_i * sum_{a,c} T(mu,a) T(nu,c) (G1_i[a][c] + G2_i[c][a]) for every
-// matrix i of the call, G2_i = G1_i unless the density was flagged non-symmetric.
+// AX_i[mu + nu*ld] += f_i * sum_{a,c} T(mu,a) T(nu,c) (G_i[a][c] + G'_i[c][a]) for every matrix
+// i of the call.  Exchange: the updates are in A (as they are) and B (transposed), G = A + B^T,
+// and G' = G for a symmetric density; for a non-symmetric one B holds the updates from the
+// transposed density as well and G' adds nothing.  Coulomb: A holds G(s1,s2) of the canonical
+// blocks in pair order (jtab), G' = G, or the matrix B for a non-symmetric density.
 struct FinList {
   double* AX[MAX_MATS];
-  const double* G1[MAX_MATS];
-  const double* G2alt[MAX_MATS];
+  const double* A[MAX_MATS];
+  const double* B[MAX_MATS];
   const int* nonsym[MAX_MATS];
+  int coulomb[MAX_MATS];
   double f[MAX_MATS];
   int n;
 };
+// Coulomb list offsets by ordered shell pair: element (i of s, j of t) is at
+// jtab + i * ncart(t) + j, or, for a pair held as (t, s) (code negated), at
+// ~jtab + j * ncart(s) + i; JTAB_NONE: the pair has no two-electron list entry.
+#define JTAB_NONE 0x7fffffff
+__global__ void jtab_kernel(const PairInfo* __restrict__ pairs, int npair, int nshell, int* __restrict__ jtab) {
+  const int P = blockIdx.x * blockDim.x + threadIdx.x;
+  if (P >= npair) return;
+  const PairInfo p = pairs[P];
+  jtab[(long)p.b * nshell + p.a] = ~p.joff;
+  jtab[(long)p.a * nshell + p.b] = p.joff;   // (last: the one code of a pair of one shell)
+}
+__global__ void jtab_clear_kernel(long n, int* __restrict__ jtab) {
+  for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x)
+    jtab[k] = JTAB_NONE;
+}
 __global__ void finalize_kernel(FinList fl, int n, int ld, const ShellMeta* __restrict__ sh,
-                                const int* __restrict__ sph2shell, int ncart,
+                                const int* __restrict__ sph2shell, int ncart, const int* __restrict__ jtab, int nshell,
                                 const double* __restrict__ tco, const int* __restrict__ tco_off) {
   const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= (long)n * n) return;
   const int mu = k % n, nu = k / n;
-  const ShellMeta A = sh[sph2shell[mu]], B = sh[sph2shell[nu]];
+  const int sa = sph2shell[mu], sb = sph2shell[nu];
+  const ShellMeta A = sh[sa], B = sh[sb];
   const int im = mu - A.sph_off, in = nu - B.sph_off;
   const int nca = (A.l + 1) * (A.l + 2) / 2, ncb = (B.l + 1) * (B.l + 2) / 2;
+  const int jc = jtab[(long)sa * nshell + sb];
   for (int i = 0; i < fl.n; ++i) {
-    const double* G1 = fl.G1[i];
-    const double* g2 = *fl.nonsym[i] ? fl.G2alt[i] : G1;
+    const double* GA = fl.A[i];
+    const double* GB = fl.B[i];
+    const bool ns = *fl.nonsym[i] != 0;
     double s = 0.0;
     for (int a = 0; a < nca; ++a) {
       const double ta = tcoef(A, im, a, tco, tco_off);
@@ -511,8 +533,21 @@ __global__ void finalize_kernel(FinList fl, int n, int ld, const ShellMeta* __re
       for (int c = 0; c < ncb; ++c) {
         const double tc = tcoef(B, in, c, tco, tco_off);
         if (tc == 0.0) continue;
-        const long ia = A.cart_off + a, ic = B.cart_off + c;
-        s += ta * tc * (G1[ia * ncart + ic] + g2[ic * ncart + ia]);
+        const long ac = (long)(A.cart_off + a) * ncart + B.cart_off + c;
+        const long ca = (long)(B.cart_off + c) * ncart + A.cart_off + a;
+        double g = 0.0;
+        if (fl.coulomb[i]) {
+          if (jc != JTAB_NONE) {
+            const double v = GA[jc >= 0 ? jc + a * ncb + c : ~jc + c * nca + a];
+            if (!ns) g = sa == sb ? v + GA[jc + c * ncb + a] : v;
+            else if (sa >= sb) g = v;
+          }
+          if (ns) g += GB[ca];
+        } else {
+          g = GA[ac] + GB[ca];
+          if (!ns) g += GA[ca] + GB[ac];
+        }
+        s += ta * tc * g;
       }
     }
     fl.AX[i][(long)nu * ld + mu] += fl.f[i] * s;
@@ -852,7 +887,7 @@ struct cq_ctx {
   DevBuf<double> d_alpha, d_coef, d_origin, d_onee;
   // device
   DevBuf<ShellMeta> d_shells;
-  DevBuf<int> d_cart2shell, d_sph2shell, d_tco_off, d_flags;
+  DevBuf<int> d_cart2shell, d_sph2shell, d_tco_off, d_flags, d_jtab;
   DevBuf<double> d_tco, d_boys, d_pairQ, d_Nmax, d_Npair, d_work, d_mats;
   DevBuf<PairInfo> d_pairs, d_pairs_1e;
   std::vector<PairInfo> pairs_1e_h;   // host copies kept for the asynchronous uploads
@@ -897,7 +932,7 @@ struct cq_ctx {
   std::string err;
 
   ~cq_ctx() {
-    d_shells.release(); d_cart2shell.release(); d_sph2shell.release(); d_tco_off.release();
+    d_shells.release(); d_cart2shell.release(); d_sph2shell.release(); d_tco_off.release(); d_jtab.release();
     d_uorder.release(); d_groups[0].release(); d_groups[1].release(); d_flags.release(); d_tco.release(); d_boys.release(); d_pairQ.release();
     d_Nmax.release(); d_Npair.release(); d_work.release(); d_mats.release(); d_pairs.release(); d_pairs_1e.release(); d_prims.release();
     d_cps[0].release(); d_cps[1].release(); d_tasks.release(); d_segs.release(); d_work_q.release(); d_ovf.release(); d_qcounts.release(); d_nglob.release(); d_pair_nblk.release(); d_pair_nublk.release();
@@ -1198,10 +1233,9 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
   for (int s = 0; s < nshell; ++s) {
     if (l[s] < 0 || l[s] > 2) throw std::invalid_argument("shell angular momentum above d is not supported");
     if (nprim[s] < 1) throw std::invalid_argument("shell with no primitives");
-    c->shells[s] = ShellMeta{l[s], pure[s] ? 1 : 0, sph, cart};
+    c->shells[s] = ShellMeta{l[s], pure[s] ? 1 : 0, sph, 0};
     const int nsz = pure[s] ? 2 * l[s] + 1 : ncart_l(l[s]);
     for (int k = 0; k < nsz; ++k) c->sph2shell.push_back(s);
-    for (int k = 0; k < ncart_l(l[s]); ++k) c->cart2shell.push_back(s);
     sph += nsz;
     cart += ncart_l(l[s]);
     poff[s + 1] = poff[s] + nprim[s];
@@ -1223,8 +1257,23 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     }
   }
   c->nmol = nshell > 0 ? c->shell_mol[nshell - 1] + 1 : 1;
+  // Cartesian functions by molecule, then angular momentum, then shell: the functions of a pair
+  // class's shells (an LDS accumulator's rows) are then at most two runs of consecutive
+  // functions, so the accumulators' flushes and the digestion's reads of the density along them
+  // are coalesced
+  std::vector<int> cart_order(nshell);
+  std::iota(cart_order.begin(), cart_order.end(), 0);
+  std::stable_sort(cart_order.begin(), cart_order.end(), [&](int x, int y) {
+    return c->shell_mol[x] != c->shell_mol[y] ? c->shell_mol[x] < c->shell_mol[y] : l[x] < l[y];
+  });
   std::vector<int> mol_cart0(c->nmol + 1, cart);
-  for (int s = nshell - 1; s >= 0; --s) mol_cart0[c->shell_mol[s]] = c->shells[s].cart_off;
+  for (int k = 0, off = 0; k < nshell; ++k) {
+    const int s = cart_order[k];
+    if (k == 0 || c->shell_mol[s] != c->shell_mol[cart_order[k - 1]]) mol_cart0[c->shell_mol[s]] = off;
+    c->shells[s].cart_off = off;
+    c->cart2shell.insert(c->cart2shell.end(), ncart_l(l[s]), s);
+    off += ncart_l(l[s]);
+  }
   c->npc = 6;   // ss ps pp ds dp dd
   // LDS rows per pair class: shell s's first row among the functions of its molecule's shells
   // with angular momentum in {la, lb} (crow, -1 outside the set), and the inverse map
@@ -1237,8 +1286,9 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
         const int pc = pair_class(la, lb);
         c->lds_n_set[pc] = 0;
         int r = 0;
-        for (int sh = 0; sh < nshell; ++sh) {
-          if (sh > 0 && c->shell_mol[sh] != c->shell_mol[sh - 1]) r = 0;
+        for (int k = 0; k < nshell; ++k) {
+          const int sh = cart_order[k];
+          if (k > 0 && c->shell_mol[sh] != c->shell_mol[cart_order[k - 1]]) r = 0;
           if (l[sh] != la && l[sh] != lb) continue;
           crow[(size_t)pc * nshell + sh] = r;
           const int nf = (l[sh] + 1) * (l[sh] + 2) / 2;
@@ -1362,10 +1412,13 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
   // (allprim, uploaded once), the pair pointing at its range
   auto flatten = [&]() {
     c->pairs.resize(hp.size());
+    int joff = 0;   // at most ncart^2 < 2^31 elements: each ordered shell pair at most once
     for (size_t k = 0; k < hp.size(); ++k) {
       PairInfo pi_ = hp[k].info;
       pi_.p0 = (int)hp[k].off;
       pi_.p1 = (int)(hp[k].off + hp[k].n);
+      pi_.joff = joff;
+      joff += ncart_l(l[pi_.a]) * ncart_l(l[pi_.b]);
       c->pairs[k] = pi_;
     }
   };
@@ -1480,6 +1533,15 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
   flatten();
   c->d_pairs.upload(c->pairs, c->stream);
   c->d_pairQ.upload(c->pairQ, c->stream);
+  {
+    const long ns2 = (long)nshell * nshell;
+    c->d_jtab.ensure((size_t)ns2);
+    hipLaunchKernelGGL(jtab_clear_kernel, dim3((int)std::min<long>(1024, grid_for(ns2, WG))), dim3(WG), 0, c->stream, ns2,
+                       c->d_jtab.p);
+    hipLaunchKernelGGL(jtab_kernel, dim3(grid_for(npair, WG)), dim3(WG), 0, c->stream, c->d_pairs.p, npair, nshell,
+                       c->d_jtab.p);
+    HIPCHK(hipGetLastError());
+  }
   // primitive-count groups per class: grp[cls_grp_off[X] .. cls_grp_off[X+1]] are the group
   // starts (class-local), closed by the class size
   c->cls_grp_off.assign(c->npc + 1, 0);
@@ -1886,22 +1948,23 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   }
   }
   // 5. back to the shells' basis and accumulate, every matrix in one launch:
-  //    AX += 1/2 scale (G + G'^T); COULOMB G = GJ, G' = (nonsym ? GJ2 : GJ); EXCHANGE with GK/GK2
+  //    AX += 1/2 scale (G + G'^T) (finalize_kernel)
   FinList fl{};
   for (int i = 0; i < nmat; ++i) {
     const int k = mat_slot[i];
     if (k < 0) continue;
     double* base = work + (size_t)k * 5 * nc2;
     fl.AX[fl.n] = AX[i];
-    fl.G1[fl.n] = base + (types[i] == CQ_COULOMB ? 1 : 3) * nc2;
-    fl.G2alt[fl.n] = base + (types[i] == CQ_COULOMB ? 2 : 4) * nc2;
+    fl.coulomb[fl.n] = types[i] == CQ_COULOMB;
+    fl.A[fl.n] = base + (types[i] == CQ_COULOMB ? 1 : 3) * nc2;
+    fl.B[fl.n] = base + (types[i] == CQ_COULOMB ? 2 : 4) * nc2;
     fl.nonsym[fl.n] = flags + k;
     fl.f[fl.n] = 0.5 * scales[i];
     ++fl.n;
   }
   if (fl.n > 0) {
     hipLaunchKernelGGL(finalize_kernel, dim3(grid_for((long)n * n, WG)), dim3(WG), 0, s, fl, n, ld, c->d_shells.p,
-                       c->d_sph2shell.p, c->ncart, c->d_tco.p, c->d_tco_off.p);
+                       c->d_sph2shell.p, c->ncart, c->d_jtab.p, ns, c->d_tco.p, c->d_tco_off.p);
     HIPCHK(hipGetLastError());
   }
 }

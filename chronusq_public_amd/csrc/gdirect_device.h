@@ -37,6 +37,7 @@ struct PairInfo {
   int loff;        // first Cartesian function of the pair's molecule (0 for one molecule)
   int ar, br;      // first LDS row of a and b: their place among the functions of the
                    // molecule's shells whose angular momentum is la or lb (the pair's class)
+  int joff;        // first element of the pair's na x nb block in the pair-ordered Coulomb list
 };
 
 struct QuartetArgs {
@@ -57,10 +58,15 @@ struct JKArgs {
                                  // molecule's functions of the swept pair class's shells
   const int* rowfn;              // Cartesian function of LDS row r: rowfn[loff + r]
   const double* D[MAX_SLOTS];    // density in the Cartesian basis, row-major ncart x ncart
-  double* GJ[MAX_SLOTS];         // forward Coulomb updates
-  double* GJ2[MAX_SLOTS];        // forward Coulomb updates from the transposed density
-  double* GK[MAX_SLOTS];         // forward exchange updates
-  double* GK2[MAX_SLOTS];        // forward exchange updates from the transposed density
+  // Accumulators.  An FP64 atomic whose wavefront hits 64 consecutive doubles runs at 163 G/s
+  // for the whole chip, at scattered or strided addresses at 23 G/s (measured on 160000
+  // doubles), so the LDS flushes address memory along their lanes: J in pair order, the K
+  // columns of the ket-keyed kernels transposed.
+  double* GJ[MAX_SLOTS];         // forward Coulomb updates, pair order (PairInfo::joff)
+  double* GJ2[MAX_SLOTS];        // Coulomb updates from the transposed density (matrix, added transposed)
+  double* GK[MAX_SLOTS];         // forward exchange updates (matrix)
+  double* GK2[MAX_SLOTS];        // exchange updates held transposed: the ket-keyed kernels' K columns
+                                 // and the updates from the transposed density (matrix)
   int do_j[MAX_SLOTS];
   int do_k[MAX_SLOTS];
   const int* nonsym;             // device flags: density slot is not symmetric

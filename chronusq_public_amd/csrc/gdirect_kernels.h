@@ -110,23 +110,6 @@ __device__ __forceinline__ long next_item(unsigned* __restrict__ work, int* s_it
   return (long)__builtin_amdgcn_readfirstlane(*s_item);
 }
 
-// Coulomb block (1,2) of a pair held in kernel orientation: address of element (i, j), i a
-// component of its a shell, j of its b shell, in the canonical order (s1, s2).
-__device__ __forceinline__ long jaddr(const PairInfo& P, int N, int i, int j) {
-  const bool sw = P.a != P.s1;
-  return sw ? (long)(P.b0 + j) * N + P.a0 + i : (long)(P.a0 + i) * N + P.b0 + j;
-}
-// The same address kept in one int while a swept pair's J slot fills: element (0, 0) of the
-// block, bitwise negated when the pair is held swapped (the context keeps N^2 < 2^31).
-__device__ __forceinline__ int jcode(const PairInfo& P, int N) {
-  const bool sw = P.a != P.s1;
-  const int a00 = sw ? P.b0 * N + P.a0 : P.a0 * N + P.b0;
-  return sw ? ~a00 : a00;
-}
-__device__ __forceinline__ long jcode_addr(int code, int N, int i, int j) {
-  return code < 0 ? (long)(~code) + (long)j * N + i : (long)code + (long)i * N + j;
-}
-
 // Group kernels.  Work items are (task region, group of cpi chunks) pairs from an atomic queue
 // (cpi divides the class pair's chunk count); each workgroup spreads the item's (chunk, member,
 // block of 64 of that member's entries) units over its wavefronts -- the member wavefront-
@@ -136,8 +119,13 @@ __device__ __forceinline__ long jcode_addr(int code, int N, int i, int j) {
 //    every union bra;
 //  * bra-keyed (eri_grpb, DIG 2): K rows of the shared a shell and of every member's b shell,
 //    J(a, b_m) of every member, and J of every union ket.
+// The flush's lanes walk consecutive LDS words, i.e. consecutive Cartesian functions of one K
+// column or row (functions are ordered by angular momentum within a molecule, so a swept class's
+// functions are one or two runs) and consecutive elements of the pair-ordered J list: whole
+// cache lines per atomic instruction ((H2O)16/cc-pVDZ, (ss|ps): 7.7 M atomics per launch, at
+// 23 G/s scattered 0.33 of its 0.57 ms).
 // Dynamic LDS, ket-keyed: [(NC + mmax ND) LN K columns (DIG 1)][mmax NC ND J(c,d)][ub NA NB J slots]
-//                         [ub ints: the J address code of each slot's swept pair]
+//                         [ub ints: PairInfo::joff of each slot's swept pair]
 //              bra-keyed: [(NA + mmax NB) LN K rows][mmax NA NB J(a,b)][ub NC ND J slots][ub ints]
 #define DEFINE_CLASS_KERNELS(NAME, LTOT)                                                        \
   template <int WGS, int DIG, typename R>                                                     \
@@ -195,7 +183,7 @@ __device__ __forceinline__ long jcode_addr(int code, int N, int i, int j) {
         const bool active = t < s_mcnt[mu];                                                   \
         const uint2 e = reg[s_moff[mu] + (active ? t : b0)];                                  \
         const PairInfo B = pairs[pair_of(e.x)];                                               \
-        if (active) spair[e.y] = jcode(B, N);                                                 \
+        if (active) spair[e.y] = B.joff;                                                      \
         const unsigned kk = __builtin_amdgcn_readfirstlane((unsigned)uorder[gr.first + mu]);  \
         QuartetArgs q;                                                                        \
         make_quartet_uniform_ket(B, e.x, kk, kblk, active, pairs, prims, q);                  \
@@ -211,7 +199,7 @@ __device__ __forceinline__ long jcode_addr(int code, int N, int i, int j) {
             const int col = k / LN, row = jk.rowfn[K0.loff + k - col * LN];                   \
             const int md = (col - NC) / ND;                                                   \
             const int gcol = col < NC ? K0.a0 + col : s_dcol[md] + (col - NC - md * ND);       \
-            atomicAdd(&jk.GK[0][(long)row * N + gcol], v);                                    \
+            atomicAdd(&jk.GK2[0][(long)gcol * N + row], v);                                   \
             colK[k] = 0.0;                                                                    \
           }                                                                                   \
         }                                                                                     \
@@ -219,16 +207,16 @@ __device__ __forceinline__ long jcode_addr(int code, int N, int i, int j) {
       for (int k = threadIdx.x; k < n * NCD; k += WGS) {                                      \
         const double v = jcdL[k];                                                             \
         if (v != 0.0) {                                                                       \
-          const int m = k / NCD, ic = (k - m * NCD) / ND, idd = k - m * NCD - ic * ND;        \
-          atomicAdd(&jk.GJ[0][jaddr(pairs[uorder[gr.first + m]], N, ic, idd)], v);            \
+          const int m = k / NCD;                                                              \
+          atomicAdd(&jk.GJ[0][pairs[uorder[gr.first + m]].joff + k - m * NCD], v);            \
           jcdL[k] = 0.0;                                                                      \
         }                                                                                     \
       }                                                                                       \
       for (int k = threadIdx.x; k < U * NAB; k += WGS) {                                      \
         const double v = jsl[k];                                                              \
         if (v != 0.0) {                                                                       \
-          const int u = k / NAB, ia = (k - u * NAB) / NB, ib = k - u * NAB - ia * NB;         \
-          atomicAdd(&jk.GJ[0][jcode_addr(spair[u], N, ia, ib)], v);                           \
+          const int u = k / NAB;                                                              \
+          atomicAdd(&jk.GJ[0][spair[u] + k - u * NAB], v);                                    \
           jsl[k] = 0.0;                                                                       \
         }                                                                                     \
       }                                                                                       \
@@ -315,7 +303,7 @@ __device__ __forceinline__ long jcode_addr(int code, int N, int i, int j) {
         const bool active = t < s_mcnt[mu];                                                     \
         const uint2 e = reg[s_moff[mu] + (active ? t : b0)];                                    \
         const PairInfo K = pairs[pair_of(e.x)];                                                 \
-        if (active) spair[e.y] = jcode(K, N);                                                   \
+        if (active) spair[e.y] = K.joff;                                                        \
         const unsigned bb = __builtin_amdgcn_readfirstlane((unsigned)uorder[gr.first + mu]);    \
         QuartetArgs q;                                                                          \
         make_quartet_uniform_bra(K, e.x, bb, bblk, active, pairs, prims, q);                    \
@@ -337,16 +325,16 @@ __device__ __forceinline__ long jcode_addr(int code, int N, int i, int j) {
       for (int k = threadIdx.x; k < n * NAB; k += WG) {                                         \
         const double v = jabL[k];                                                               \
         if (v != 0.0) {                                                                         \
-          const int m = k / NAB, ia = (k - m * NAB) / NB, ib = k - m * NAB - ia * NB;           \
-          atomicAdd(&jk.GJ[0][jaddr(pairs[uorder[gr.first + m]], N, ia, ib)], v);               \
+          const int m = k / NAB;                                                                \
+          atomicAdd(&jk.GJ[0][pairs[uorder[gr.first + m]].joff + k - m * NAB], v);              \
           jabL[k] = 0.0;                                                                        \
         }                                                                                       \
       }                                                                                         \
       for (int k = threadIdx.x; k < U * NCD; k += WG) {                                         \
         const double v = jsl[k];                                                                \
         if (v != 0.0) {                                                                         \
-          const int u = k / NCD, ic = (k - u * NCD) / ND, idd = k - u * NCD - ic * ND;          \
-          atomicAdd(&jk.GJ[0][jcode_addr(spair[u], N, ic, idd)], v);                            \
+          const int u = k / NCD;                                                                \
+          atomicAdd(&jk.GJ[0][spair[u] + k - u * NCD], v);                                      \
           jsl[k] = 0.0;                                                                         \
         }                                                                                       \
       }                                                                                         \
