@@ -11,6 +11,7 @@ import argparse
 import concurrent.futures as cf
 import glob
 import os
+import re
 import subprocess
 import sys
 
@@ -59,8 +60,11 @@ def build(incremental: bool = False, resource_usage: bool = False, jobs: int = 0
         todo.append((s, o))
     jobs = jobs or min(len(todo) or 1, os.cpu_count() or 4, 16)
     logs = {}
-    # the biggest units first so the tail stays short
-    todo.sort(key=lambda so: -os.path.getsize(so[0]))
+    # the biggest units (with the generated headers they include) first so the tail stays short
+    def weight(src):
+        text = open(src).read()
+        return len(text) + sum(os.path.getsize(os.path.join(GEN, h)) for h in set(re.findall(r'#include "(cls_\w+\.h)"', text)))
+    todo.sort(key=lambda so: -weight(so[0]))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         futs = {ex.submit(_compile, s, o, extra): s for s, o in todo}
         for f in cf.as_completed(futs):

@@ -46,10 +46,11 @@
 #include "_gen/eri_registry.inc"
 
 static ClassKernels kClassKernels[CQ_NUM_CLASS_PAIRS];
+static MergedTier kMergedTiers[CQ_NUM_TIERS];
 #define MAX_MATS 8   // matrices of one contraction
 // dynamic LDS of the group kernels: what the 64 KiB per workgroup leaves beside the static
-// LDS (Boys table, 25992 B, the work-item slot and the members' column offsets)
-static const size_t kStaticLds = BOYS_NGRID * BOYS_LDS_W * sizeof(double) + 256;
+// LDS (Boys table, 26064 B, the work item's members)
+static const size_t kStaticLds = BOYS_ROWS * BOYS_LDS_W * sizeof(double) + 384;
 static const size_t kMaxDynLds = 64 * 1024 - kStaticLds;
 
 // Dynamic LDS the group kernels may use on this device: the device's per-workgroup limit
@@ -76,20 +77,27 @@ static size_t device_dyn_lds() {
         }
       }
     }
+    for (const MergedTier& t : kMergedTiers)
+      if (hipFuncSetAttribute((const void*)t.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)want) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+      }
     v = want;
   });
   return v;
 }
 static const int kNumClassPairs = CQ_NUM_CLASS_PAIRS;
-static const bool kClassKernelsReady = (cq_register_all(kClassKernels), true);
+static const bool kClassKernelsReady = (cq_register_all(kClassKernels), cq_merged_all(kMergedTiers), true);
 
-// Per-call workspace of cq_contract_direct_device_noalloc: the Cartesian density and the four
-// J/K accumulators of every density slot, then the slots' symmetry flags.  One copy per device,
+// Per-call workspace of cq_contract_direct_device_noalloc: the Cartesian density's copies and the
+// four J/K accumulators of every density slot, then the slots' symmetry flags.  One copy per device,
 // held until the process ends; every call on a device shares it, so calls that overlap on one
 // device race.  Host code never uses the array's name as an address: the device address comes
 // from hipGetSymbolAddress, resolved once per device at context creation (scratch_address).
+// A call is accepted while 5 ncart^2 doubles per density (and a flag each) fit the limit; the
+// array also holds the two further copies of each density (at most 2 ncart^2).
 #define CQ_NOALLOC_SCRATCH_BYTES (64ull << 20)
-static __device__ __align__(256) double scratch[CQ_NOALLOC_SCRATCH_BYTES / sizeof(double)];
+static __device__ __align__(256) double scratch[CQ_NOALLOC_SCRATCH_BYTES / 5 * 7 / sizeof(double) + 512];
 
 static std::mutex g_scratch_mu;
 static std::vector<double*> g_scratch_ptr;   // by device id; null until resolved
@@ -159,19 +167,21 @@ __device__ __forceinline__ T wave_sum(T v) {
 // One launch may hold every class pair that screens once per call (all in one batch): the
 // waves of all of them share the device instead of 21 launches of a few hundred waves each.
 struct ScreenList {
-  const CPMeta* cps[2];
-  const GroupRec* groups[2];
+  const CPMeta* cps[3];
+  const GroupRec* groups[3];
+  const int* uorder[3];
+  const unsigned char* nblk[3];   // primitive blocks of every pair as a swept pair
   int n;
   int cp[CQ_NUM_CLASS_PAIRS], tb[CQ_NUM_CLASS_PAIRS], item0[CQ_NUM_CLASS_PAIRS], nres[CQ_NUM_CLASS_PAIRS];
   int cum[CQ_NUM_CLASS_PAIRS + 1];
 };
 
 __global__ void __launch_bounds__(WG) screen_kernel(
-    ScreenList sl, const int* __restrict__ uorder, const int2* __restrict__ s12, const double* __restrict__ pairQ,
+    ScreenList sl, const int2* __restrict__ s12, const double* __restrict__ pairQ,
     const int* __restrict__ grp, const int* __restrict__ cls_grp_off, const int* __restrict__ pair_mol,
     const int* __restrict__ cmg, int nmol, const double* __restrict__ Nmax, const double* __restrict__ Npair,
     const unsigned long long* __restrict__ nglob_bits, int nshell, double tau, double tau_hi,
-    const unsigned char* __restrict__ pair_nblk, uint2* __restrict__ tasks,
+    uint2* __restrict__ tasks,
     unsigned long long* __restrict__ qcounts, Segment* __restrict__ segs, unsigned* __restrict__ ovf_all,
     int count_quartets) {
   __shared__ int ucode[WG / 64][UNION_MAX];
@@ -189,6 +199,8 @@ __global__ void __launch_bounds__(WG) screen_kernel(
   const CPMeta m = sl.cps[sl.tb[e]][cp];
   const int g = m.grp_off + sl.item0[e] + (wave - sl.cum[e]);
   const GroupRec gr = sl.groups[sl.tb[e]][g];
+  const int* __restrict__ uorder = sl.uorder[sl.tb[e]];
+  const unsigned char* __restrict__ pair_nblk = sl.nblk[sl.tb[e]];
   const int nres = sl.nres[e];
   unsigned* const ovf = ovf_all + cp;
   const int n = gr.n, ublk = gr.ublk;
@@ -432,54 +444,108 @@ __global__ void norm_kernel(MatList ml, int ld, const ShellMeta* __restrict__ sh
   if (in && s < t && mx != mxT) atomicOr(&nglob_bits[1 + MAX_MATS], 1ull);
 }
 
-// Npair[P] = N(s1, s2) of every shell pair (the pair's own block norm, read coalesced by the
-// screening).
-__global__ void pair_norm_kernel(const int2* __restrict__ s12, int npair, const double* __restrict__ Nmax,
-                                 int nshell, double* __restrict__ Npair) {
+// (row, column) of X(2,1) for every element of the pair-ordered list (PairInfo::joff).
+__global__ void pair_elements_kernel(const PairInfo* __restrict__ pairs, int npair, const ShellMeta* __restrict__ sh,
+                                     int2* __restrict__ jel) {
   const int P = blockIdx.x * blockDim.x + threadIdx.x;
   if (P >= npair) return;
-  const int2 sp = s12[P];
-  Npair[P] = Nmax[sp.x * nshell + sp.y];
+  const PairInfo p = pairs[P];
+  const int la = sh[p.a].l, lb = sh[p.b].l;
+  const int na = (la + 1) * (la + 2) / 2, nb = (lb + 1) * (lb + 2) / 2;
+  for (int i = 0; i < na; ++i)
+    for (int j = 0; j < nb; ++j)
+      jel[p.joff + i * nb + j] = p.a == p.s1 ? make_int2(p.b0 + j, p.a0 + i) : make_int2(p.a0 + i, p.b0 + j);
 }
 
+// The nonzero coefficients of one shell function or component in the solid-harmonic transform
+// (l <= 2: at most three Cartesian components per function, two functions per component).
+struct TList {
+  int n, idx[3];
+  double c[3];
+};
+__device__ __forceinline__ TList sph_to_cart(const ShellMeta& s, int mu, const double* __restrict__ tco,
+                                             const int* __restrict__ tco_off) {
+  TList t{1, {mu, 0, 0}, {1.0, 0.0, 0.0}};
+  if (s.pure && s.l >= 2) {
+    t.n = 0;
+    const int nc = (s.l + 1) * (s.l + 2) / 2;
+    const double* T = tco + tco_off[s.l] + mu * nc;
+    double v[6];
+#pragma unroll
+    for (int a = 0; a < 6; ++a) v[a] = T[a];
+#pragma unroll
+    for (int a = 0; a < 6; ++a)
+      if (v[a] != 0.0 && t.n < 3) { t.idx[t.n] = a; t.c[t.n] = v[a]; ++t.n; }
+  }
+  return t;
+}
+__device__ __forceinline__ TList cart_to_sph(const ShellMeta& s, int a, const double* __restrict__ tco,
+                                             const int* __restrict__ tco_off) {
+  TList t{1, {a, 0, 0}, {1.0, 0.0, 0.0}};
+  if (s.pure && s.l >= 2) {
+    t.n = 0;
+    const int nc = (s.l + 1) * (s.l + 2) / 2;
+    const double* T = tco + tco_off[s.l] + a;
+    double v[5];
+#pragma unroll
+    for (int m = 0; m < 5; ++m) v[m] = T[m * nc];
+#pragma unroll
+    for (int m = 0; m < 5; ++m)
+      if (v[m] != 0.0 && t.n < 3) { t.idx[t.n] = m; t.c[t.n] = v[m]; ++t.n; }
+  }
+  return t;
+}
 
-// Cartesian density (row-major ncart x ncart): Dc = T^T X T.
-// D_cart = T^T X T for one density; threads below n*n also flag a non-symmetric X: one whose
-// X(i,j) and X(j,i) differ by more than 1e-12 of this X's own largest |X| (xmax_bits, from
+// D_cart = T^T X T for one density: row-major (Dc), transposed (Dt) and the shell pairs' blocks
+// X(2,1) in pair order (Dp, njel elements).  Threads below n*n also flag a non-symmetric X: one
+// whose X(i,j) and X(j,i) differ by more than 1e-12 of this X's own largest |X| (xmax_bits, from
 // norm_kernel).  Differences below that are GEMM rounding (C C^T need not round (i,j) and
 // (j,i) alike).  Digesting such an X as symmetric replaces it by (X + X^T)/2, an entrywise
 // change of at most 5e-13 max|X|, so each G element moves by at most 5e-13 max|X| times the
 // sum of |ERI| over the quartets that element collects; the non-symmetric path would digest
-// the transposed density as well (about four times the work).
+// the transposed density as well (about four times the work).  The threads behind the elements
+// (npair > 0: for one density of the call) write Npair[P] = N(s1, s2), the shell pairs' own block
+// norms, read coalesced by the screening.
 __global__ void cart_density_kernel(const double* __restrict__ X, int n, int ld, const ShellMeta* __restrict__ sh,
                                     const int* __restrict__ cart2shell, int ncart,
                                     const double* __restrict__ tco, const int* __restrict__ tco_off,
                                     const unsigned long long* __restrict__ xmax_bits,
-                                    double* __restrict__ Dc, int* __restrict__ nonsym) {
+                                    double* __restrict__ Dc, double* __restrict__ Dt, double* __restrict__ Dp,
+                                    const int2* __restrict__ jel, long njel, int* __restrict__ nonsym,
+                                    const int2* __restrict__ s12, int npair, const double* __restrict__ Nmax,
+                                    int nshell, double* __restrict__ Npair) {
   const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k < (long)n * n) {
     const int i = k % n, j = k / n;
     const double tol = 1e-12 * __longlong_as_double((long long)*xmax_bits);
     if (i < j && !(fabs(X[(long)j * ld + i] - X[(long)i * ld + j]) <= tol)) atomicOr(nonsym, 1);
   }
-  if (k >= (long)ncart * ncart) return;
-  const int a = k / ncart, b = k - (long)a * ncart;
-  const int sa = cart2shell[a], sb = cart2shell[b];
-  const ShellMeta A = sh[sa], B = sh[sb];
-  const int ia = a - A.cart_off, ib = b - B.cart_off;
-  const int na = A.pure ? 2 * A.l + 1 : (A.l + 1) * (A.l + 2) / 2;
-  const int nb = B.pure ? 2 * B.l + 1 : (B.l + 1) * (B.l + 2) / 2;
-  double sk = 0.0;
-  for (int mu = 0; mu < na; ++mu) {
-    const double ta = tcoef(A, mu, ia, tco, tco_off);
-    if (ta == 0.0) continue;
-    for (int nu = 0; nu < nb; ++nu) {
-      const double tb = tcoef(B, nu, ib, tco, tco_off);
-      if (tb == 0.0) continue;
-      sk += ta * tb * X[(long)(B.sph_off + nu) * ld + A.sph_off + mu];
+  const long nc2 = (long)ncart * ncart;
+  if (k >= nc2 + njel) {
+    const long P = k - nc2 - njel;
+    if (P < npair) {
+      const int2 sp = s12[P];
+      Npair[P] = Nmax[(long)sp.x * nshell + sp.y];
     }
+    return;
   }
-  Dc[k] = sk;
+  const int2 el = k < nc2 ? make_int2((int)(k / ncart), (int)(k % ncart)) : jel[k - nc2];
+  const int a = el.x, b = el.y;
+  const ShellMeta A = sh[cart2shell[a]], B = sh[cart2shell[b]];
+  const TList ta = cart_to_sph(A, a - A.cart_off, tco, tco_off), tb = cart_to_sph(B, b - B.cart_off, tco, tco_off);
+  double sk = 0.0;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (i < ta.n && j < tb.n)
+        sk += ta.c[i] * tb.c[j] * X[(long)(B.sph_off + tb.idx[j]) * ld + A.sph_off + ta.idx[i]];
+  if (k < nc2) {
+    Dc[k] = sk;
+    Dt[(long)b * ncart + a] = sk;
+  } else {
+    Dp[k - nc2] = sk;
+  }
 }
 
 // AX_i[mu + nu*ld] += f_i * sum_{a,c} T(mu,a) T(nu,c) (G_i[a][c] + G'_i[c][a]) for every matrix
@@ -519,7 +585,7 @@ __global__ void finalize_kernel(FinList fl, int n, int ld, const ShellMeta* __re
   const int mu = k % n, nu = k / n;
   const int sa = sph2shell[mu], sb = sph2shell[nu];
   const ShellMeta A = sh[sa], B = sh[sb];
-  const int im = mu - A.sph_off, in = nu - B.sph_off;
+  const TList ta = sph_to_cart(A, mu - A.sph_off, tco, tco_off), tb = sph_to_cart(B, nu - B.sph_off, tco, tco_off);
   const int nca = (A.l + 1) * (A.l + 2) / 2, ncb = (B.l + 1) * (B.l + 2) / 2;
   const int jc = jtab[(long)sa * nshell + sb];
   for (int i = 0; i < fl.n; ++i) {
@@ -527,12 +593,13 @@ __global__ void finalize_kernel(FinList fl, int n, int ld, const ShellMeta* __re
     const double* GB = fl.B[i];
     const bool ns = *fl.nonsym[i] != 0;
     double s = 0.0;
-    for (int a = 0; a < nca; ++a) {
-      const double ta = tcoef(A, im, a, tco, tco_off);
-      if (ta == 0.0) continue;
-      for (int c = 0; c < ncb; ++c) {
-        const double tc = tcoef(B, in, c, tco, tco_off);
-        if (tc == 0.0) continue;
+    // (unrolled: the up to nine elements' loads are in flight together)
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        if (p >= ta.n || q >= tb.n) continue;
+        const int a = ta.idx[p], c = tb.idx[q];
         const long ac = (long)(A.cart_off + a) * ncart + B.cart_off + c;
         const long ca = (long)(B.cart_off + c) * ncart + A.cart_off + a;
         double g = 0.0;
@@ -547,15 +614,14 @@ __global__ void finalize_kernel(FinList fl, int n, int ld, const ShellMeta* __re
           g = GA[ac] + GB[ca];
           if (!ns) g += GA[ca] + GB[ac];
         }
-        s += ta * tc * g;
+        s += ta.c[p] * tb.c[q] * g;
       }
-    }
     fl.AX[i][(long)nu * ld + mu] += fl.f[i] * s;
   }
 }
 
 // Zero a list of word ranges in one launch (accumulators, counters, flags).
-#define MAX_ZERO 12
+#define MAX_ZERO (5 + MAX_MATS)
 struct ZeroList {
   unsigned* p[MAX_ZERO];
   long n[MAX_ZERO];   // 32-bit words
@@ -641,7 +707,7 @@ __global__ void schwarz_kernel(const double* __restrict__ blocks, const int* __r
 __global__ void work_stats_kernel(const uint2* __restrict__ tasks, const Segment* __restrict__ segs,
                                   int nres, const unsigned* __restrict__ ovf, const GroupRec* __restrict__ groups,
                                   const int* __restrict__ uorder, int flip, const PairInfo* __restrict__ pairs,
-                                  const ShellMeta* __restrict__ sh, double* __restrict__ acc) {
+                                  int pblk, int ublk, const ShellMeta* __restrict__ sh, double* __restrict__ acc) {
   const long nseg = (long)nres + *ovf;
   const int lane = threadIdx.x & 63;
   const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) / 64;
@@ -655,13 +721,13 @@ __global__ void work_stats_kernel(const uint2* __restrict__ tasks, const Segment
     for (int m = 0; m < gr.n; ++m) {
       const PairInfo Up = pairs[uorder[gr.first + m]];
       int up0, up1;
-      prim_range<UNI_BLOCK>(Up, (unsigned)sg.blk, up0, up1);
+      prim_range(Up, (unsigned)sg.blk, ublk, up0, up1);
       const uint2 hm = reg[1 + m];
       for (int t = lane; t < (int)hm.x; t += 64) {
         const uint2 e = reg[hm.y + t];
         const PairInfo Sp = pairs[pair_of(e.x)];
         int sp0, sp1;
-        prim_range(Sp, block_of(e.x), sp0, sp1);
+        prim_range(Sp, block_of(e.x), pblk, sp0, sp1);
         const PairInfo& B = flip ? Up : Sp;
         const PairInfo& K = flip ? Sp : Up;
         const double kab = flip ? up1 - up0 : sp1 - sp0, kcd = flip ? sp1 - sp0 : up1 - up0;
@@ -834,7 +900,8 @@ struct cq_ctx {
   double mixed_threshold = 1e-5;
   double prim_threshold = 1e-17;
   // class-pair tables: [0] every class pair ket-keyed, [1] with bra-keyed (flipped) class pairs
-  std::vector<CPMeta> cps[2];
+  // [2] the merged launches' own plan (merge_tab)
+  std::vector<CPMeta> cps[3];
   long long task_capacity = 0;
   // task lists per class pair are at most task_budget entries (8 B each); a class pair whose
   // worst case is larger screens and digests its groups in batches:
@@ -844,9 +911,9 @@ struct cq_ctx {
   // order groups are cut from (molecule, primitive blocks, first shell, second shell);
   // groups_h[t] the groups of every class pair of table t (CPMeta::grp_off)
   std::vector<int> uorder_h;
-  std::vector<GroupRec> groups_h[2];
-  DevBuf<int> d_uorder;
-  DevBuf<GroupRec> d_groups[2];
+  std::vector<GroupRec> groups_h[3];
+  DevBuf<int> d_uorder, d_uorder_m;
+  DevBuf<GroupRec> d_groups[3];
   // per class pair: dynamic LDS budget of the group kernels (bytes) and an optional cap on
   // the group size and on the union bound (0: from the budget)
   std::vector<long long> tile_lds = std::vector<long long>(CQ_NUM_CLASS_PAIRS, 0);
@@ -856,9 +923,16 @@ struct cq_ctx {
   std::vector<int> last_table = std::vector<int>(CQ_NUM_CLASS_PAIRS, 0);
   bool plan_ok = false;   // task and segment buffers are allocated for the current plan
   double* scratch = nullptr;   // this device's address of the no-allocation workspace
-  std::vector<std::vector<int>> batch_start[2];
-  std::vector<std::vector<int>> batch_slots[2];   // reserved segment slots of each batch (one set per group)
+  std::vector<std::vector<int>> batch_start[3];
+  std::vector<std::vector<int>> batch_slots[3];   // reserved segment slots of each batch (one set per group)
   std::vector<unsigned char> nblk_h, nublk_h;
+  // merged launches: primitive blocks of mpblk (lane side) and mublk (uniform side), and the plan
+  // they run: table 1, or a table 2 of their own where their blocks differ or table 1 keys a class
+  // pair on a side that has no merged kernel
+  int mpblk = PRIM_BLOCK, mublk = UNI_BLOCK, merge_tab = 1;
+  bool own_blocks() const { return mpblk != PRIM_BLOCK || mublk != UNI_BLOCK; }
+  std::vector<unsigned char> nblk_m, nublk_m;   // with blocks of their own: blocks per pair
+  std::vector<int> uorder_m;                    // and uniform order
   std::vector<int> pair_mol_h;
   std::vector<unsigned long long> last_counts;
   // profiling: events around every class-pair kernel of every contraction
@@ -892,7 +966,8 @@ struct cq_ctx {
   DevBuf<PairInfo> d_pairs, d_pairs_1e;
   std::vector<PairInfo> pairs_1e_h;   // host copies kept for the asynchronous uploads
   std::vector<int> rowfn_h;
-  DevBuf<int2> d_s12;
+  DevBuf<int2> d_s12, d_jel;
+  size_t njel = 0;   // elements of the pair-ordered Coulomb list (at most ncart^2)
   std::vector<int> grp, cls_grp_off;
   DevBuf<int> d_grp, d_cls_grp_off;
   // several molecules in one context: shell pairs and quartets only within a molecule
@@ -916,7 +991,7 @@ struct cq_ctx {
   hipStream_t aux[kAux] = {};
   hipEvent_t ev_fork = nullptr, ev_join[kAux] = {};
   DevBuf<PrimPair> d_prims;
-  DevBuf<CPMeta> d_cps[2];
+  DevBuf<CPMeta> d_cps[3];
   DevBuf<uint2> d_tasks;
   DevBuf<Segment> d_segs;
   DevBuf<unsigned> d_work_q, d_ovf;
@@ -928,14 +1003,14 @@ struct cq_ctx {
   // per class pair: chunks per work item of the group kernels (0: the built-in choice)
   std::vector<int> class_cpi = std::vector<int>(CQ_NUM_CLASS_PAIRS, 0);
   DevBuf<unsigned long long> d_qcounts, d_nglob;
-  DevBuf<unsigned char> d_pair_nblk, d_pair_nublk;
+  DevBuf<unsigned char> d_pair_nblk, d_pair_nublk, d_pair_nblk_m;
   std::string err;
 
   ~cq_ctx() {
-    d_shells.release(); d_cart2shell.release(); d_sph2shell.release(); d_tco_off.release(); d_jtab.release();
-    d_uorder.release(); d_groups[0].release(); d_groups[1].release(); d_flags.release(); d_tco.release(); d_boys.release(); d_pairQ.release();
+    d_shells.release(); d_cart2shell.release(); d_sph2shell.release(); d_tco_off.release(); d_jtab.release(); d_jel.release(); d_rowfn.release();
+    d_uorder.release(); d_uorder_m.release(); d_pair_nblk_m.release(); for (auto& g : d_groups) g.release(); d_flags.release(); d_tco.release(); d_boys.release(); d_pairQ.release();
     d_Nmax.release(); d_Npair.release(); d_work.release(); d_mats.release(); d_pairs.release(); d_pairs_1e.release(); d_prims.release();
-    d_cps[0].release(); d_cps[1].release(); d_tasks.release(); d_segs.release(); d_work_q.release(); d_ovf.release(); d_qcounts.release(); d_nglob.release(); d_pair_nblk.release(); d_pair_nublk.release();
+    for (auto& m : d_cps) m.release(); d_tasks.release(); d_segs.release(); d_work_q.release(); d_ovf.release(); d_qcounts.release(); d_nglob.release(); d_pair_nblk.release(); d_pair_nublk.release();
     d_prim_off.release(); d_alpha.release(); d_coef.release(); d_origin.release(); d_onee.release();
     for (auto e : event_pool) (void)hipEventDestroy(e);
     for (int k = 0; k < kAux; ++k) {
@@ -1075,17 +1150,28 @@ void class_tile(const cq_ctx* c, int k, int variant, int& mmax, int& ub) {
 void plan_tasks(cq_ctx* c) {
   c->plan_ok = false;
   const int nm = c->nmol;
-  const std::vector<unsigned char>& nblk = c->nblk_h;
-  const std::vector<unsigned char>& nublk = c->nublk_h;
   const std::vector<int>& pair_mol = c->pair_mol_h;
-  for (int t = 0; t < 2; ++t) {
+  const bool own = c->own_blocks();
+  // bra-keyed in table 1: few bra pairs, and the bra-keyed LDS rows fit
+  auto bra_keyed = [&](int k) {
+    const ClassKernels& ck = kClassKernels[k];
+    const long long nb = c->class_start[ck.bi + 1] - c->class_start[ck.bi], nk = c->class_start[ck.ki + 1] - c->class_start[ck.ki];
+    int mm2 = 0, ub2 = 64;
+    if (ck.grp[0][2]) class_tile(c, k, 2, mm2, ub2);
+    return ck.i != ck.j && mm2 > 0 && 2 * nb <= nk;
+  };
+  c->merge_tab = own ? 2 : 1;
+  for (int k = 0; k < kNumClassPairs; ++k)
+    if (!(kClassKernels[k].merged >> (bra_keyed(k) ? 1 : 0) & 1)) c->merge_tab = 2;
+  const int ntab = c->merge_tab + 1;
+  for (int t = 0; t < 3; ++t) {
     c->cps[t].clear();
     c->groups_h[t].clear();
     c->batch_start[t].assign(kNumClassPairs, std::vector<int>());
     c->batch_slots[t].assign(kNumClassPairs, std::vector<int>());
   }
   const long long budget = c->task_budget;
-  long long off = 0, seg_total[2] = {0, 0};
+  long long off = 0, off_m = 0, seg_total[3] = {0, 0, 0};
   for (int k = 0; k < kNumClassPairs; ++k) {
     const ClassKernels& ck = kClassKernels[k];
     CPMeta m{};
@@ -1096,18 +1182,21 @@ void plan_tasks(cq_ctx* c) {
     m.same = ck.i == ck.j;
     m.bra_class = ck.bi;
     m.ket_class = ck.ki;
-    // swept-side pairs and primitive blocks per molecule
-    std::vector<long long> bp_m(nm, 0), kp_m(nm, 0), bb_m(nm, 0), kb_m(nm, 0);
-    for (int i = 0; i < m.nbra; ++i) { bp_m[pair_mol[m.bra_start + i]] += 1; bb_m[pair_mol[m.bra_start + i]] += nblk[m.bra_start + i]; }
-    for (int i = 0; i < m.nket; ++i) { kp_m[pair_mol[m.ket_start + i]] += 1; kb_m[pair_mol[m.ket_start + i]] += nblk[m.ket_start + i]; }
     int mm2 = 0, ub2 = 64;
     if (ck.grp[0][2]) class_tile(c, k, 2, mm2, ub2);
-    const int flip = (!m.same && ck.grp[0][2] && mm2 > 0 && 2LL * m.nbra <= m.nket) ? 1 : 0;
-    CPMeta mt[2] = {m, m};
+    const int flip = bra_keyed(k);
+    CPMeta mt[3] = {m, m, m};
     long long region = 0;
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < ntab; ++t) {
+      const std::vector<unsigned char>& nblk = t < 2 || !own ? c->nblk_h : c->nblk_m;
+      const std::vector<unsigned char>& nublk = t < 2 || !own ? c->nublk_h : c->nublk_m;
+      const std::vector<int>& uorder = t < 2 || !own ? c->uorder_h : c->uorder_m;
+      // swept-side pairs and primitive blocks per molecule
+      std::vector<long long> bp_m(nm, 0), kp_m(nm, 0), bb_m(nm, 0), kb_m(nm, 0);
+      for (int i = 0; i < m.nbra; ++i) { bp_m[pair_mol[m.bra_start + i]] += 1; bb_m[pair_mol[m.bra_start + i]] += nblk[m.bra_start + i]; }
+      for (int i = 0; i < m.nket; ++i) { kp_m[pair_mol[m.ket_start + i]] += 1; kb_m[pair_mol[m.ket_start + i]] += nblk[m.ket_start + i]; }
       CPMeta& mc = mt[t];
-      mc.flip = t == 1 ? flip : 0;
+      mc.flip = t == 0 ? 0 : t == 1 || ck.merged == 3 ? flip : ck.merged == 2;
       int mmax = 0, ub = 64;
       if (mc.flip) {
         mmax = mm2;
@@ -1126,10 +1215,10 @@ void plan_tasks(cq_ctx* c) {
       mc.grp_off = (int)c->groups_h[t].size();
       const int u0 = c->class_start[ucls], u1 = c->class_start[ucls + 1];
       for (int x = u0; x < u1;) {
-        const int P0 = c->uorder_h[x];
+        const int P0 = uorder[x];
         int y = x + 1;
         while (y < u1 && y - x < mmax) {
-          const int P = c->uorder_h[y];
+          const int P = uorder[y];
           if (pair_mol[P] != pair_mol[P0] || nublk[P] != nublk[P0] || c->pairs[P].a != c->pairs[P0].a) break;
           ++y;
         }
@@ -1166,11 +1255,11 @@ void plan_tasks(cq_ctx* c) {
       };
       for (int gi = 0; gi < mc.ngrp; ++gi) {
         GroupRec& gr = c->groups_h[t][mc.grp_off + gi];
-        const int mol = pair_mol[c->uorder_h[gr.first]];
+        const int mol = pair_mol[uorder[gr.first]];
         long long S, Bk;
         if (m.same) {
           int lmin = 0x7fffffff;
-          for (int q = 0; q < gr.n; ++q) lmin = std::min(lmin, c->uorder_h[gr.first + q] - uni_start);
+          for (int q = 0; q < gr.n; ++q) lmin = std::min(lmin, uorder[gr.first + q] - uni_start);
           S = suf_p[lmin];
           Bk = suf_b[lmin];
         } else {
@@ -1195,26 +1284,44 @@ void plan_tasks(cq_ctx* c) {
       mc.seg_cap = seg_cap;
       mc.seg_off = seg_total[t];
       seg_total[t] += seg_cap;
-      region = std::max(region, cap);
+      if (t < 2) region = std::max(region, cap);
     }
-    for (int t = 0; t < 2; ++t) {
-      mt[t].task_off = off;
+    for (int t = 0; t < ntab; ++t) {
+      mt[t].task_off = t < 2 ? off : off_m;
       c->cps[t].push_back(mt[t]);
     }
     off += region;
+    if (ntab > 2) off_m += mt[2].task_cap;
   }
   c->task_capacity = off;
   // one call may take table 0 for some class pairs and table 1 for others (per-class digestion
   // variants): table 1's segments live after table 0's
   for (auto& mt : c->cps[1]) mt.seg_off += seg_total[0];
-  for (int t = 0; t < 2; ++t) {
+  for (int t = 0; t < ntab; ++t) {
     c->d_cps[t].upload(c->cps[t], c->stream);
     c->d_groups[t].upload(c->groups_h[t], c->stream);
   }
-  c->d_tasks.ensure((size_t)std::max<long long>(1, off));
-  c->d_segs.ensure((size_t)std::max<long long>(1, seg_total[0] + seg_total[1]));
+  // (a call uses tables 0 and 1 or table 2: they share the buffers)
+  c->d_tasks.ensure((size_t)std::max<long long>({1, off, off_m}));
+  c->d_segs.ensure((size_t)std::max<long long>({1, seg_total[0] + seg_total[1], seg_total[2]}));
   HIPCHK(hipStreamSynchronize(c->stream));
   c->plan_ok = true;
+}
+
+// Primitive block sizes of the merged launches' plan for a context of npair shell pairs with at most
+// np_max primitive pairs each.  Few quartets leave most of the device idle, and then the longest
+// lane task (block x block primitive quartets in series) sets the time: smaller blocks.  More
+// quartets fill the device, and every block more digests its quartet once more.
+// Measured, G[D] in us with blocks (lane, uniform) 2,8 / 4,8 / 8,32:
+//   H2O/6-31G* (55 pairs) 243 / 286 / 412, O2/cc-pVDZ UHF (78) 255 / 302 / 543,
+//   (H2O)4/cc-pVDZ (1176) 548 / 496 / 598, (H2O)11/6-31G UHF (4851) 809 / 772 / 783,
+//   C12H26/6-31G* (7750) 2354 / 2121 / 2064, (H2O)16/cc-pVDZ (18528) 4116 / 3632 / 3544.
+void choose_merge_blocks(cq_ctx* c, int npair, int np_max) {
+  c->mpblk = npair <= 300 ? 2 : npair <= 6000 ? 4 : PRIM_BLOCK;
+  c->mublk = npair <= 6000 ? 8 : UNI_BLOCK;
+  // (block codes: at most 64 blocks of a pair)
+  c->mpblk = std::max(c->mpblk, (np_max + 63) / 64);
+  c->mublk = std::max(c->mublk, (np_max + 63) / 64);
 }
 
 void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const int* nprim, const double* alpha,
@@ -1540,6 +1647,10 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
                        c->d_jtab.p);
     hipLaunchKernelGGL(jtab_kernel, dim3(grid_for(npair, WG)), dim3(WG), 0, c->stream, c->d_pairs.p, npair, nshell,
                        c->d_jtab.p);
+    c->njel = npair ? (size_t)c->pairs[npair - 1].joff + ncart_l(l[c->pairs[npair - 1].a]) * ncart_l(l[c->pairs[npair - 1].b]) : 0;
+    c->d_jel.ensure(std::max<size_t>(1, c->njel));
+    hipLaunchKernelGGL(pair_elements_kernel, dim3(grid_for(npair, WG)), dim3(WG), 0, c->stream, c->d_pairs.p, npair,
+                       c->d_shells.p, c->d_jel.p);
     HIPCHK(hipGetLastError());
   }
   // primitive-count groups per class: grp[cls_grp_off[X] .. cls_grp_off[X+1]] are the group
@@ -1583,30 +1694,51 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     c->Q[(size_t)pi_.s2 * nshell + pi_.s1] = c->pairQ[k];
   }
   // primitive blocks per pair (1: unsplit) as the per-lane side and as the uniform side
+  int np_max = 1;
+  for (int k = 0; k < npair; ++k) np_max = std::max(np_max, c->pairs[k].p1 - c->pairs[k].p0);
+  if (np_max > 64 * PRIM_BLOCK) throw std::invalid_argument("more than 512 primitive pairs in one shell pair");
+  choose_merge_blocks(c, npair, np_max);
   std::vector<unsigned char> nblk(npair), nublk(npair);
+  if (c->own_blocks()) {
+    c->nblk_m.resize(npair);
+    c->nublk_m.resize(npair);
+  }
   for (int k = 0; k < npair; ++k) {
     const int np = c->pairs[k].p1 - c->pairs[k].p0;
-    if (np > 64 * PRIM_BLOCK) throw std::invalid_argument("more than 512 primitive pairs in one shell pair");
-    nblk[k] = (unsigned char)(np > PRIM_BLOCK ? (np + PRIM_BLOCK - 1) / PRIM_BLOCK : 1);
-    nublk[k] = (unsigned char)(np > UNI_BLOCK ? (np + UNI_BLOCK - 1) / UNI_BLOCK : 1);
+    nblk[k] = (unsigned char)((np + PRIM_BLOCK - 1) / PRIM_BLOCK);
+    nublk[k] = (unsigned char)((np + UNI_BLOCK - 1) / UNI_BLOCK);
+    if (!c->own_blocks()) continue;
+    c->nblk_m[k] = (unsigned char)((np + c->mpblk - 1) / c->mpblk);
+    c->nublk_m[k] = (unsigned char)((np + c->mublk - 1) / c->mublk);
   }
   if ((unsigned)npair > PAIR_MASK) throw std::invalid_argument("too many shell pairs");
   c->d_pair_nblk.upload(nblk, c->stream);
   c->d_pair_nublk.upload(nublk, c->stream);
   c->nblk_h.swap(nblk);
   c->nublk_h.swap(nublk);
-  // uniform order of every class: by molecule, primitive blocks, first and second shell (groups
-  // are cut from runs sharing the first three)
-  c->uorder_h.resize(npair);
-  std::iota(c->uorder_h.begin(), c->uorder_h.end(), 0);
-  for (int X = 0; X < c->npc; ++X)
-    std::stable_sort(c->uorder_h.begin() + c->class_start[X], c->uorder_h.begin() + c->class_start[X + 1],
-                     [&](int x, int y) {
-                       if (c->pair_mol_h[x] != c->pair_mol_h[y]) return c->pair_mol_h[x] < c->pair_mol_h[y];
-                       if (c->nublk_h[x] != c->nublk_h[y]) return c->nublk_h[x] < c->nublk_h[y];
-                       if (c->pairs[x].a != c->pairs[y].a) return c->pairs[x].a < c->pairs[y].a;
-                       return c->pairs[x].b < c->pairs[y].b;
-                     });
+  // uniform order of every class: by molecule, primitive blocks and the first shell's contraction
+  // (most first: work items are handed out in this order, and a heavily contracted group's items
+  // take up to 100 us, so they must not be the last ones), first and second shell (groups are cut
+  // from runs sharing the first shell and the block count)
+  auto uniform_order = [&](std::vector<int>& ord, const std::vector<unsigned char>& nub) {
+    ord.resize(npair);
+    std::iota(ord.begin(), ord.end(), 0);
+    for (int X = 0; X < c->npc; ++X)
+      std::stable_sort(ord.begin() + c->class_start[X], ord.begin() + c->class_start[X + 1], [&](int x, int y) {
+        if (c->pair_mol_h[x] != c->pair_mol_h[y]) return c->pair_mol_h[x] < c->pair_mol_h[y];
+        if (nub[x] != nub[y]) return nub[x] > nub[y];
+        const int ax = c->pairs[x].a, ay = c->pairs[y].a;
+        if (nprim[ax] != nprim[ay]) return nprim[ax] > nprim[ay];
+        if (ax != ay) return ax < ay;
+        return c->pairs[x].b < c->pairs[y].b;
+      });
+  };
+  uniform_order(c->uorder_h, c->nublk_h);
+  if (c->own_blocks()) {
+    uniform_order(c->uorder_m, c->nublk_m);
+    c->d_uorder_m.upload(c->uorder_m, c->stream);
+    c->d_pair_nblk_m.upload(c->nblk_m, c->stream);
+  }
   c->d_uorder.upload(c->uorder_h, c->stream);
   plan_tasks(c);
   c->scratch = scratch_address();
@@ -1668,12 +1800,13 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   const int ns = c->nshell;
   const long nc2 = (long)c->ncart * c->ncart;
   const int nslot = (int)slots.size();
-  // workspace: per slot Dc, GJ, GJ2, GK, GK2, then one flag per slot
-  const size_t work_words = (size_t)std::max(1, nslot) * 5 * nc2;
+  // workspace: per slot Dc, GJ, GJ2, GK, GK2, Dt (ncart^2 each) and Dp, then one flag per slot
+  const size_t slot_words = 6 * (size_t)nc2 + c->njel;
+  const size_t work_words = (size_t)std::max(1, nslot) * slot_words;
   double* work = nullptr;
   int* flags = nullptr;
   if (noalloc) {
-    const size_t need = work_words * sizeof(double) + (size_t)std::max(1, nslot) * sizeof(int);
+    const size_t need = (size_t)std::max(1, nslot) * (5 * (size_t)nc2 * sizeof(double) + sizeof(int));
     if (need > CQ_NOALLOC_SCRATCH_BYTES)
       throw std::invalid_argument("the no-allocation workspace (64 MiB) is too small for this call: it needs " +
                                   std::to_string(need) + " bytes (5 ncart^2 doubles per distinct density)");
@@ -1699,9 +1832,10 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   zero(c->d_qcounts.p, 2 * kNumClassPairs * sizeof(unsigned long long));
   zero(c->d_work_q.p, (size_t)kNumClassPairs * MAX_MATS * WORK_QUEUES * sizeof(unsigned));
   zero(c->d_ovf.p, kNumClassPairs * sizeof(unsigned));
-  // the whole workspace (the Cartesian densities in it are rewritten below)
-  zero(work, (size_t)std::max(1, nslot) * 5 * nc2 * sizeof(double));
-  hipLaunchKernelGGL(zero_kernel, dim3(1024), dim3(WG), 0, s, zl);
+  // (every slot's accumulators; its density copies are rewritten below)
+  for (int k = 0; k < nslot; ++k) zero(work + k * slot_words + nc2, 4 * (size_t)nc2 * sizeof(double));
+  const int zgrid = (int)std::min<long>(1024, grid_for(std::max<long>(8 * nc2, 64 * kNumClassPairs), WG));
+  hipLaunchKernelGGL(zero_kernel, dim3(zgrid), dim3(WG), 0, s, zl);
   HIPCHK(hipGetLastError());
   // 2. block norms over every input matrix (scale 0 included)
   MatList ml{};
@@ -1710,20 +1844,16 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   hipLaunchKernelGGL(norm_kernel, dim3(grid_for((long)ns * ns, WG)), dim3(WG), 0, s, ml, ld, c->d_shells.p, ns,
                      c->d_Nmax.p, c->d_nglob.p);
   HIPCHK(hipGetLastError());
-  {
-    const int np = (int)c->pairs.size();
-    hipLaunchKernelGGL(pair_norm_kernel, dim3(grid_for(np, WG)), dim3(WG), 0, s, c->d_s12.p, np, c->d_Nmax.p, ns,
-                       c->d_Npair.p);
-    HIPCHK(hipGetLastError());
-  }
   if (nslot == 0) return;
-  // 3. Cartesian densities and symmetry flags; per slot: [Dc | GJ | GJ2 | GK | GK2], ncart^2 each
+  // 3. Cartesian densities and symmetry flags (with the first density, the shell pairs' own norms)
   for (int k = 0; k < nslot; ++k) {
-    double* base = work + (size_t)k * 5 * nc2;
-    hipLaunchKernelGGL(cart_density_kernel, dim3(grid_for(std::max<long>(nc2, (long)n * n), WG)), dim3(WG), 0, s,
+    double* base = work + (size_t)k * slot_words;
+    const int np = k == 0 ? (int)c->pairs.size() : 0;
+    hipLaunchKernelGGL(cart_density_kernel, dim3(grid_for(std::max<long>(nc2 + c->njel + np, (long)n * n), WG)), dim3(WG), 0, s,
                        slots[k].X, n, ld, c->d_shells.p, c->d_cart2shell.p, c->ncart, c->d_tco.p, c->d_tco_off.p,
                        c->d_nglob.p + 1 + (std::find(uniq.begin(), uniq.end(), slots[k].X) - uniq.begin()), base,
-                       flags + k);
+                       base + 5 * nc2, base + 6 * nc2, c->d_jel.p, (long)c->njel, flags + k, c->d_s12.p, np,
+                       c->d_Nmax.p, ns, c->d_Npair.p);
     HIPCHK(hipGetLastError());
   }
   // digestion variant per class pair (the lds_mode, or the class's own choice below it)
@@ -1756,10 +1886,13 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   // task regions of this round's bound window [lo, hi)
   auto screen_list_base = [&]() {
     ScreenList sl{};
-    sl.cps[0] = c->d_cps[0].p;
-    sl.cps[1] = c->d_cps[1].p;
-    sl.groups[0] = c->d_groups[0].p;
-    sl.groups[1] = c->d_groups[1].p;
+    for (int t = 0; t < 3; ++t) {
+      sl.cps[t] = c->d_cps[t].p;
+      sl.groups[t] = c->d_groups[t].p;
+      const bool own = t == 2 && c->own_blocks();
+      sl.uorder[t] = own ? c->d_uorder_m.p : c->d_uorder.p;
+      sl.nblk[t] = own ? c->d_pair_nblk_m.p : c->d_pair_nblk.p;
+    }
     return sl;
   };
   auto add_screen_entry = [&](ScreenList& sl, int k, int tb, int g0, int ng, int nres) {
@@ -1780,9 +1913,8 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
       q1 = c->get_event();
       HIPCHK(hipEventRecord(q0, st));
     }
-    hipLaunchKernelGGL(screen_kernel, dim3(grid_for(waves, WG / 64)), dim3(WG), 0, st, sl, c->d_uorder.p,
-                       c->d_s12.p, c->d_pairQ.p, c->d_grp.p, c->d_cls_grp_off.p, c->d_pair_mol.p, c->d_cmg.p,
-                       c->nmol, c->d_Nmax.p, c->d_Npair.p, c->d_nglob.p, ns, lo, hi, c->d_pair_nblk.p,
+    hipLaunchKernelGGL(screen_kernel, dim3(grid_for(waves, WG / 64)), dim3(WG), 0, st, sl, c->d_s12.p, c->d_pairQ.p, c->d_grp.p, c->d_cls_grp_off.p, c->d_pair_mol.p, c->d_cmg.p,
+                       c->nmol, c->d_Nmax.p, c->d_Npair.p, c->d_nglob.p, ns, lo, hi,
                        c->d_tasks.p, c->d_qcounts.p + (fp32 ? kNumClassPairs : 0), c->d_segs.p, c->d_ovf.p,
                        count ? 1 : 0);
     HIPCHK(hipGetLastError());
@@ -1826,35 +1958,109 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   // its class pairs behind it, so the kernels start early and the bulk of the screening runs
   // beside other streams' kernels; with CQ_SCREEN_ONE one launch on s before the fork screens
   // them all
+  // merged launches (FP64, default settings): the class pairs of a tier that run in one batch, per
+  // tier one screening and one merged launch on a stream of its own.  Settings that address
+  // class pairs one by one (their variant or stream, profiling, the screening mode, one stream)
+  // and class pairs in several batches keep a launch per class pair.  (H2O)16/cc-pVDZ 3638 us with
+  // a launch per class pair, 3544 merged; smaller systems gain more (choose_merge_blocks).
+  static_assert(CQ_NUM_TIERS == cq_ctx::kAux + 1, "one stream per merged tier");
+  const int mt = c->merge_tab;
+  const bool can_merge = nround == 1 && !profiling && c->n_streams == cq_ctx::kAux + 1 &&
+                         c->screen_mode == CQ_SCREEN_PER_STREAM && c->lds_mode == 2;
+  std::vector<char> merged(kNumClassPairs, 0);
+  for (int k = 0; k < kNumClassPairs && can_merge; ++k) {
+    const CPMeta& m = c->cps[mt][k];
+    merged[k] = c->class_variant[k] < 0 && c->class_stream[k] < 0 && stream_of[k] >= 0 && m.ngrp > 0 &&
+                c->batch_start[mt][k].size() == 2 && m.mmax >= 1 &&
+                group_lds(c, kClassKernels[k], m.flip ? 2 : 1, m.mmax, m.ub) <= c->max_dyn_lds;
+  }
   std::vector<char> fused(kNumClassPairs, 0);
   std::vector<int> once[cq_ctx::kAux + 1];   // per stream, in launch order
   if (c->screen_mode != CQ_SCREEN_PER_CLASS)
     for (int kk = kNumClassPairs - 1; kk >= 0; --kk) {
       const int k = c->launch_order[kk];
+      if (merged[k]) continue;
       if (stream_of[k] < 0 || c->batch_start[variant_of(k) >= 2 ? 1 : 0][k].size() != 2) continue;
       once[stream_of[k]].push_back(k);
       fused[k] = 1;
     }
-  auto screen_of = [&](const int* ks, int n) {
+  auto screen_of = [&](const int* ks, int n, bool merge) {
     ScreenList sl = screen_list_base();
     for (int i = 0; i < n; ++i) {
-      const int k = ks[i], tb = variant_of(k) >= 2 ? 1 : 0;
+      const int k = ks[i], tb = merge ? mt : variant_of(k) >= 2 ? 1 : 0;
       const std::vector<int>& bs = c->batch_start[tb][k];
       add_screen_entry(sl, k, tb, bs[0], bs[1] - bs[0], c->batch_slots[tb][k][0]);
     }
     return sl;
   };
+  auto launch_tier = [&](int t, hipStream_t st) {
+    MergedArgs ma{};
+    std::vector<int> ks;
+    size_t lds = 0;
+    int nblk = 0;
+    for (int kk = kNumClassPairs - 1; kk >= 0; --kk) {   // highest angular momentum first
+      const int k = c->launch_order[kk];
+      const ClassKernels& ck = kClassKernels[k];
+      if (ck.tier != t || !merged[k]) continue;
+      const CPMeta& m = c->cps[mt][k];
+      const int kv = m.flip ? 2 : 1;
+      c->last_table[k] = mt;
+      ks.push_back(k);
+      MergedEntry& e = ma.e[ma.n++];
+      e.k = k;
+      e.bra = m.flip;
+      e.blk0 = nblk;
+      e.cpi = class_chunks_per_item(c, k);
+      e.nblk = (int)std::max<long long>(1, std::min<long long>(persistent_grid() / 4, m.seg_cap * (ck.nchunk / e.cpi)));
+      nblk += e.nblk;
+      e.nres = c->batch_slots[mt][k][0];
+      e.mmax = m.mmax;
+      e.ub = m.ub;
+      e.lds_n = lds_rows(c, ck, kv);
+      e.rowfn = (kv == 2 ? ck.ki : ck.bi) * c->ncart;
+      e.task_off = m.task_off;
+      e.seg_off = m.seg_off;
+      lds = std::max(lds, group_lds(c, ck, kv, m.mmax, m.ub));
+    }
+    if (ks.empty()) return;
+    launch_screen(screen_of(ks.data(), (int)ks.size(), true), st, c->prof_screen_events[kNumClassPairs], true);
+    ma.slot_words = (long long)slot_words;
+    JKArgs jk{};
+    jk.ncart = c->ncart;
+    jk.rowfn = c->d_rowfn.p;
+    jk.D[0] = work;
+    jk.GJ[0] = work + nc2;
+    jk.GJ2[0] = work + 2 * nc2;
+    jk.GK[0] = work + 3 * nc2;
+    jk.GK2[0] = work + 4 * nc2;
+    jk.Dt[0] = work + 5 * nc2;
+    jk.Dp[0] = work + 6 * nc2;
+    jk.nonsym = flags;
+    jk.pblk = c->mpblk;
+    jk.ublk = c->mublk;
+    for (int k = 0; k < nslot; ++k) {
+      ma.jmask |= (unsigned)slots[k].do_j << k;
+      ma.kmask |= (unsigned)slots[k].do_k << k;
+    }
+    hipLaunchKernelGGL(kMergedTiers[t].kernel, dim3(nblk, nslot), dim3(kMergedTiers[t].wgs), lds, st, ma, c->d_tasks.p,
+                       c->d_segs.p, c->d_ovf.p, c->d_work_q.p, c->d_pairs.p, c->d_prims.p, c->d_boys.p, jk,
+                       c->d_groups[mt].p,
+                       (mt == 2 && c->own_blocks() ? c->d_uorder_m : c->d_uorder).p);
+    HIPCHK(hipGetLastError());
+  };
   if (c->screen_mode == CQ_SCREEN_ONE) {
     std::vector<int> all;
     for (int si = 0; si < c->n_streams; ++si) all.insert(all.end(), once[si].begin(), once[si].end());
-    launch_screen(screen_of(all.data(), (int)all.size()), s, c->prof_screen_events[kNumClassPairs], true);
+    launch_screen(screen_of(all.data(), (int)all.size(), false), s, c->prof_screen_events[kNumClassPairs], true);
   }
   HIPCHK(hipEventRecord(c->ev_fork, s));
   for (int a = 0; a < cq_ctx::kAux; ++a) HIPCHK(hipStreamWaitEvent(c->aux[a], c->ev_fork, 0));
+  if (can_merge)
+    for (int t = 0; t < CQ_NUM_TIERS; ++t) launch_tier(t, stream_at(t));
   if (c->screen_mode == CQ_SCREEN_PER_STREAM)
     for (int si = 0; si < c->n_streams; ++si)
       if (!once[si].empty())
-        launch_screen(screen_of(once[si].data(), 1), stream_at(si), c->prof_screen_events[kNumClassPairs], true);
+        launch_screen(screen_of(once[si].data(), 1, false), stream_at(si), c->prof_screen_events[kNumClassPairs], true);
   // 4. per class pair, on its stream: screening into its task regions (unless screened above),
   //    then ERI + J/K digestion, one density slot per pass (the lists are screened once and kept
   //    for every slot when the class pair is one batch); joined back into s before the
@@ -1862,8 +2068,10 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   for (int s0 = 0; s0 < nslot; ++s0) {
     JKArgs jk{};
     jk.ncart = c->ncart;
-    double* base = work + (size_t)s0 * 5 * nc2;
+    double* base = work + (size_t)s0 * slot_words;
     jk.D[0] = base;
+    jk.Dt[0] = base + 5 * nc2;
+    jk.Dp[0] = base + 6 * nc2;
     jk.GJ[0] = base + nc2;
     jk.GJ2[0] = base + 2 * nc2;
     jk.GK[0] = base + 3 * nc2;
@@ -1871,9 +2079,12 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
     jk.do_j[0] = slots[s0].do_j;
     jk.do_k[0] = slots[s0].do_k;
     jk.nonsym = flags + s0;
+    jk.pblk = PRIM_BLOCK;
+    jk.ublk = UNI_BLOCK;
     for (int kk = kNumClassPairs - 1; kk >= 0; --kk) {
       const int k = c->launch_order[kk];
       const ClassKernels& ck = kClassKernels[k];
+      if (merged[k]) continue;
       const int var = variant_of(k);
       const int tb = var >= 2 ? 1 : 0;
       const CPMeta& m = c->cps[tb][k];
@@ -1939,7 +2150,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
       // once-per-call class pairs
       const std::vector<int>& ol = once[stream_of[k]];
       if (s0 == 0 && c->screen_mode == CQ_SCREEN_PER_STREAM && ol.size() > 1 && ol[0] == k)
-        launch_screen(screen_of(ol.data() + 1, (int)ol.size() - 1), sk, c->prof_screen_events[kNumClassPairs], true);
+        launch_screen(screen_of(ol.data() + 1, (int)ol.size() - 1, false), sk, c->prof_screen_events[kNumClassPairs], true);
     }
   }
   for (int a = 0; a < cq_ctx::kAux; ++a) {
@@ -1953,7 +2164,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   for (int i = 0; i < nmat; ++i) {
     const int k = mat_slot[i];
     if (k < 0) continue;
-    double* base = work + (size_t)k * 5 * nc2;
+    double* base = work + (size_t)k * slot_words;
     fl.AX[fl.n] = AX[i];
     fl.coulomb[fl.n] = types[i] == CQ_COULOMB;
     fl.A[fl.n] = base + (types[i] == CQ_COULOMB ? 1 : 3) * nc2;
@@ -2555,7 +2766,8 @@ int cq_get_work_stats(cq_ctx_t* c, double* out, int max_n) {
       hipLaunchKernelGGL(work_stats_kernel, dim3(persistent_grid()), dim3(WG), 0, c->stream,
                          c->d_tasks.p + m.task_off, c->d_segs.p + m.seg_off, c->batch_slots[tb][k][0], c->d_ovf.p + k,
                          c->d_groups[tb].p,
-                         c->d_uorder.p, m.flip, c->d_pairs.p, c->d_shells.p, acc.p + 4 * k);
+                         (tb == 2 && c->own_blocks() ? c->d_uorder_m : c->d_uorder).p, m.flip, c->d_pairs.p,
+                         tb == 2 ? c->mpblk : PRIM_BLOCK, tb == 2 ? c->mublk : UNI_BLOCK, c->d_shells.p, acc.p + 4 * k);
       HIPCHK(hipGetLastError());
     }
     std::vector<double> h((size_t)4 * kNumClassPairs);

@@ -3,15 +3,18 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 // Boys-function table: F_m(T_i) on T_i = i * BOYS_STEP, i = 0..BOYS_NGRID-1, for
-// m = 0..BOYS_MTAB-1, plus exp(-T_i) in the last column.  Each kernel stages the
-// slice m = L..L+7 and the exp column (9 doubles per grid point) into LDS.
-#define BOYS_STEP 0.1
-#define BOYS_INV_STEP 10.0
+// m = 0..BOYS_MTAB-1, plus exp(-T_i) in the last column.  Each kernel stages a scaled slice
+// (9 doubles per grid point) into LDS, with one more row for the asymptotic range (stage_boys).
+// The step is just below 0.1 and short in binary (13107 / 2^17), so that i * step is exact.
+#define BOYS_STEP (13107.0 / 131072.0)
+#define BOYS_INV_STEP (131072.0 / 13107.0)
 #define BOYS_TMAX 36.0
 #define BOYS_NGRID 361
 #define BOYS_MTAB 24
+#define BOYS_ROWS (BOYS_NGRID + 1)
 #define BOYS_LDS_W 9
 
 // One primitive pair of a shell pair (a, b):
@@ -29,7 +32,7 @@ struct alignas(16) PrimPair {
 };
 
 // Per shell pair, in kernel orientation (l_a >= l_b).
-struct PairInfo {
+struct alignas(16) PairInfo {
   int a, b;        // shells in kernel orientation
   int s1, s2;      // canonical shells (s1 >= s2), as the reference loop visits them
   int p0, p1;      // primitive-pair range in the PrimPair array
@@ -48,6 +51,7 @@ struct QuartetArgs {
   bool ket_uniform;          // every lane of the wavefront holds the same ket pair
   bool bra_swap, ket_swap;   // pair held reversed relative to its canonical (s1 >= s2) order
   int ar, br, cr, dr;        // LDS rows of the swept pair's shells (PairInfo::ar, br)
+  int jb, jk;                // PairInfo::joff of the bra and of the ket
 };
 
 // One density slot per kernel launch (a call with several densities runs one pass per slot).
@@ -57,7 +61,14 @@ struct JKArgs {
   int lds_n;                     // rows of an LDS accumulator column (or row): the largest
                                  // molecule's functions of the swept pair class's shells
   const int* rowfn;              // Cartesian function of LDS row r: rowfn[loff + r]
-  const double* D[MAX_SLOTS];    // density in the Cartesian basis, row-major ncart x ncart
+  int pblk, ublk;                // primitive block sizes: lane side, uniform side
+  // Density in the Cartesian basis, three copies, so that the digestion reads it along its lanes
+  // (with lanes across rows each lane touches a cache line of its own: 8.4 GB of L2 reads per
+  // (ss|ps) launch on (H2O)16/cc-pVDZ).  The uniform pair's functions pick rows (a scalar base),
+  // the lanes' functions the columns.
+  const double* D[MAX_SLOTS];    // row-major ncart x ncart
+  const double* Dt[MAX_SLOTS];   // its transpose
+  const double* Dp[MAX_SLOTS];   // blocks X(s2,s1) of the shell pairs in pair order (PairInfo::joff)
   // Accumulators.  An FP64 atomic whose wavefront hits 64 consecutive doubles runs at 163 G/s
   // for the whole chip, at scattered or strided addresses at 23 G/s (measured on 160000
   // doubles), so the LDS flushes address memory along their lanes: J in pair order, the K
@@ -71,6 +82,12 @@ struct JKArgs {
   int do_k[MAX_SLOTS];
   const int* nonsym;             // device flags: density slot is not symmetric
 };
+
+// Element `off` bytes behind a wavefront-uniform row: one scalar base and a 32-bit lane offset
+// (an int index would cost a 64-bit address per lane and load)
+__device__ __forceinline__ double row_at(const double* __restrict__ row, unsigned off) {
+  return *(const double*)((const char*)row + off);
+}
 
 // a * b + c rounded once, in the integral type of a kernel (FP64, or FP32 for the mixed
 // window's kernels)
@@ -89,103 +106,137 @@ __device__ __forceinline__ double rsqrt_f64(double x) {
   return __builtin_fma(y * e, c, y);
 }
 
-// F_0..F_L at T.  T < 36: 8-term Taylor expansion of F_L about the nearest grid point
-// (|dT| <= 0.05, truncation below 1e-15 relative), F(T0 - dT) = sum_k F_{L+k}(T0) dT^k / k!;
-// for L >= 2 exp(-T) = exp(-T0) exp(dT) by an 8-term series and the downward recursion
-// F_m = (2T F_{m+1} + e^-T) / (2m+1).  For L <= 1 the staged coefficients are already divided
-// by k! (one FMA per term), and for L = 1 the slice holds F_0..F_8 / k!: F_0 is the polynomial
-// and F_1 = -dF_0/dT its derivative in dT, both from one Horner pass (8 terms each).
-// T >= 36: F_0 = sqrt(pi/T)/2, upward recursion F_{m+1} = (2m+1)/(2T) F_m (the dropped
-// e^-T term is below 2.4e-16).
+// Scaled Boys values of a primitive quartet with exponents p, q, s = p + q and centre distance r
+// (or, with s = 1 and pq2 = 2 p, of a charge distribution and a point charge).  One rsqrt serves
+// the prefactor, the exponent and the asymptotic range:
+//   T = p q r^2 / s < 36:  x = s,          b2 = 2 p q / s = 2 alpha,  T2 = r^2 b2 = 2 T
+//   T >= 36:               x = 2 p q r^2,  b2 = 1 / r^2
+// with rs = 1/sqrt(x), b2 = 2 p q rs^2; then for both
+//   (2 alpha)^n F_n(T) / sqrt(s) = rs b2^n G_n,
+// G_n = F_n(T) below 36 and sqrt(pi/2) (2n-1)!! above (F_n's asymptotic form; the dropped e^-T
+// term is below 2.4e-16), which is the table's last row: nothing is selected behind the table.
+// Selecting the argument instead of evaluating both ranges takes the second rsqrt and the
+// selects out of the primitive loop: (ss|ps) 68 -> 57 VALU instructions per primitive quartet.
+struct BoysArg {
+  double rs, b2, T2;
+  bool big;
+};
+__device__ __forceinline__ BoysArg boys_arg(double s, double pq2, double r2) {
+  BoysArg a;
+  const double xb = pq2 * r2;
+  a.big = xb >= 2.0 * BOYS_TMAX * s;
+  a.rs = rsqrt_f64(a.big ? xb : s);
+  a.b2 = pq2 * (a.rs * a.rs);
+  a.T2 = r2 * a.b2;
+  return a;
+}
+
+// G_0..G_L of a (below 36: F_0..F_L).  Table row i (i * 2 step nearest to T2, or the asymptotic
+// row), 8-term Taylor expansion in d = T2_i - T2 (|dT| <= 0.05, truncation below 1e-15 relative):
+// the staged coefficients carry 1 / (2^k k!), one FMA per term.  L = 1: F_0 by 9 terms and
+// F_1 = -dF_0/dT as the same pass's derivative (d counts in 2T, hence twice it).  L >= 2: F_L, then
+// F_m = (2T F_{m+1} + e^-T) / (2m+1) downward with e^-T = e^-T_i e^dT (8 terms); the asymptotic
+// row holds G_L with e^-T = 0, and T2 = 1 makes the same recursion G_m = G_{m+1} / (2m+1) (set
+// to exactly 1: r^2 b2 would carry its rounding through L steps).  Errors against long double
+// over random primitive quartets equal those of evaluating both ranges (3.7e-16 for F_0 of
+// L = 0, 8.7e-16 of L = 8).
 template <int L>
-__device__ __forceinline__ void boys_eval(double T, const double* __restrict__ lds, double* F) {
-  // Both branches are evaluated and the result selected, so that the primitive loop has no
-  // divergent branch (unrolled iterations then interleave): the table path at min(T, T_max)
-  // (index always in range), the asymptotic path at max(T, T_max).
-  const bool big = T >= BOYS_TMAX;
-  const double Tt = fmin(T, BOYS_TMAX);   // (the table's last point for the asymptotic range)
-  const int i = (int)(Tt * BOYS_INV_STEP + 0.5);
-  const double dT = (double)i * BOYS_STEP - Tt;
-  const double* f = lds + i * BOYS_LDS_W;
-  if constexpr (L >= 2) {
-    // unscaled coefficients F_L..F_{L+7} (measured faster for these kernels than the scaled form)
-    double s = f[7];
-    s = f[6] + s * dT * (1.0 / 7.0);
-    s = f[5] + s * dT * (1.0 / 6.0);
-    s = f[4] + s * dT * (1.0 / 5.0);
-    s = f[3] + s * dT * (1.0 / 4.0);
-    s = f[2] + s * dT * (1.0 / 3.0);
-    s = f[1] + s * dT * (1.0 / 2.0);
-    s = f[0] + s * dT;
-    const double Ta = big ? T : BOYS_TMAX;
-    const double rs = rsqrt_f64(Ta);
-    double fa = 0.88622692545275801365 * rs;   // sqrt(pi)/2 T^-1/2
-    // table: F_L by Taylor, then downward recursion with e^{-T} (Taylor about T_i)
-    double e = 1.0 + dT * (1.0 / 8.0);
-    e = 1.0 + dT * (1.0 / 7.0) * e;
-    e = 1.0 + dT * (1.0 / 6.0) * e;
-    e = 1.0 + dT * (1.0 / 5.0) * e;
-    e = 1.0 + dT * (1.0 / 4.0) * e;
-    e = 1.0 + dT * (1.0 / 3.0) * e;
-    e = 1.0 + dT * (1.0 / 2.0) * e;
-    e = 1.0 + dT * e;
-    e *= f[8];
-    const double T2 = 2.0 * Tt;
-    double Ft[L + 1];
-    Ft[L] = s;
+__device__ __forceinline__ void boys_table(const BoysArg& a, const double* __restrict__ lds, double* G) {
+  constexpr double step2 = 2.0 * BOYS_STEP, shift = 6755399441055744.0;   // 1.5 * 2^52
+  // L <= 1: the asymptotic row's own T2, so that d = 0; L >= 2: 1, and the row index on its own
+  // (the row's higher coefficients are zero)
+  const double Tt = a.big ? (L <= 1 ? BOYS_NGRID * step2 : 1.0) : a.T2;
+  const double t = __builtin_fma(Tt, 0.5 * BOYS_INV_STEP, shift);   // nearest integer in the low bits
+  const unsigned i = L >= 2 && a.big ? BOYS_NGRID : (unsigned)__double2loint(t);
+  const double d = __builtin_fma(t - shift, step2, -Tt);
+  const double* f = lds + __umul24(i, BOYS_LDS_W);
+  if constexpr (L == 0) {
+    double p = f[7];
 #pragma unroll
-    for (int m = L - 1; m >= 0; --m) Ft[m] = (T2 * Ft[m + 1] + e) * (1.0 / (2 * m + 1));
-    // asymptotic: F_0 = sqrt(pi/T)/2, upward F_{m+1} = F_m (2m+1) / (2T)
-    const double hr = 0.5 * rs * rs;
-    F[0] = big ? fa : Ft[0];
+    for (int k = 6; k >= 0; --k) p = __builtin_fma(p, d, f[k]);
+    G[0] = p;
+  } else if constexpr (L == 1) {
+    // (the first step of the derivative's recurrence, dp = 0 d + f[8], taken out)
+    double dp = f[8], p = __builtin_fma(f[8], d, f[7]);
 #pragma unroll
-    for (int m = 0; m < L; ++m) {
-      fa = fa * (double)(2 * m + 1) * hr;
-      F[m + 1] = big ? fa : Ft[m + 1];
+    for (int k = 6; k >= 0; --k) {
+      dp = __builtin_fma(dp, d, p);
+      p = __builtin_fma(p, d, f[k]);
     }
+    G[0] = p;
+    G[1] = 2.0 * dp;
   } else {
-    const double Ta = big ? T : BOYS_TMAX;
-    const double rs = rsqrt_f64(Ta);
-    const double fa = 0.88622692545275801365 * rs;   // sqrt(pi)/2 T^-1/2
-    if constexpr (L == 1) {
-      // (the first step of the derivative's recurrence, dp = 0 dT + f[8], taken out: the
-      // compiler cannot fold the product with zero itself)
-      double dp = f[8], p = __builtin_fma(f[8], dT, f[7]);
+    double p = f[7];
 #pragma unroll
-      for (int k = 6; k >= 0; --k) {
-        dp = __builtin_fma(dp, dT, p);
-        p = __builtin_fma(p, dT, f[k]);
-      }
-      F[0] = big ? fa : p;
-      F[1] = big ? fa * (0.5 * rs * rs) : dp;
-    } else {
-      double s = f[7];
+    for (int k = 6; k >= 0; --k) p = __builtin_fma(p, d, f[k]);
+    constexpr double c[9] = {1.0, 1.0 / 2, 1.0 / 8, 1.0 / 48, 1.0 / 384, 1.0 / 3840, 1.0 / 46080, 1.0 / 645120,
+                             1.0 / 10321920};   // 1 / (2^k k!)
+    double e = c[8];
 #pragma unroll
-      for (int k = 6; k >= 0; --k) s = __builtin_fma(s, dT, f[k]);
-      F[0] = big ? fa : s;
-    }
+    for (int k = 7; k >= 0; --k) e = __builtin_fma(e, d, c[k]);
+    e *= f[8];
+    G[L] = p;
+#pragma unroll
+    for (int m = L - 1; m >= 0; --m) G[m] = __builtin_fma(Tt, G[m + 1], e) * (1.0 / (2 * m + 1));
   }
 }
 
-// FP32 integrals take the Boys values from the FP64 evaluation, rounded.
+// Rb_n = (2 alpha)^n F_n(T) K / sqrt(s), n = 0..L (arguments as in boys_arg).
 template <int L>
-__device__ __forceinline__ void boys_eval(double T, const double* __restrict__ lds, float* F) {
-  double Fd[L + 1];
-  boys_eval<L>(T, lds, Fd);
+__device__ __forceinline__ void boys_scaled(double s, double pq2, double r2, double K, const double* __restrict__ lds,
+                                            double* Rb) {
+  const BoysArg a = boys_arg(s, pq2, r2);
+  double G[L + 1];
+  boys_table<L>(a, lds, G);
+  double pw = K * a.rs;
 #pragma unroll
-  for (int m = 0; m <= L; ++m) F[m] = (float)Fd[m];
+  for (int n = 0; n <= L; ++n) {
+    Rb[n] = G[n] * pw;
+    pw *= a.b2;
+  }
+}
+// The FP32 integrals' form: F_n in double, rounded, and the prefactors' powers in float (the
+// asymptotic range on its own: folding it into the prefactor would round differently).
+template <int L>
+__device__ __forceinline__ void boys_scaled(double s, double pq2, double r2, double K, const double* __restrict__ lds,
+                                            float* Rb) {
+  BoysArg a;
+  a.rs = rsqrt_f64(s);
+  a.b2 = pq2 * (a.rs * a.rs);
+  a.T2 = fmin(r2 * a.b2, 2.0 * BOYS_TMAX);
+  a.big = false;
+  const bool big = r2 * a.b2 >= 2.0 * BOYS_TMAX;
+  double F[L + 1];
+  boys_table<L>(a, lds, F);
+  const double T = big ? 0.5 * (r2 * a.b2) : BOYS_TMAX;
+  const double rs = rsqrt_f64(T);
+  double fa = 0.88622692545275801365 * rs;   // sqrt(pi)/2 T^-1/2
+  const double hr = 0.5 * rs * rs;           // F_{m+1} = F_m (2m+1) / (2T)
+  float pw = (float)(K * a.rs);
+#pragma unroll
+  for (int n = 0; n <= L; ++n) {
+    Rb[n] = (float)(big ? fa : F[n]) * pw;
+    pw *= (float)a.b2;
+    fa = fa * (double)(2 * n + 1) * hr;
+  }
 }
 
 // Stage the Boys slice for total angular momentum L into LDS (whole workgroup): per grid point
-// F_{L+c}, c = 0..7, and e^{-T_i}; divided by c! for L = 0, and F_c / c!, c = 0..8, for L = 1.
+// F_{L+c} / (2^c c!), c = 0..7, and e^{-T_i}; for L = 1 F_c / (2^c c!), c = 0..8.  The last row
+// is the asymptotic range's: G_L (L = 1: G_0 and half of G_1) and zeros.
 __device__ __forceinline__ void stage_boys(const double* __restrict__ tab, int L, double* lds) {
-  constexpr double ifact[9] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040,
-                               1.0 / 40320};
+  constexpr double ifact[9] = {1.0, 1.0 / 2, 1.0 / 8, 1.0 / 48, 1.0 / 384, 1.0 / 3840, 1.0 / 46080, 1.0 / 645120,
+                               1.0 / 10321920};
   for (int k = threadIdx.x; k < BOYS_NGRID * BOYS_LDS_W; k += blockDim.x) {
     const int i = k / BOYS_LDS_W, c = k - i * BOYS_LDS_W;
-    lds[k] = L == 1 ? tab[i * (BOYS_MTAB + 1) + c] * ifact[c]
-             : L == 0 ? (c < 8 ? tab[i * (BOYS_MTAB + 1) + c] * ifact[c] : tab[i * (BOYS_MTAB + 1) + BOYS_MTAB])
-                      : (c < 8) ? tab[i * (BOYS_MTAB + 1) + L + c] : tab[i * (BOYS_MTAB + 1) + BOYS_MTAB];
+    lds[k] = L == 1 || c < 8 ? tab[i * (BOYS_MTAB + 1) + (L == 1 ? 0 : L) + c] * ifact[c]
+                             : tab[i * (BOYS_MTAB + 1) + BOYS_MTAB];
+  }
+  if (threadIdx.x < BOYS_LDS_W) {
+    double g = 1.25331413731550025121;   // sqrt(pi / 2)
+    if (L >= 2)
+      for (int n = 1; n <= L; ++n) g *= 2 * n - 1;
+    lds[BOYS_NGRID * BOYS_LDS_W + threadIdx.x] = threadIdx.x == 0 ? g : L == 1 && threadIdx.x == 1 ? 0.5 * g : 0.0;
   }
   __syncthreads();
 }
@@ -198,32 +249,53 @@ struct Segment {
 
 // Primitive blocks.  A pair with many primitive pairs is split into blocks so that one heavily
 // contracted quartet becomes several shorter lane tasks (the digestion is linear in the
-// integrals, so partial sums digest independently): blocks of PRIM_BLOCK on the per-lane side
-// of a task list, blocks of UNI_BLOCK on the wavefront-uniform side (each uniform block is a
-// separate work item that repeats the per-lane J atomics and the LDS flush, so it is kept
-// coarse).  Task entries and segments carry a block code in bits 24..31 of the pair index:
-// 0 = the whole primitive range, k >= 1 = primitives [p0 + (k-1) B, min(p1, p0 + k B)).
+// integrals, so partial sums digest independently): blocks of JKArgs::pblk on the per-lane side
+// of a task list, blocks of JKArgs::ublk on the wavefront-uniform side (each uniform block is a
+// separate work item with an LDS flush of its own).  Task entries and segments carry a block
+// code in bits 24..31 of the pair index: 0 = the whole primitive range, k >= 1 = primitives
+// [p0 + (k-1) B, min(p1, p0 + k B)).  PRIM_BLOCK and UNI_BLOCK are the sizes of the launches per
+// class pair (and PRIM_BLOCK of the Schwarz quartets).
 #define PRIM_BLOCK 8
 #define UNI_BLOCK 32
 #define PAIR_MASK 0xFFFFFFu
 __host__ __device__ __forceinline__ unsigned pair_of(unsigned code) { return code & PAIR_MASK; }
 __host__ __device__ __forceinline__ unsigned block_of(unsigned code) { return code >> 24; }
-template <int BLK = PRIM_BLOCK>
-__host__ __device__ __forceinline__ void prim_range(const PairInfo& P, unsigned blk, int& p0, int& p1) {
+__host__ __device__ __forceinline__ void prim_range(const PairInfo& P, unsigned blk, int size, int& p0, int& p1) {
   if (blk == 0) {
     p0 = P.p0;
     p1 = P.p1;
   } else {
-    p0 = P.p0 + (int)(blk - 1) * BLK;
-    p1 = P.p1 < p0 + BLK ? P.p1 : p0 + BLK;
+    p0 = P.p0 + (int)(blk - 1) * size;
+    p1 = P.p1 < p0 + size ? P.p1 : p0 + size;
   }
 }
 
-// Wavefront-reduced add into LDS (every lane targets the same LDS word).
-__device__ __forceinline__ void wave_add_lds(double* p, double v) {
+// Sums over the wavefront's lanes of up to four values, added to the LDS words p[0 .. n - 1].
+// The FP64 matrix unit, idle otherwise, does the first factor of four: v_mfma_f64_4x4x4 with
+// A = 1 (lane = 16 k + 4 b + j holds B[k][j] of block b and D[i = lane / 16][j]) sums a value over
+// k into every lane; lanes 16 i .. 16 i + 15 keep value i's, two DPP steps sum over j and four
+// lanes per value (b) add to its word.  (Ones in row i only would merge the four values without
+// the selects, but 0 x inf would carry an infinity of one value into the other three.)
+// 4 matrix + 12 vector instructions and one LDS atomic for four values, where a shuffle tree
+// takes 48 LDS and 24 vector instructions.
+template <int N>
+__device__ __forceinline__ void wave_sum_lds(double* p, const double (&v)[N]) {
+  static_assert(N >= 1 && N <= 4, "up to four values");
+  const int lane = (int)(threadIdx.x & 63);
+  double d = 0.0;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  if ((threadIdx.x & 63) == 0) atomicAdd(p, v);
+  for (int i = 0; i < N; ++i) {
+    const double di = __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, v[i], 0.0, 0, 0, 0);
+    d = i == 0 || (lane >> 4) == i ? di : d;
+  }
+  auto quad = [](double x, auto ctrl) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), decltype(ctrl)::value, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), decltype(ctrl)::value, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+  };
+  d += quad(d, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+  d += quad(d, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  if ((lane & 3) == 0 && (N == 4 || lane < 16 * N)) atomicAdd(p + (lane >> 4), d);
 }
 
 // Atomic add of a value whose target is the same on every lane when `uniform` (wavefront-

@@ -11,7 +11,8 @@ digested into J and K (forward updates) before the next one starts.
 Two kernels are instantiated per class from the generated core:
   * eri_block_<cls>: writes the contracted Cartesian block (ab|cd) of each task (used for
     Schwarz bounds and for per-quartet parity tests);
-  * eri_jk_<cls>: digests the block into the forward J/K accumulators.
+  * eri_grp_<cls> / eri_grpb_<cls>: digest the block into the J/K accumulators.
+A merged kernel per tier runs several class pairs in one launch (small molecules).
 
 The algorithm restated here replaces libint2::Engine::compute as called at
 include/aointegrals/aointegrals_contract.h:138-143; the digestion reproduces the scatter at
@@ -133,6 +134,9 @@ def mul(*fs):
 
 # --------------------------------------------------------------------------- R integrals
 class RGen:
+    """R_tuv from the scaled Boys values Rb_n = (2 alpha)^n F_n prefactor.  With the sign of
+    (-2 alpha)^n left out at every order n, the recursion R^n_{t+1} = (P - Q) R^{n+1}_t + t R^{n+1}_{t-1}
+    becomes (Q - P) R^{n+1}_t - t R^{n+1}_{t-1}: the signs cost nothing."""
     def __init__(self, em: Emitter, L: int):
         self.em = em
         self.L = L
@@ -149,18 +153,18 @@ class RGen:
         if t > 0:
             a = self.get(n + 1, t - 1, u, v)
             b = self.get(n + 1, t - 2, u, v) if t > 1 else None
-            X, k = "PQx", t - 1
+            X, k = "QPx", t - 1
         elif u > 0:
             a = self.get(n + 1, t, u - 1, v)
             b = self.get(n + 1, t, u - 2, v) if u > 1 else None
-            X, k = "PQy", u - 1
+            X, k = "QPy", u - 1
         else:
             a = self.get(n + 1, t, u, v - 1)
             b = self.get(n + 1, t, u, v - 2) if v > 1 else None
-            X, k = "PQz", v - 1
+            X, k = "QPz", v - 1
         name = f"R{n}_{t}_{u}_{v}"
         if b is not None:
-            expr = f"{X}*{a} + {b}" if k == 1 else f"{X}*{a} + {lit(k)}*{b}"
+            expr = f"{X}*{a} - {b}" if k == 1 else f"{X}*{a} - {lit(k)}*{b}"
         else:
             expr = f"{X}*{a}"
         self.em(f"const {RT} {name} = {expr};")
@@ -171,6 +175,15 @@ class RGen:
 # --------------------------------------------------------------------------- class core
 REG_SOFT = 125     # live doubles targeted by the chunk-by-c plan (about 250 VGPRs at most)
 REG_HARD = 170     # above this even one c component per chunk spills: use (c,d) chunks
+
+
+# Wavefronts per SIMD that the default group kernel of a class pair is compiled for (its
+# __launch_bounds__; 1: no bound).  Left alone, the scheduler spends registers on latency it could
+# hide with more wavefronts: (ss|ps) 103 registers (4 wavefronts), (ps|ps) 148 (3, and a
+# 512-thread workgroup needs two per SIMD, so one workgroup per CU), (dp|ds) 276 (1).  A bound is
+# as high as it goes while what spills is the flush's addresses outside the primitive loops.
+WAVES = {"ssss": 8, "ssps": 6, "psps": 4, "sspp": 4, "ssds": 4, "psds": 2, "ssdp": 2, "ppps": 2, "pppp": 2,
+         "ppds": 2, "dsds": 2, "dpps": 2, "dppp": 2, "dpds": 2, "dpdp": 2, "ddss": 2, "ddps": 2}
 
 
 def plan_class(LA, LB, LC, LD):
@@ -253,6 +266,7 @@ def gen_class(LA, LB, LC, LD, kind: str) -> str:
         em("for (int ip = q.bra_p0; ip < q.bra_p1; ++ip) {")
         em.ind += 1
         em("const PrimPair bp = q.prim[ip];")
+        em("const double bp_2p = 2.0 * bp.p;")
         em("const R bp_K = R(bp.K), bp_o2p = R(bp.o2p);")
         em("const R bp_PA0 = R(bp.PA[0]), bp_PA1 = R(bp.PA[1]), bp_PA2 = R(bp.PA[2]);")
         em("const R bp_PB0 = R(bp.PB[0]), bp_PB1 = R(bp.PB[1]), bp_PB2 = R(bp.PB[2]);")
@@ -265,20 +279,13 @@ def gen_class(LA, LB, LC, LD, kind: str) -> str:
         em("for (int iq = q.ket_p0; iq < q.ket_p1; ++iq) {")
         em.ind += 1
         em("const PrimPair kp = q.prim[iq];")
-        # the Boys argument and PQ are formed in double, the rest in R
-        em("const double pqd = bp.p + kp.p;")
-        em("const double rsd = rsqrt_f64(pqd);")
-        em("const double alphad = bp.p * kp.p * (rsd * rsd);")
-        em("const double PQxd = bp.P[0] - kp.P[0], PQyd = bp.P[1] - kp.P[1], PQzd = bp.P[2] - kp.P[2];")
-        em(f"R F[{L + 1}];")
-        em(f"boys_eval<{L}>(alphad * (PQxd * PQxd + PQyd * PQyd + PQzd * PQzd), boys_lds, F);")
-        em("const R PQx = R(PQxd), PQy = R(PQyd), PQz = R(PQzd);")
-        em("const R alpha = R(alphad);")
-        em("R pw = R(kp.K * rsd);   // K of both pairs carry sqrt(2 pi^(5/2)) each")
+        # the Boys argument and Q - P are formed in double, the rest in R
+        em("const double QPxd = kp.P[0] - bp.P[0], QPyd = kp.P[1] - bp.P[1], QPzd = kp.P[2] - bp.P[2];")
+        em(f"R Rb[{L + 1}];   // (K of both pairs carry sqrt(2 pi^(5/2)) each)")
+        em(f"boys_scaled<{L}>(bp.p + kp.p, bp_2p * kp.p, QPxd * QPxd + QPyd * QPyd + QPzd * QPzd, kp.K, boys_lds, Rb);")
+        em("const R QPx = R(QPxd), QPy = R(QPyd), QPz = R(QPzd);")
         for n in range(L + 1):
-            em(f"const R Rb{n} = F[{n}] * pw;")
-            if n < L:
-                em("pw *= R(-2.0) * alpha;")
+            em(f"const R Rb{n} = Rb[{n}];")
         em("const R kp_o2p = R(kp.o2p);")
         em("const R kp_PA0 = R(kp.PA[0]), kp_PA1 = R(kp.PA[1]), kp_PA2 = R(kp.PA[2]);")
         em("const R kp_PB0 = R(kp.PB[0]), kp_PB1 = R(kp.PB[1]), kp_PB2 = R(kp.PB[2]);")
@@ -355,31 +362,34 @@ def gen_class(LA, LB, LC, LD, kind: str) -> str:
     em.ind = 0
     em("}")
     if kind == "jk":
-        em(f"constexpr int kChunks_{name} = {1 if persist else len(chunks)};")
-        em(f"constexpr int kNC_{name} = {NC}, kND_{name} = {ND}, kNA_{name} = {NA}, kNB_{name} = {NB};")
+        em(f"struct Cls_{name} {{   // sizes and quartet function for the group kernels")
+        em(f"  static constexpr int NCH = {1 if persist else len(chunks)}, L = {L}, WAVES = {WAVES.get(name, 1)};")
+        em(f"  static constexpr int NA = {NA}, NB = {NB}, NC = {NC}, ND = {ND};")
+        em("  template <int DIG, typename R>")
+        em("  static __device__ __forceinline__ void jk(const QuartetArgs& q, const JKArgs& jk, const double* __restrict__ boys_lds, int chunk, double* colC, double* colD, double* jcdL, double* jl) {")
+        em(f"    quartet_jk_{name}<1, DIG, R>(q, jk, boys_lds, chunk, colC, colD, jcdL, jl);")
+        em("  }")
+        em("};")
     return "\n".join(em.lines) + "\n"
 
 
 def _jk_addressing(em: Emitter):
-    """Index forms for the Coulomb scatter in each pair's canonical order (s1 >= s2).
+    """Index forms for the Coulomb scatter of a non-symmetric density in each pair's canonical
+    order (s1 >= s2).
 
     The reference's updates G(1,2) += X(4,3) v, G(3,4) += X(2,1) v (and the transposed
     G(2,1) += X(3,4) v, G(4,3) += X(1,2) v; aointegrals_contract.h:153-157) refer to the
     canonical order inside each pair; the kernel may hold a pair reversed (bra_swap,
     ket_swap).  Address of element (i, j) of a block = base + i*stride_i + j*stride_j with
     i the kernel-order a (or c) component and j the b (or d) component:
-      tab: (1,2) = (s1,s2) of the bra   xba: (2,1)
-      tcd: (3,4) = (s3,s4) of the ket   xdc: (4,3)"""
+      tab: (1,2) = (s1,s2) of the bra   tcd: (3,4) = (s3,s4) of the ket
+    (X(2,1) and X(4,3) come in kernel order from the pair-ordered density)."""
     em("const int N = jk.ncart;")
     em("const int LN = jk.lds_n;   // LDS accumulator rows: the swept shells' functions")
     em("const int tab = q.bra_swap ? q.b0 * N + q.a0 : q.a0 * N + q.b0;")
     em("const int tab_a = q.bra_swap ? 1 : N, tab_b = q.bra_swap ? N : 1;")
-    em("const int xba = q.bra_swap ? q.a0 * N + q.b0 : q.b0 * N + q.a0;")
-    em("const int xba_a = q.bra_swap ? N : 1, xba_b = q.bra_swap ? 1 : N;")
     em("const int tcd = q.ket_swap ? q.d0 * N + q.c0 : q.c0 * N + q.d0;")
     em("const int tcd_c = q.ket_swap ? 1 : N, tcd_d = q.ket_swap ? N : 1;")
-    em("const int xdc = q.ket_swap ? q.c0 * N + q.d0 : q.d0 * N + q.c0;")
-    em("const int xdc_c = q.ket_swap ? N : 1, xdc_d = q.ket_swap ? 1 : N;")
 
 
 def _ab(form, ia, ib):
@@ -388,6 +398,17 @@ def _ab(form, ia, ib):
 
 def _cd(form, ic, idd):
     return f"{form} + {ic} * {form}_c + {idd} * {form}_d"
+
+
+def _emit_jab(em: Emitter, NA, NB, var, live):
+    """J of the bra: summed over the wavefront for a uniform bra (DIG 2), four components at a
+    time, else added to the lane's own slot."""
+    comps = [(ia, ib) for ia in range(NA) for ib in range(NB)]
+    for g in range(0, len(comps), 4):
+        part = comps[g:g + 4]
+        em(f"{{ const double js[{len(part)}] = {{{', '.join(f'double(dg * {var(ia, ib)})' for ia, ib in part)}}};")
+        em(f"  if constexpr (DIG == 2) wave_sum_lds(&jcdL[{g}], js);")
+        em(f"  else if ({live}) for (int n = 0; n < {len(part)}; ++n) atomicAdd(&jl[{g} + n], js[n]); }}")
 
 
 def gen_digest_chunk(em: Emitter, NA, NB, NC, ND, ks, persist):
@@ -405,6 +426,9 @@ def gen_digest_chunk(em: Emitter, NA, NB, NC, ND, ks, persist):
     em("for (int s = 0; s < NSLOT; ++s) {")
     em.ind += 1
     em("const double* __restrict__ D = jk.D[s];")
+    em("const double* __restrict__ xb = jk.Dp[s] + q.jb;   // X(2,1) of the bra")
+    em("const double* __restrict__ Dt = jk.Dt[s];")
+    em("const double* __restrict__ xk = jk.Dp[s] + q.jk;   // X(4,3) of the ket")
     _jk_addressing(em)
     em("const R dg = R(q.deg);")
     em("const R hk = R(0.5 * q.deg);")
@@ -416,21 +440,24 @@ def gen_digest_chunk(em: Emitter, NA, NB, NC, ND, ks, persist):
         for ia in range(NA):
             for ib in range(NB):
                 em(f"R jab_{ia}_{ib} = R(0);")
-    for (ic, idd) in ks:
-        em(f"{{ const R x43 = R(D[{_cd('xdc', ic, idd)}]);")
-        em("  R jcd = R(0);")
-        for ia in range(NA):
-            for ib in range(NB):
-                em(f"  jcd += o_{ia}_{ib}_{ic}_{idd} * R(D[{_ab('xba', ia, ib)}]);")
-                tgt = f"jab_{ia}_{ib}[s]" if persist else f"jab_{ia}_{ib}"
-                em(f"  {tgt} += o_{ia}_{ib}_{ic}_{idd} * x43;")
-        em(f"  if constexpr (DIG == 2) {{ if (live) atomicAdd(&jl[{ic * ND + idd}], double(dg * jcd)); }}")
-        em(f"  else wave_add_lds(&jcdL[{ic * ND + idd}], double(dg * jcd)); }}")
+    # (a chunk's ket components are consecutive: four at a time share one reduction)
+    for g in range(0, len(ks), 4):
+        part = ks[g:g + 4]
+        em(f"{{ double js[{len(part)}];")
+        for n, (ic, idd) in enumerate(part):
+            em(f"  {{ const R x43 = R(xk[{ic * ND + idd}]);")
+            em("    R jcd = R(0);")
+            for ia in range(NA):
+                for ib in range(NB):
+                    em(f"    jcd += o_{ia}_{ib}_{ic}_{idd} * R(xb[{ia * NB + ib}]);")
+                    tgt = f"jab_{ia}_{ib}[s]" if persist else f"jab_{ia}_{ib}"
+                    em(f"    {tgt} += o_{ia}_{ib}_{ic}_{idd} * x43;")
+            em(f"    js[{n}] = double(dg * jcd); }}")
+        base = part[0][0] * ND + part[0][1]
+        em(f"  if constexpr (DIG == 2) {{ if (live) for (int n = 0; n < {len(part)}; ++n) atomicAdd(&jl[{base} + n], js[n]); }}")
+        em(f"  else wave_sum_lds(&jcdL[{base}], js); }}")
     if not persist:
-        for ia in range(NA):
-            for ib in range(NB):
-                em(f"if constexpr (DIG == 2) wave_add_lds(&jcdL[{ia * NB + ib}], double(dg * jab_{ia}_{ib}));")
-                em(f"else if (live) atomicAdd(&jl[{ia * NB + ib}], double(dg * jab_{ia}_{ib}));")
+        _emit_jab(em, NA, NB, lambda ia, ib: f"jab_{ia}_{ib}", "live")
     em("if (ns) {")
     em.ind += 1
     for (ic, idd) in ks:
@@ -451,9 +478,13 @@ def gen_digest_chunk(em: Emitter, NA, NB, NC, ND, ks, persist):
     em.ind += 1
 
     def X(r0, ri, c0, ci, trans):
+        """X(r0 + ri, c0 + ci) (trans: X^T), r0 a bra and c0 a ket function.  Uniform ket (DIG 0
+        and 1): along a row of the transpose (of D for X^T), the lane's function the column;
+        uniform bra (DIG 2): along a row of D, the lane's ket function the column."""
         if trans:
-            return f"R(D[(q.{c0} + {ci}) * N + q.{r0} + {ri}])"
-        return f"R(D[(q.{r0} + {ri}) * N + q.{c0} + {ci}])"
+            return f"R(row_at(D + (long)(q.{c0} + {ci}) * N, 8u * (unsigned)q.{r0} + {8 * ri}u))"
+        return (f"R(DIG == 2 ? row_at(D + (long)(q.{r0} + {ri}) * N, 8u * (unsigned)q.{c0} + {8 * ci}u) : "
+                f"row_at(Dt + (long)(q.{c0} + {ci}) * N, 8u * (unsigned)q.{r0} + {8 * ri}u))")
 
     NCOL = NC + ND
 
@@ -548,10 +579,7 @@ def gen_digest_final(em: Emitter, NA, NB, NC, ND):
     em("const R dg = R(q.deg);")
     em("const R hk = R(0.5 * q.deg);")
     em("if (jk.do_j[s]) {")
-    for ia in range(NA):
-        for ib in range(NB):
-            em(f"  if constexpr (DIG == 2) wave_add_lds(&jcdL[{ia * NB + ib}], double(dg * jab_{ia}_{ib}[s]));")
-            em(f"  else if (q.deg != 0.0) atomicAdd(&jl[{ia * NB + ib}], double(dg * jab_{ia}_{ib}[s]));")
+    _emit_jab(em, NA, NB, lambda ia, ib: f"jab_{ia}_{ib}[s]", "q.deg != 0.0")
     em("}")
     em("if (q.deg != 0.0 && jk.do_k[s]) {")
     for ia in range(NA):
@@ -586,12 +614,31 @@ def orientation(X, Y):
     return (X, Y) if w1 <= w2 else (Y, X)
 
 
+# Merged launches: (workgroup size, wavefronts per SIMD, class pairs).  A tier's kernel needs the
+# registers of its largest class pair, so the tiers follow the register counts.
+TIERS = [
+    (512, 4, ["ssss", "ssps", "psps", "sspp", "ssds"]),
+    (256, 2, ["psds", "ssdp", "ppps", "pppp", "ppds", "dsds", "dpps"]),
+    (256, 2, ["dppp", "dpds", "dpdp", "ddss", "ddps"]),
+    (256, 1, ["ddpp", "ddds", "dddp", "dddd"]),
+]
+
+
+def merged_forms(name, segb):
+    """Digestion forms (1 ket-keyed, 2 bra-keyed) of a class pair's merged kernel: both where
+    either side can have fewer pairs; the bra-keyed one alone for the other class pairs that have
+    it (few pairs of the higher class, many lanes of the lower), which halves their code."""
+    return (1, 2) if name in ("psds", "ppds") else (2,) if segb else (1,)
+
+
 def main(out_dir: str, maxl: int = 2):
-    """Write one translation unit per class pair plus the registry include."""
+    """Write, per class pair, a header (quartet functions) and a translation unit (its kernels),
+    one translation unit per merged tier, and the registry includes."""
     import os
     os.makedirs(out_dir, exist_ok=True)
     pcl = class_list(maxl)
     table = []
+    segbs = {}
     for i, X in enumerate(pcl):
         for j, Y in enumerate(pcl):
             if j > i:
@@ -601,36 +648,79 @@ def main(out_dir: str, maxl: int = 2):
             LC, LD = ket
             name = f"{CLS_NAME[LA]}{CLS_NAME[LB]}{CLS_NAME[LC]}{CLS_NAME[LD]}"
             L = LA + LB + LC + LD
-            src = ["// GENERATED by gen_eri.py -- do not edit.",
-                   '#include "../gdirect_kernels.h"', ""]
-            src.append(gen_class(LA, LB, LC, LD, "jk"))
-            src.append(gen_class(LA, LB, LC, LD, "block"))
-            src.append(f"DEFINE_CLASS_KERNELS({name}, {L})")
+            hdr = ["// GENERATED by gen_eri.py -- do not edit.", "#pragma once",
+                   '#include "../gdirect_kernels.h"', "", gen_class(LA, LB, LC, LD, "jk")]
+            _write_if_changed(os.path.join(out_dir, f"cls_{name}.h"), "\n".join(hdr) + "\n")
+            # (the block kernel and the FP32 kernels in units of their own: they compile in parallel)
+            src = ["// GENERATED by gen_eri.py -- do not edit.", f'#include "cls_{name}.h"', "",
+                   gen_class(LA, LB, LC, LD, "block"), f"DEFINE_CLASS_BLOCK({name})",
+                   f"BlockKernel cq_block_{name}() {{ return eri_block_{name}; }}"]
+            _write_if_changed(os.path.join(out_dir, f"blk_{name}.hip"), "\n".join(src) + "\n")
+            src = ["// GENERATED by gen_eri.py -- do not edit.", f'#include "cls_{name}.h"', ""]
+            src.append(f"DEFINE_CLASS_KERNELS({name})")
             # bra-uniform groups pay off where the bra class has far fewer pairs than the ket
             # class (few bras survive per ket): different pair classes and a bra above (ss)
             segb = i != j and (LA, LB) != (0, 0)
+            segbs[name] = segb
             if segb:
-                src.append(f"DEFINE_CLASS_SEGB({name}, {L})")
+                src.append(f"DEFINE_CLASS_SEGB({name})")
             # ket-keyed groups of an (ss) or (ps) bra class hold many bras per ket: 512-thread
             # workgroups share one Boys table and one set of K columns over 8 wavefronts
             seg_wg = 512 if (LA, LB) in ((0, 0), (1, 0)) else 256
+            tier = [t for t, (_, _, names) in enumerate(TIERS) if name in names][0]
             gb = (lambda R: f"eri_grpb_{name}<{R}>") if segb else (lambda R: "nullptr")
+            f32 = src + [f"void cq_f32_{name}(GroupKernel* g) {{",
+                         f"  g[0] = eri_grp_{name}<{seg_wg}, 0, float>;",
+                         f"  g[1] = eri_grp_{name}<{seg_wg}, 1, float>;",
+                         f"  g[2] = {gb('float')};", "}"]
+            _write_if_changed(os.path.join(out_dir, f"f32_{name}.hip"), "\n".join(f32) + "\n")
+            src += [f"BlockKernel cq_block_{name}();", f"void cq_f32_{name}(GroupKernel* g);"]
             src.append(f"void cq_register_{name}(ClassKernels& ck) {{")
-            src.append(f"  ck = ClassKernels{{{i}, {j}, {pcl.index(bra)}, {pcl.index(ket)}, {L}, kChunks_{name}, \"{name}\", "
-                       f"eri_block_{name}, "
-                       f"{{{{eri_grp_{name}<{seg_wg}, 0, double>, eri_grp_{name}<{seg_wg}, 1, double>, {gb('double')}}}, "
-                       f"{{eri_grp_{name}<{seg_wg}, 0, float>, eri_grp_{name}<{seg_wg}, 1, float>, {gb('float')}}}}}, "
-                       f"kNC_{name}, kND_{name}, kNA_{name}, kNB_{name}, {seg_wg}}};")
+            src.append(f"  ck = ClassKernels{{{i}, {j}, {pcl.index(bra)}, {pcl.index(ket)}, {L}, Cls_{name}::NCH, \"{name}\", "
+                       f"cq_block_{name}(), "
+                       f"{{{{eri_grp_{name}<{seg_wg}, 0, double>, eri_grp_{name}<{seg_wg}, 1, double>, {gb('double')}}}, {{}}}}, "
+                       f"Cls_{name}::NC, Cls_{name}::ND, Cls_{name}::NA, Cls_{name}::NB, {seg_wg}, {tier}, {sum(merged_forms(name, segb))}}};")
+            src.append(f"  cq_f32_{name}(ck.grp[1]);")
             src.append("}")
             _write_if_changed(os.path.join(out_dir, f"eri_{name}.hip"), "\n".join(src) + "\n")
             table.append(name)
+    for t, (wgs, waves, names) in enumerate(TIERS):
+        src = ["// GENERATED by gen_eri.py -- do not edit."]
+        src += [f'#include "cls_{n}.h"' for n in names]
+        src += [f"__global__ void __launch_bounds__({wgs}, {waves}) eri_merged_{t}(MERGED_KERNEL_PARAMS) {{",
+                "  __shared__ double boys_lds[BOYS_ROWS * BOYS_LDS_W];",
+                "  __shared__ ItemLds s_it;",
+                "  extern __shared__ double dyn_lds[];",
+                "  JKArgs jk;",
+                "  const MergedEntry& e = merged_entry(ma, jk0, jk);",
+                "  unsigned* const wq = work + ((size_t)blockIdx.y * CQ_NUM_CLASS_PAIRS + e.k) * WORK_QUEUES;",
+                "  const unsigned blk = blockIdx.x - (unsigned)e.blk0;",
+                "  switch (2 * e.k + e.bra) {"]
+        for n in names:
+            for dig in merged_forms(n, segbs[n]):
+                src += [f"    case {2 * table.index(n) + (dig == 2)}:",
+                        f"      group_body<Cls_{n}, {wgs}, {dig}, double>(tasks + e.task_off, segs + e.seg_off, e.nres, ovf + e.k, wq, pairs,",
+                        "          prims, boys, jk, groups, uorder, e.mmax, e.ub, e.cpi, blk, (unsigned)e.nblk, boys_lds, s_it, dyn_lds);",
+                        "      break;"]
+        src += ["    default: break;", "  }", "}",
+                f"MergedKernel cq_merged_{t}() {{ return eri_merged_{t}; }}"]
+        _write_if_changed(os.path.join(out_dir, f"merged_{t}.hip"), "\n".join(src) + "\n")
+    cnt = ["// GENERATED by gen_eri.py -- do not edit.", f"#define CQ_NUM_CLASS_PAIRS {len(table)}",
+           f"#define CQ_NUM_TIERS {len(TIERS)}"]
+    _write_if_changed(os.path.join(out_dir, "eri_counts.inc"), "\n".join(cnt) + "\n")
     reg = ["// GENERATED by gen_eri.py -- do not edit."]
     for name in table:
         reg.append(f"void cq_register_{name}(ClassKernels& ck);")
-    reg.append(f"#define CQ_NUM_CLASS_PAIRS {len(table)}")
     reg.append("static inline void cq_register_all(ClassKernels* t) {")
     for k, name in enumerate(table):
         reg.append(f"  cq_register_{name}(t[{k}]);")
+    reg.append("}")
+    for t in range(len(TIERS)):
+        reg.append(f"MergedKernel cq_merged_{t}();")
+    reg.append("struct MergedTier { MergedKernel kernel; int wgs; };")
+    reg.append("static inline void cq_merged_all(MergedTier* t) {")
+    for t, (wgs, _, _) in enumerate(TIERS):
+        reg.append(f"  t[{t}] = MergedTier{{cq_merged_{t}(), {wgs}}};")
     reg.append("}")
     _write_if_changed(os.path.join(out_dir, "eri_registry.inc"), "\n".join(reg) + "\n")
 

@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(WG) onee_kernel(const PairInfo* __restrict__ p
                                                   double* __restrict__ S, double* __restrict__ T,
                                                   double* __restrict__ V) {
   constexpr int NA = (LA + 1) * (LA + 2) / 2, NB = (LB + 1) * (LB + 2) / 2, L = LA + LB;
-  __shared__ double boys_lds[BOYS_NGRID * BOYS_LDS_W];
+  __shared__ double boys_lds[BOYS_ROWS * BOYS_LDS_W];
   if (DO_V) stage_boys(boys, L, boys_lds);
   const int P = p_begin + blockIdx.x * blockDim.x + threadIdx.x;
   if (P >= p_end) return;
@@ -143,18 +143,15 @@ __global__ void __launch_bounds__(WG) onee_kernel(const PairInfo* __restrict__ p
 #pragma unroll
         for (int h = 0; h < NH; ++h) Rs[h] = 0.0;
         for (int c = c0; c < c1; ++c) {
-          const double X = Px - xyz[3 * c], Y = Py - xyz[3 * c + 1], Z = Pz - xyz[3 * c + 2];
-          double F[L + 1];
-          boys_eval<L>(p * (X * X + Y * Y + Z * Z), boys_lds, F);
-          double fac[L + 1];
-          fac[0] = Zc[c];
-#pragma unroll
-          for (int n = 1; n <= L; ++n) fac[n] = fac[n - 1] * (-2.0 * p);
+          // X, Y, Z = C - P: the sign of (-2p)^n goes into the recursion
+          const double X = xyz[3 * c] - Px, Y = xyz[3 * c + 1] - Py, Z = xyz[3 * c + 2] - Pz;
+          double Rb[L + 1];
+          boys_scaled<L>(1.0, 2.0 * p, X * X + Y * Y + Z * Z, Zc[c], boys_lds, Rb);
           double Rc[NH], Rn[NH];
-          Rc[0] = fac[L] * F[L];
+          Rc[0] = Rb[L];
 #pragma unroll
           for (int n = L - 1; n >= 0; --n) {
-            Rn[0] = fac[n] * F[n];
+            Rn[0] = Rb[n];
 #pragma unroll
             for (int sl = 1; sl <= L; ++sl) {
               if (sl > L - n) break;
@@ -164,9 +161,9 @@ __global__ void __launch_bounds__(WG) onee_kernel(const PairInfo* __restrict__ p
                 for (int w = 0; w <= sl - tt; ++w) {
                   const int u = sl - tt - w;
                   double r;
-                  if (tt > 0) r = X * Rc[hidx(tt - 1, u, w)] + (tt > 1 ? (tt - 1) * Rc[hidx(tt - 2, u, w)] : 0.0);
-                  else if (u > 0) r = Y * Rc[hidx(tt, u - 1, w)] + (u > 1 ? (u - 1) * Rc[hidx(tt, u - 2, w)] : 0.0);
-                  else r = Z * Rc[hidx(tt, u, w - 1)] + (w > 1 ? (w - 1) * Rc[hidx(tt, u, w - 2)] : 0.0);
+                  if (tt > 0) r = X * Rc[hidx(tt - 1, u, w)] - (tt > 1 ? (tt - 1) * Rc[hidx(tt - 2, u, w)] : 0.0);
+                  else if (u > 0) r = Y * Rc[hidx(tt, u - 1, w)] - (u > 1 ? (u - 1) * Rc[hidx(tt, u - 2, w)] : 0.0);
+                  else r = Z * Rc[hidx(tt, u, w - 1)] - (w > 1 ? (w - 1) * Rc[hidx(tt, u, w - 2)] : 0.0);
                   Rn[hidx(tt, u, w)] = r;
                 }
             }
