@@ -635,27 +635,28 @@ __global__ void zero_kernel(ZeroList zl) {
   }
 }
 
-// out[mu + nu*ld] = sum_{a,c} T(mu,a) T(nu,c) Mc[a][c]   (Cartesian row-major -> shells' basis)
-__global__ void sph_transform_kernel(const double* __restrict__ Mc, double* __restrict__ out, int n, int ld,
+// out_i[mu + nu*ld] = sum_{a,c} T(mu,a) T(nu,c) Mc_i[a][c]   (Cartesian row-major -> shells'
+// basis), the matrices i = blockIdx.y back to back in Mc.
+struct OutList {
+  double* p[19];
+};
+__global__ void sph_transform_kernel(const double* __restrict__ Mc, OutList out, int n, int ld,
                                      const ShellMeta* __restrict__ sh, const int* __restrict__ sph2shell, int ncart,
                                      const double* __restrict__ tco, const int* __restrict__ tco_off) {
   const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= (long)n * n) return;
+  Mc += (long)blockIdx.y * ncart * ncart;
   const int mu = k % n, nu = k / n;
   const ShellMeta A = sh[sph2shell[mu]], B = sh[sph2shell[nu]];
-  const int im = mu - A.sph_off, in = nu - B.sph_off;
-  const int nca = (A.l + 1) * (A.l + 2) / 2, ncb = (B.l + 1) * (B.l + 2) / 2;
+  const TList ta = sph_to_cart(A, mu - A.sph_off, tco, tco_off), tb = sph_to_cart(B, nu - B.sph_off, tco, tco_off);
   double s = 0.0;
-  for (int a = 0; a < nca; ++a) {
-    const double ta = tcoef(A, im, a, tco, tco_off);
-    if (ta == 0.0) continue;
-    for (int c = 0; c < ncb; ++c) {
-      const double tc = tcoef(B, in, c, tco, tco_off);
-      if (tc == 0.0) continue;
-      s += ta * tc * Mc[(long)(A.cart_off + a) * ncart + B.cart_off + c];
-    }
-  }
-  out[(long)nu * ld + mu] = s;
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      if (p < ta.n && q < tb.n)
+        s += ta.c[p] * tb.c[q] * Mc[(long)(A.cart_off + ta.idx[p]) * ncart + B.cart_off + tb.idx[q]];
+  out.p[blockIdx.y][(long)nu * ld + mu] = s;
 }
 
 // Schwarz: Q(P) = sqrt(max_{ij} |(ij|ij)|) in the shells' own (pure or Cartesian) basis,
@@ -1500,7 +1501,11 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     for (auto& h : hp) { all.push_back(h.info); cls_all.push_back(h.cls); }
     std::vector<int> order(all.size());
     std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cls_all[x] < cls_all[y]; });
+    // (inside a class the most contracted pairs first: the lanes of a wavefront stay in step)
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+      if (cls_all[x] != cls_all[y]) return cls_all[x] < cls_all[y];
+      return nprim[all[x].a] * nprim[all[x].b] > nprim[all[y].a] * nprim[all[y].b];
+    });
     std::vector<PairInfo>& sorted_all = c->pairs_1e_h;
     sorted_all.clear();
     sorted_all.reserve(all.size());
@@ -2211,18 +2216,13 @@ void one_electron(cq_ctx* c, int natom, const double* Z, const double* xyz, cons
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
   // nuclei per molecule
   std::vector<int> mol_atom0(c->nmol + 1, 0);
-  int max_atoms = natom;
   if (atom_mol) {
     for (int a = 0; a < natom; ++a) {
       if (atom_mol[a] < 0 || atom_mol[a] >= c->nmol || (a > 0 && atom_mol[a] < atom_mol[a - 1]))
         throw std::invalid_argument("atom_molecule must be nondecreasing molecule ids of the context");
       mol_atom0[atom_mol[a] + 1]++;
     }
-    max_atoms = 0;
-    for (int m = 0; m < c->nmol; ++m) {
-      max_atoms = std::max(max_atoms, mol_atom0[m + 1]);
-      mol_atom0[m + 1] += mol_atom0[m];
-    }
+    for (int m = 0; m < c->nmol; ++m) mol_atom0[m + 1] += mol_atom0[m];
   }
   const long nc2 = (long)c->ncart * c->ncart;
   const int na1 = std::max(1, natom);
@@ -2246,33 +2246,30 @@ void one_electron(cq_ctx* c, int natom, const double* Z, const double* xyz, cons
     sd.shell_mol = d_smol.p;
     sd.mol_atom0 = d_mat0.p;
   }
-  ZeroList zl{};
-  zl.p[0] = (unsigned*)Sc;
-  zl.n[0] = 3 * nc2 * 2;
-  zl.count = 1;
-  hipLaunchKernelGGL(zero_kernel, dim3(1024), dim3(WG), 0, s, zl);
-  int max_prim = 1;
-  for (size_t k = 0; k + 1 < c->prim_off_host.size(); ++k)
-    max_prim = std::max(max_prim, c->prim_off_host[k + 1] - c->prim_off_host[k]);
+  if (c->nmol > 1) {   // (elements between molecules; within one every element is stored)
+    ZeroList zl{};
+    zl.p[0] = (unsigned*)Sc;
+    zl.n[0] = 3 * nc2 * 2;
+    zl.count = 1;
+    hipLaunchKernelGGL(zero_kernel, dim3(1024), dim3(WG), 0, s, zl);
+  }
   // the pair classes' kernels (small grids, latency-bound) side by side on s and the context's
   // auxiliary streams; every class adds into its own blocks
   HIPCHK(hipEventRecord(c->ev_fork, s));
   for (int a = 0; a < cq_ctx::kAux; ++a) HIPCHK(hipStreamWaitEvent(c->aux[a], c->ev_fork, 0));
   for (int X = 0; X < c->npc; ++X) {
     const int si = X % (cq_ctx::kAux + 1);
-    launch_onee(X, c->d_pairs_1e.p, c->class_start_1e[X], c->class_start_1e[X + 1], sd, max_prim, dZ, dxyz, natom,
-                max_atoms, c->d_boys.p, c->ncart, Sc, Tc, Vc, si == 0 ? s : c->aux[si - 1]);
+    launch_onee(X, c->d_pairs_1e.p, c->class_start_1e[X], c->class_start_1e[X + 1], sd, dZ, dxyz, natom, c->d_boys.p,
+                c->ncart, Sc, Tc, Vc, si == 0 ? s : c->aux[si - 1]);
   }
   HIPCHK(hipGetLastError());
   for (int a = 0; a < cq_ctx::kAux; ++a) {
     HIPCHK(hipEventRecord(c->ev_join[a], c->aux[a]));
     HIPCHK(hipStreamWaitEvent(s, c->ev_join[a], 0));
   }
-  double* outs[3] = {S, T, V};
-  for (int k = 0; k < 3; ++k)
-    hipLaunchKernelGGL(sph_transform_kernel, dim3(grid_for((long)c->nsph * c->nsph, WG)), dim3(WG), 0, s,
-                       c->d_onee.p + k * nc2, outs[k], c->nsph, ld, c->d_shells.p, c->d_sph2shell.p, c->ncart,
-                       c->d_tco.p, c->d_tco_off.p);
+  const OutList outs{{S, T, V}};
+  hipLaunchKernelGGL(sph_transform_kernel, dim3(grid_for((long)c->nsph * c->nsph, WG), 3), dim3(WG), 0, s, c->d_onee.p,
+                     outs, c->nsph, ld, c->d_shells.p, c->d_sph2shell.p, c->ncart, c->d_tco.p, c->d_tco_off.p);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s));   // the host staging vectors and device tables are released on return
   d_smol.release();
@@ -2304,10 +2301,10 @@ void multipole(cq_ctx* c, int order, const double* origin, double* out, int ld, 
     launch_multipole(X, c->d_pairs_1e.p, c->class_start_1e[X], c->class_start_1e[X + 1], sd, max_prim, C, order,
                      c->ncart, Mc, s);
   HIPCHK(hipGetLastError());
-  for (int k = 0; k < nops; ++k)
-    hipLaunchKernelGGL(sph_transform_kernel, dim3(grid_for((long)c->nsph * c->nsph, WG)), dim3(WG), 0, s,
-                       Mc + k * nc2, out + (long)k * ld * c->nsph, c->nsph, ld, c->d_shells.p, c->d_sph2shell.p,
-                       c->ncart, c->d_tco.p, c->d_tco_off.p);
+  OutList outs{};
+  for (int k = 0; k < nops; ++k) outs.p[k] = out + (long)k * ld * c->nsph;
+  hipLaunchKernelGGL(sph_transform_kernel, dim3(grid_for((long)c->nsph * c->nsph, WG), nops), dim3(WG), 0, s, Mc, outs,
+                     c->nsph, ld, c->d_shells.p, c->d_sph2shell.p, c->ncart, c->d_tco.p, c->d_tco_off.p);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s));
 }

@@ -17,12 +17,10 @@ struct OneEShellData {
 };
 
 // S, T, V Cartesian blocks of the shell pairs [p_begin, p_end) of one pair class
-// (0 ss, 1 ps, 2 pp, 3 ds, 4 dp, 5 dd), added into zeroed row-major ncart x ncart matrices;
-// max_prim bounds the primitive count of any shell, max_atoms the nuclei acting on one pair
-// (natom, or the largest molecule's atom count).
+// (0 ss, 1 ps, 2 pp, 3 ds, 4 dp, 5 dd), stored into row-major ncart x ncart matrices.
 void launch_onee(int pair_class, const PairInfo* pairs, int p_begin, int p_end, const OneEShellData& sd,
-                 int max_prim, const double* Z, const double* xyz, int natom, int max_atoms, const double* boys,
-                 int ncart, double* S, double* T, double* V, hipStream_t stream);
+                 const double* Z, const double* xyz, int natom, const double* boys, int ncart, double* S, double* T,
+                 double* V, hipStream_t stream);
 
 // Multipole moment integrals about C[3] (host array, bohr) of one pair class: order 1 .. 3 gives
 // the 3, 9 or 19 Cartesian operators x, y, z; xx, xy, xz, yy, yz, zz; xxx, xxy, xxz, xyy, xyz,

@@ -6,11 +6,12 @@
 // S_1D(i,j) = E^{ij}_0 sqrt(pi/p),
 // T_1D(i,j) = -1/2 [ j(j-1) S(i,j-2) - 2b(2j+1) S(i,j) + 4b^2 S(i,j+2) ],
 // V = -(2 pi / p) sum_C Z_C sum_tuv E_t E_u E_v R_tuv(p, P - C).
-// One thread per (shell pair, slice), every loop unrolled at compile time: S and T in one pass
-// whose slices are the primitives of shell a, V in a second pass whose slices are groups of
-// ONEE_ATOMS nuclei (summing R_tuv over them first).  Partial blocks are added atomically to
-// zeroed row-major ncart x ncart matrices (and their transposes for a != b).
+// S, T and V: one lane per shell pair, the nuclei and primitives over the wavefronts of its
+// workgroup, every element of the row-major ncart x ncart matrices stored once.  Multipoles: one
+// thread per (shell pair, primitive of a), partial blocks added atomically to zeroed matrices.
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "gdirect_kernels.h"
 #include "onee.h"
@@ -68,146 +69,207 @@ __device__ __forceinline__ double hermE(int i, int j, int t, double PA, double P
   return s;
 }
 
-// nuclei per thread of the nuclear-attraction kernels (more slices: more threads in flight)
-#define ONEE_ATOMS 2
+// f(0), .., f(N - 1) with compile-time indices
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
 
-template <int LA, int LB, bool DO_V>
-__global__ void __launch_bounds__(WG) onee_kernel(const PairInfo* __restrict__ pairs, int p_begin, int p_end,
-                                                  const OneEShellData sd, const double* __restrict__ Zc,
-                                                  const double* __restrict__ xyz, int natom,
-                                                  const double* __restrict__ boys, int ncart,
-                                                  double* __restrict__ S, double* __restrict__ T,
-                                                  double* __restrict__ V) {
-  constexpr int NA = (LA + 1) * (LA + 2) / 2, NB = (LB + 1) * (LB + 2) / 2, L = LA + LB;
-  __shared__ double boys_lds[BOYS_ROWS * BOYS_LDS_W];
-  if (DO_V) stage_boys(boys, L, boys_lds);
-  const int P = p_begin + blockIdx.x * blockDim.x + threadIdx.x;
-  if (P >= p_end) return;
-  const PairInfo pi = pairs[P];
-  const int a = pi.a, b = pi.b;
-  // slice: one primitive of a (S, T) or nuclei [c0, c1) (V)
-  const int ip0 = DO_V ? sd.prim_off[a] : sd.prim_off[a] + (int)blockIdx.y;
-  const int ip1 = DO_V ? sd.prim_off[a + 1] : ip0 + 1;
-  if (ip0 >= sd.prim_off[a + 1]) return;
-  // nuclei of this slice: those of the pair's molecule when several molecules share the context
-  int at0 = 0, at1 = natom;
-  if (DO_V && sd.mol_atom0) {
-    const int m = sd.shell_mol[a];
-    at0 = sd.mol_atom0[m];
-    at1 = sd.mol_atom0[m + 1];
+// E^{ij}_t, i <= LA, j <= LB, of one direction by the recursion over i, then j (every index a
+// compile-time constant: the table lives in registers, unused entries are never computed).
+template <int LA, int LB>
+struct HermE {
+  double v[LA + 1][LB + 1][LA + LB + 1];
+  __device__ __forceinline__ HermE(double PA, double PB, double o2p) {
+    static_for<LA + 1>([&](auto I) {
+      static_for<LB + 1>([&](auto J) {
+        constexpr int i = I.value, j = J.value;
+        if constexpr (i + j == 0) {
+          v[0][0][0] = 1.0;
+        } else {
+          constexpr int si = i > 0 ? i - 1 : i, sj = i > 0 ? j : j - 1, n = i + j;
+          const double X = i > 0 ? PA : PB;
+          static_for<n + 1>([&](auto T) {
+            constexpr int t = T.value;
+            double r = 0.0;
+            if constexpr (t < n) r = X * v[si][sj][t];
+            if constexpr (t > 0) r += o2p * v[si][sj][t - 1];
+            if constexpr (t + 1 < n) r += (t + 1) * v[si][sj][t + 1];
+            v[i][j][t] = r;
+          });
+        }
+      });
+    });
   }
-  const int c0 = DO_V ? at0 + (int)blockIdx.y * ONEE_ATOMS : 0;
-  const int c1 = DO_V ? min(at1, c0 + ONEE_ATOMS) : 0;
-  if (DO_V && c0 >= at1) return;
+};
+
+// A workgroup takes 64 shell pairs (one per lane) and spreads the nuclei, and the primitives of
+// contracted classes, over its wavefronts: NW = PS x (NW / PS) of them, wavefront w taking the
+// primitive pairs = w mod PS and the nuclei = w / PS mod NW / PS (S and T: the primitive pairs
+// = w mod NW).  The wavefronts' partial blocks meet in LDS and every element is stored once.
+// What bounds it is the latency of the (nucleus, primitive pair) evaluations in series per
+// wavefront; a thread per (pair, two nuclei) that redid the pair's Hermite coefficients (from
+// their closed form, with component loops the compiler left rolled: run-time indices in scratch)
+// and added its partial block to HBM atomically took 1.29 ms for (H2O)16/cc-pVDZ.
+template <int LA, int LB>
+struct OneEShape {
+  static constexpr int L = LA + LB;
+  static constexpr int NW = L <= 1 ? 16 : 8;
+  static constexpr int PS = L <= 1 ? 4 : L == 2 ? 2 : 1;
+};
+
+template <int LA, int LB>
+__global__ void __launch_bounds__((64 * OneEShape<LA, LB>::NW)) onee_kernel(
+    const PairInfo* __restrict__ pairs, int p_begin, int p_end, const OneEShellData sd, const double* __restrict__ Zc,
+    const double* __restrict__ xyz, int natom, const double* __restrict__ boys, int ncart, double* __restrict__ S,
+    double* __restrict__ T, double* __restrict__ V) {
+  constexpr int NA = (LA + 1) * (LA + 2) / 2, NB = (LB + 1) * (LB + 2) / 2, NAB = NA * NB, L = LA + LB;
+  constexpr int NW = OneEShape<LA, LB>::NW, PS = OneEShape<LA, LB>::PS, CS = NW / PS;
+  __shared__ double boys_lds[BOYS_ROWS * BOYS_LDS_W];
+  __shared__ double red[NAB * 64];
+  const int wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  for (int k = threadIdx.x; k < NAB * 64; k += 64 * NW) red[k] = 0.0;
+  stage_boys(boys, L, boys_lds);
+  const int base = p_begin + (int)blockIdx.x * 64;
+  const bool in = base + lane < p_end;
+  const PairInfo pi = pairs[in ? base + lane : base];
+  const int a = pi.a, b = pi.b;
   const double A[3] = {sd.origin[3 * a], sd.origin[3 * a + 1], sd.origin[3 * a + 2]};
   const double B[3] = {sd.origin[3 * b], sd.origin[3 * b + 1], sd.origin[3 * b + 2]};
-  const double AB2 = (A[0] - B[0]) * (A[0] - B[0]) + (A[1] - B[1]) * (A[1] - B[1]) + (A[2] - B[2]) * (A[2] - B[2]);
-  double s[NA][NB], t[NA][NB];
+  const double AB[3] = {B[0] - A[0], B[1] - A[1], B[2] - A[2]};
+  const double AB2 = AB[0] * AB[0] + AB[1] * AB[1] + AB[2] * AB[2];
+  const int pa0 = sd.prim_off[a], pb0 = sd.prim_off[b], npb = sd.prim_off[b + 1] - pb0;
+  const int np = in ? (sd.prim_off[a + 1] - pa0) * npb : 0;
+  // adds the wavefronts' blocks up and stores them (and their transposes); red is clear again after
+  auto store = [&](const double (&x)[NAB], double* M) {
 #pragma unroll
-  for (int i = 0; i < NA; ++i)
+    for (int k = 0; k < NAB; ++k) atomicAdd(&red[k * 64 + lane], x[k]);
+    __syncthreads();
+    for (int k = threadIdx.x; k < NAB * 64; k += 64 * NW) {
+      const int q = base + (k & 63);
+      if (q < p_end) {
+        const PairInfo o = pairs[q];
+        const int ab = k >> 6;
+        const long r = o.a0 + ab / NB, c = o.b0 + ab % NB;
+        M[r * ncart + c] = red[k];
+        if (o.a != o.b) M[c * ncart + r] = red[k];
+      }
+      red[k] = 0.0;
+    }
+    __syncthreads();
+  };
+  // ---- nuclear attraction: nuclei of the pair's molecule when several share the context
+  {
+    int at0 = 0, at1 = natom;
+    if (sd.mol_atom0) {
+      const int m = sd.shell_mol[a];
+      at0 = sd.mol_atom0[m];
+      at1 = sd.mol_atom0[m + 1];
+    }
+    double v[NAB];
 #pragma unroll
-    for (int j = 0; j < NB; ++j) { s[i][j] = 0.0; t[i][j] = 0.0; }
-  for (int ip = ip0; ip < ip1; ++ip)
-    for (int jp = sd.prim_off[b]; jp < sd.prim_off[b + 1]; ++jp) {
+    for (int k = 0; k < NAB; ++k) v[k] = 0.0;
+    for (int k = wid % PS; k < np; k += PS) {
+      const int ip = pa0 + k / npb, jp = pb0 + k % npb;
       const double al = sd.alpha[ip], be = sd.alpha[jp];
-      const double p = al + be, o2p = 0.5 / p;
-      const double K = exp(-al * be / p * AB2) * sd.coef[ip] * sd.coef[jp];
-      const double PA0 = be / p * (B[0] - A[0]), PA1 = be / p * (B[1] - A[1]), PA2 = be / p * (B[2] - A[2]);
-      const double PB0 = al / p * (A[0] - B[0]), PB1 = al / p * (A[1] - B[1]), PB2 = al / p * (A[2] - B[2]);
-      if (!DO_V) {
-        const double sq = sqrt(3.14159265358979323846 / p);
+      const double p = al + be, rp = 1.0 / p;
+      const double K = exp(-al * be * rp * AB2) * sd.coef[ip] * sd.coef[jp];
+      const double fa = be * rp, fb = -al * rp;   // P - A = fa AB, P - B = fb AB
+      const double Px = A[0] + fa * AB[0], Py = A[1] + fa * AB[1], Pz = A[2] + fa * AB[2];
+      // Rsum_tuv = sum_C Z_C R_tuv(p, P - C), t + u + w <= L, in the compact index hidx
+      constexpr int NH = (L + 1) * (L + 2) * (L + 3) / 6;
+      double Rs[NH];
 #pragma unroll
-        for (int ia = 0; ia < NA; ++ia)
-#pragma unroll
-          for (int ib = 0; ib < NB; ++ib) {
-            const int ax = comp_x(LA, ia), ay = comp_y(LA, ia), az = comp_z(LA, ia);
-            const int bx = comp_x(LB, ib), by = comp_y(LB, ib), bz = comp_z(LB, ib);
-            const double sx = hermE(ax, bx, 0, PA0, PB0, o2p) * sq;
-            const double sy = hermE(ay, by, 0, PA1, PB1, o2p) * sq;
-            const double sz = hermE(az, bz, 0, PA2, PB2, o2p) * sq;
-            auto kin = [&](int i, int j, double PAd, double PBd, double sij) {
-              double d2 = 4.0 * be * be * hermE(i, j + 2, 0, PAd, PBd, o2p) * sq - 2.0 * be * (2 * j + 1) * sij;
-              if (j >= 2) d2 += (double)(j * (j - 1)) * hermE(i, j - 2, 0, PAd, PBd, o2p) * sq;
-              return -0.5 * d2;
-            };
-            s[ia][ib] += K * sx * sy * sz;
-            t[ia][ib] += K * (kin(ax, bx, PA0, PB0, sx) * sy * sz + sx * kin(ay, by, PA1, PB1, sy) * sz +
-                              sx * sy * kin(az, bz, PA2, PB2, sz));
-          }
-      } else {
-        const double Px = A[0] + PA0, Py = A[1] + PA1, Pz = A[2] + PA2;
-        // Rsum_tuv = sum_C Z_C R_tuv(p, P - C), t + u + w <= L, in the compact index hidx;
-        // the recursion over n keeps two levels
-        constexpr int NH = (L + 1) * (L + 2) * (L + 3) / 6;
-        double Rs[NH];
-#pragma unroll
-        for (int h = 0; h < NH; ++h) Rs[h] = 0.0;
-        for (int c = c0; c < c1; ++c) {
-          // X, Y, Z = C - P: the sign of (-2p)^n goes into the recursion
-          const double X = xyz[3 * c] - Px, Y = xyz[3 * c + 1] - Py, Z = xyz[3 * c + 2] - Pz;
-          double Rb[L + 1];
-          boys_scaled<L>(1.0, 2.0 * p, X * X + Y * Y + Z * Z, Zc[c], boys_lds, Rb);
-          double Rc[NH], Rn[NH];
-          Rc[0] = Rb[L];
-#pragma unroll
-          for (int n = L - 1; n >= 0; --n) {
-            Rn[0] = Rb[n];
-#pragma unroll
-            for (int sl = 1; sl <= L; ++sl) {
-              if (sl > L - n) break;
-#pragma unroll
-              for (int tt = sl; tt >= 0; --tt)
-#pragma unroll
-                for (int w = 0; w <= sl - tt; ++w) {
-                  const int u = sl - tt - w;
-                  double r;
-                  if (tt > 0) r = X * Rc[hidx(tt - 1, u, w)] - (tt > 1 ? (tt - 1) * Rc[hidx(tt - 2, u, w)] : 0.0);
-                  else if (u > 0) r = Y * Rc[hidx(tt, u - 1, w)] - (u > 1 ? (u - 1) * Rc[hidx(tt, u - 2, w)] : 0.0);
-                  else r = Z * Rc[hidx(tt, u, w - 1)] - (w > 1 ? (w - 1) * Rc[hidx(tt, u, w - 2)] : 0.0);
-                  Rn[hidx(tt, u, w)] = r;
-                }
+      for (int h = 0; h < NH; ++h) Rs[h] = 0.0;
+      for (int c = at0 + wid / PS; c < at1; c += CS) {
+        // C - P: the sign of (-2p)^n goes into the recursion
+        const double D[3] = {xyz[3 * c] - Px, xyz[3 * c + 1] - Py, xyz[3 * c + 2] - Pz};
+        double Rb[L + 1];
+        boys_scaled<L>(1.0, 2.0 * p, D[0] * D[0] + D[1] * D[1] + D[2] * D[2], Zc[c], boys_lds, Rb);
+        // level n of the recursion holds R^n_tuv, t + u + w <= L - n; level 0 is the result
+        double R[L + 1][NH];
+        static_for<L + 1>([&](auto N) {
+          constexpr int n = L - N.value;
+          R[n][0] = Rb[n];
+          static_for<NH>([&](auto H) {
+            constexpr int h = H.value;
+            constexpr int s = h < 1 ? 0 : h < 4 ? 1 : h < 10 ? 2 : h < 20 ? 3 : 4;
+            if constexpr (h > 0 && s <= L - n) {
+              constexpr int o = h - s * (s + 1) * (s + 2) / 6;   // within its sum: by s - t, then w
+              constexpr int st = o < 1 ? 0 : o < 3 ? 1 : o < 6 ? 2 : o < 10 ? 3 : 4;
+              constexpr int t = s - st, w = o - st * (st + 1) / 2, u = st - w;
+              constexpr int d = t > 0 ? 0 : u > 0 ? 1 : 2;
+              constexpr int m = t > 0 ? t : u > 0 ? u : w;   // the index that is lowered
+              constexpr int h1 = hidx(t - (d == 0), u - (d == 1), w - (d == 2));
+              double r = D[d] * R[n + 1][h1];
+              if constexpr (m > 1)
+                r -= (m - 1) * R[n + 1][hidx(t - 2 * (d == 0), u - 2 * (d == 1), w - 2 * (d == 2))];
+              R[n][h] = r;
             }
+          });
+        });
 #pragma unroll
-            for (int h = 0; h < NH; ++h) Rc[h] = Rn[h];
-          }
-#pragma unroll
-          for (int h = 0; h < NH; ++h) Rs[h] += Rc[h];
-        }
-        const double pref = -2.0 * 3.14159265358979323846 / p * K;
-#pragma unroll
-        for (int ia = 0; ia < NA; ++ia)
-#pragma unroll
-          for (int ib = 0; ib < NB; ++ib) {
-            const int ax = comp_x(LA, ia), ay = comp_y(LA, ia), az = comp_z(LA, ia);
-            const int bx = comp_x(LB, ib), by = comp_y(LB, ib), bz = comp_z(LB, ib);
-            double acc = 0.0;
-#pragma unroll
-            for (int tt = 0; tt <= ax + bx; ++tt) {
-              const double ex = hermE(ax, bx, tt, PA0, PB0, o2p);
-#pragma unroll
-              for (int u = 0; u <= ay + by; ++u) {
-                const double ey = hermE(ay, by, u, PA1, PB1, o2p);
-#pragma unroll
-                for (int w = 0; w <= az + bz; ++w) acc += ex * ey * hermE(az, bz, w, PA2, PB2, o2p) * Rs[hidx(tt, u, w)];
-              }
-            }
-            s[ia][ib] += pref * acc;   // V accumulates in s in this pass
-          }
+        for (int h = 0; h < NH; ++h) Rs[h] += R[0][h];
       }
+      const double o2p = 0.5 * rp, pref = -2.0 * 3.14159265358979323846 * rp * K;
+      const HermE<LA, LB> ex(fa * AB[0], fb * AB[0], o2p), ey(fa * AB[1], fb * AB[1], o2p), ez(fa * AB[2], fb * AB[2], o2p);
+      static_for<NAB>([&](auto I) {
+        constexpr int ia = I.value / NB, ib = I.value % NB;
+        constexpr int ax = comp_x(LA, ia), ay = comp_y(LA, ia), az = comp_z(LA, ia);
+        constexpr int bx = comp_x(LB, ib), by = comp_y(LB, ib), bz = comp_z(LB, ib);
+        double acc = 0.0;
+        static_for<ax + bx + 1>([&](auto TT) {
+          double au = 0.0;
+          static_for<ay + by + 1>([&](auto U) {
+            double aw = 0.0;
+            static_for<az + bz + 1>([&](auto W) {
+              aw += ez.v[az][bz][W.value] * Rs[hidx(TT.value, U.value, W.value)];
+            });
+            au += ey.v[ay][by][U.value] * aw;
+          });
+          acc += ex.v[ax][bx][TT.value] * au;
+        });
+        v[I.value] += pref * acc;
+      });
     }
-  double* M0 = DO_V ? V : S;
+    store(v, V);
+  }
+  // ---- overlap and kinetic energy
+  double s[NAB], t[NAB];
 #pragma unroll
-  for (int ia = 0; ia < NA; ++ia)
-#pragma unroll
-    for (int ib = 0; ib < NB; ++ib) {
-      const long r = pi.a0 + ia, cidx = pi.b0 + ib;
-      atomicAdd(&M0[r * ncart + cidx], s[ia][ib]);
-      if (a != b) atomicAdd(&M0[cidx * ncart + r], s[ia][ib]);
-      if (!DO_V) {
-        atomicAdd(&T[r * ncart + cidx], t[ia][ib]);
-        if (a != b) atomicAdd(&T[cidx * ncart + r], t[ia][ib]);
-      }
-    }
+  for (int k = 0; k < NAB; ++k) { s[k] = 0.0; t[k] = 0.0; }
+  for (int k = wid; k < np; k += NW) {
+    const int ip = pa0 + k / npb, jp = pb0 + k % npb;
+    const double al = sd.alpha[ip], be = sd.alpha[jp];
+    const double p = al + be, rp = 1.0 / p, o2p = 0.5 * rp;
+    const double sq = sqrt(3.14159265358979323846 * rp);
+    const double K = exp(-al * be * rp * AB2) * sd.coef[ip] * sd.coef[jp] * (sq * sq * sq);
+    const double fa = be * rp, fb = -al * rp;
+    const HermE<LA, LB + 2> ex(fa * AB[0], fb * AB[0], o2p), ey(fa * AB[1], fb * AB[1], o2p), ez(fa * AB[2], fb * AB[2], o2p);
+    auto kin = [&](const HermE<LA, LB + 2>& e, auto I, auto J) {
+      constexpr int i = decltype(I)::value, j = decltype(J)::value;
+      double d2 = 4.0 * be * be * e.v[i][j + 2][0] - 2.0 * be * (2 * j + 1) * e.v[i][j][0];
+      if constexpr (j >= 2) d2 += (double)(j * (j - 1)) * e.v[i][j - 2][0];
+      return -0.5 * d2;
+    };
+    static_for<NAB>([&](auto I) {
+      constexpr int ia = I.value / NB, ib = I.value % NB;
+      constexpr int ax = comp_x(LA, ia), ay = comp_y(LA, ia), az = comp_z(LA, ia);
+      constexpr int bx = comp_x(LB, ib), by = comp_y(LB, ib), bz = comp_z(LB, ib);
+      const double sx = ex.v[ax][bx][0], sy = ey.v[ay][by][0], sz = ez.v[az][bz][0];
+      using std::integral_constant;
+      s[I.value] += K * (sx * sy * sz);
+      t[I.value] += K * (kin(ex, integral_constant<int, ax>{}, integral_constant<int, bx>{}) * sy * sz +
+                         sx * kin(ey, integral_constant<int, ay>{}, integral_constant<int, by>{}) * sz +
+                         sx * sy * kin(ez, integral_constant<int, az>{}, integral_constant<int, bz>{}));
+    });
+  }
+  store(s, S);
+  store(t, T);
 }
 
 // Cartesian multipole x_C^EX y_C^EY z_C^EZ about C: per direction
@@ -304,21 +366,13 @@ void launch_multipole(int pair_class, const PairInfo* pairs, int p_begin, int p_
 }
 
 void launch_onee(int pair_class, const PairInfo* pairs, int p_begin, int p_end, const OneEShellData& sd,
-                 int max_prim, const double* Z, const double* xyz, int natom, int max_atoms, const double* boys,
-                 int ncart, double* S, double* T, double* V, hipStream_t stream) {
+                 const double* Z, const double* xyz, int natom, const double* boys, int ncart, double* S, double* T,
+                 double* V, hipStream_t stream) {
   const int n = p_end - p_begin;
   if (n <= 0) return;
-  const dim3 grid_st((n + WG - 1) / WG, std::max(1, max_prim));
-  const dim3 grid_v((n + WG - 1) / WG, std::max(1, (max_atoms + ONEE_ATOMS - 1) / ONEE_ATOMS));
-  const dim3 block(WG);
-#define CQ_ONEE(LA, LB)                                                                                 \
-  do {                                                                                                   \
-    hipLaunchKernelGGL((onee_kernel<LA, LB, false>), grid_st, block, 0, stream, pairs, p_begin, p_end, sd, Z, \
-                       xyz, natom, boys, ncart, S, T, V);                                                \
-    if (natom > 0)                                                                                       \
-      hipLaunchKernelGGL((onee_kernel<LA, LB, true>), grid_v, block, 0, stream, pairs, p_begin, p_end, sd, Z,  \
-                         xyz, natom, boys, ncart, S, T, V);                                              \
-  } while (0)
+#define CQ_ONEE(LA, LB)                                                                                  \
+  hipLaunchKernelGGL((onee_kernel<LA, LB>), dim3((n + 63) / 64), dim3(64 * OneEShape<LA, LB>::NW), 0, stream, pairs, \
+                     p_begin, p_end, sd, Z, xyz, natom, boys, ncart, S, T, V)
   switch (pair_class) {
     case 0: CQ_ONEE(0, 0); break;
     case 1: CQ_ONEE(1, 0); break;
