@@ -50,7 +50,7 @@ static MergedTier kMergedTiers[CQ_NUM_TIERS];
 #define MAX_MATS 8   // matrices of one contraction
 // dynamic LDS of the group kernels: what the 64 KiB per workgroup leaves beside the static
 // LDS (Boys table, 26064 B, the work item's members)
-static const size_t kStaticLds = BOYS_ROWS * BOYS_LDS_W * sizeof(double) + 384;
+static const size_t kStaticLds = BOYS_ROWS * BOYS_LDS_W * sizeof(double) + 512;
 static const size_t kMaxDynLds = 64 * 1024 - kStaticLds;
 
 // Dynamic LDS the group kernels may use on this device: the device's per-workgroup limit
@@ -901,7 +901,7 @@ struct cq_ctx {
   double mixed_threshold = 1e-5;
   double prim_threshold = 1e-17;
   // class-pair tables: [0] every class pair ket-keyed, [1] with bra-keyed (flipped) class pairs
-  // [2] the merged launches' own plan (merge_tab)
+  // [2] the merged launches' own plan, in their orientation (ClassKernels::mrg)
   std::vector<CPMeta> cps[3];
   long long task_capacity = 0;
   // task lists per class pair are at most task_budget entries (8 B each); a class pair whose
@@ -927,10 +927,8 @@ struct cq_ctx {
   std::vector<std::vector<int>> batch_start[3];
   std::vector<std::vector<int>> batch_slots[3];   // reserved segment slots of each batch (one set per group)
   std::vector<unsigned char> nblk_h, nublk_h;
-  // merged launches: primitive blocks of mpblk (lane side) and mublk (uniform side), and the plan
-  // they run: table 1, or a table 2 of their own where their blocks differ or table 1 keys a class
-  // pair on a side that has no merged kernel
-  int mpblk = PRIM_BLOCK, mublk = UNI_BLOCK, merge_tab = 1;
+  // merged launches (table 2): primitive blocks of mpblk (lane side) and mublk (uniform side)
+  int mpblk = PRIM_BLOCK, mublk = UNI_BLOCK;
   bool own_blocks() const { return mpblk != PRIM_BLOCK || mublk != UNI_BLOCK; }
   std::vector<unsigned char> nblk_m, nublk_m;   // with blocks of their own: blocks per pair
   std::vector<int> uorder_m;                    // and uniform order
@@ -1043,14 +1041,14 @@ int persistent_grid() {
 
 // Rows of a class pair's LDS K accumulators: the functions of the swept side's shells (the bra
 // pair class for the ket-keyed kernels, the ket pair class for the bra-keyed ones).
-int lds_rows(const cq_ctx* c, const ClassKernels& ck, int variant) {
+int lds_rows(const cq_ctx* c, const ClassShape& ck, int variant) {
   return c->lds_n_set[variant == 2 ? ck.ki : ck.bi];
 }
 
 // Dynamic LDS bytes of a group kernel: ket-keyed with LDS K columns (variant 1), with HBM K
 // atomics (variant 0), or bra-keyed (variant 2), for groups of up to mmax members and unions of
 // up to ub swept pairs.
-size_t group_lds(const cq_ctx* c, const ClassKernels& ck, int variant, int mmax, int ub) {
+size_t group_lds(const cq_ctx* c, const ClassShape& ck, int variant, int mmax, int ub) {
   const size_t ncd = (size_t)ck.nc * ck.nd, nab = (size_t)ck.na * ck.nb;
   const size_t lds_n = (size_t)lds_rows(c, ck, variant);
   // (the last term: one int per union slot, its swept pair)
@@ -1064,67 +1062,63 @@ size_t group_lds(const cq_ctx* c, const ClassKernels& ck, int variant, int mmax,
 // 64 .. 1024 pairs) and the largest group (at most the cap, default 1) that keeps the kernel's
 // dynamic LDS within the budget (default 48 KiB).  mmax = 0: the variant does not fit the
 // device even with single-pair groups.
-// Default union bound per class pair (kernel orientation), from a sweep of 256..1024 with
-// single-pair groups on (H2O)16/cc-pVDZ, tau = 1e-12 (per-class kernel + screening time): the
-// bound trades fewer K-column flushes (large) against more work items to balance (small).
-// Built-in tile of each class pair: the largest group (uniform pairs sharing a shell) and the
-// union bound (swept pairs per task region), the group size then lowered until the LDS budget
-// holds it.  One molecule (measured on (H2O)16/cc-pVDZ with per-member wavefront units and
-// LDS rows for the swept shells only): groups of 4-16 members pay where a swept pair's J slot
-// would otherwise be flushed to HBM once per uniform pair ((ps|ps) kernel 0.82 -> 0.37 ms from
-// 1 to 14 members, (ss|ps) 0.95 -> 0.61 ms at 4; G[D] 4.23 -> 4.14 ms for the whole table,
-// although the screening launch's one wavefront per group then runs longer: 0.48 -> 0.62 ms
-// serialised, hidden behind the other streams' kernels); larger groups cost where a class
-// pair has few work items ((dp|pp) 0.21 ms with one member, 0.29 with 8); elsewhere
-// single-pair groups are as fast.  Several molecules in one context (measured on 256 alkanes and water clusters,
-// 6-31G*, groups of 4096 functions): a uniform pair has few partners inside its small
-// molecule, so large groups fill the wavefronts (serialised kernel time 306 -> 273 ms).
-// cpi: chunks of the split (high angular momentum) class pairs per work item, 0 = all of them.
-// A work item's chunks share its wavefronts and its one LDS flush; more chunks per item means
-// fewer items, which starves the device when a class pair has few task regions.  (H2O)16:
-// (dp|dp) 0.29 -> 0.17 ms at 3, (dd|dd) 0.14 -> 0.08 ms; the batch: G[D] 152 -> 118 ms with all.
+// Built-in tile of each class pair, by name in its kernel's orientation: the largest group (uniform
+// pairs sharing a shell), the union bound (swept pairs per task region), the group size then lowered
+// until the LDS budget holds it, and the chunks of a split class pair per work item (0: all).  Few,
+// long work items cost balance; many short ones cost their start and flush, and a swept pair's J is
+// flushed once per group.  The rows come from a coordinate search over (1..16 members) x (128..1024)
+// on whole contractions of four molecules at once (water clusters and alkanes, 6-31G* and cc-pVDZ;
+// several molecules in one context: two mixed sets of 16 and 24), each row kept where it gained on
+// their mean: (H2O)16/cc-pVDZ 3320 -> 2890 us, C12H26/6-31G* 2000 -> 1795, (H2O)64/cc-pVDZ 90.3 ->
+// 75.4 ms, a set of 24 8130 -> 7750 us.  The gain over the rows before it is that of larger groups
+// and unions now that a wavefront takes its next unit when it is free: a workgroup's wavefronts
+// no longer wait for the one with the longest lists.  Chunks per item: (H2O)16 (dp|dp) 0.29 -> 0.17
+// ms at 3 ((dd|dd) 0.14 -> 0.08); several molecules G[D] 152 -> 118 ms with all.
 struct TileDefault { const char* name; int max_group, ub, cpi; };
 static const TileDefault kTileDefaults[] = {
-    {"ssss", 4, 256, 1}, {"ssps", 4, 256, 1}, {"psps", 16, 256, 1}, {"sspp", 4, 512, 1}, {"ppps", 12, 512, 1},
-    {"pppp", 3, 256, 1}, {"ssds", 4, 256, 1}, {"psds", 8, 256, 1}, {"ppds", 1, 256, 1}, {"dsds", 1, 256, 1},
-    {"ssdp", 1, 512, 1}, {"dpps", 1, 256, 1}, {"dppp", 1, 256, 3}, {"dpds", 1, 256, 1}, {"dpdp", 1, 512, 3},
+    {"ssss", 4, 512, 1}, {"ssps", 4, 512, 1}, {"psps", 4, 1024, 1}, {"sspp", 8, 512, 1}, {"ppps", 4, 512, 1},
+    {"pppp", 3, 256, 1}, {"ssds", 16, 512, 1}, {"psds", 8, 512, 1}, {"ppds", 4, 512, 1}, {"dsds", 8, 256, 1},
+    {"ssdp", 1, 512, 1}, {"dpps", 4, 512, 1}, {"dppp", 8, 512, 3}, {"dpds", 16, 256, 1}, {"dpdp", 8, 128, 3},
     {"ddss", 1, 256, 1}, {"ddps", 1, 512, 1}, {"ddpp", 1, 512, 1}, {"ddds", 1, 512, 1}, {"dddp", 1, 512, 2},
-    {"dddd", 1, 256, 3}};
+    {"dddd", 1, 256, 3},
+    {"ppss", 8, 512, 1}, {"dsss", 16, 512, 1}, {"dpss", 4, 128, 1}};
 static const TileDefault kTileDefaultsMulti[] = {
-    {"ssss", 4, 512, 0}, {"ssps", 16, 512, 0}, {"psps", 16, 1024, 0}, {"sspp", 4, 512, 0}, {"ppps", 16, 1024, 0},
-    {"pppp", 16, 512, 0}, {"ssds", 16, 256, 0}, {"psds", 16, 512, 0}, {"ppds", 8, 256, 0}, {"dsds", 16, 512, 0},
-    {"ssdp", 16, 1024, 0}, {"dpps", 2, 1024, 0}, {"dppp", 16, 256, 0}, {"dpds", 16, 256, 0}, {"dpdp", 16, 256, 0},
-    {"ddss", 2, 1024, 0}, {"ddps", 2, 1024, 0}, {"ddpp", 16, 512, 0}, {"ddds", 16, 256, 0}, {"dddp", 4, 1024, 0},
-    {"dddd", 4, 512, 0}};
+    {"ssss", 4, 512, 0}, {"ssps", 4, 1024, 0}, {"psps", 16, 1024, 0}, {"sspp", 4, 512, 0}, {"ppps", 2, 512, 0},
+    {"pppp", 16, 512, 0}, {"ssds", 16, 512, 0}, {"psds", 16, 512, 0}, {"ppds", 16, 256, 0}, {"dsds", 16, 512, 0},
+    {"ssdp", 8, 256, 0}, {"dpps", 2, 1024, 0}, {"dppp", 8, 512, 0}, {"dpds", 16, 256, 0}, {"dpdp", 16, 256, 0},
+    {"ddss", 2, 1024, 0}, {"ddps", 2, 1024, 0}, {"ddpp", 1, 128, 0}, {"ddds", 16, 1024, 0}, {"dddp", 4, 1024, 0},
+    {"dddd", 4, 512, 0},
+    {"ppss", 16, 512, 0}, {"dsss", 16, 512, 0}, {"dpss", 8, 256, 0}};
 
-static_assert(sizeof(kTileDefaults) / sizeof(TileDefault) == CQ_NUM_CLASS_PAIRS, "one tile per class pair");
-static_assert(sizeof(kTileDefaultsMulti) / sizeof(TileDefault) == CQ_NUM_CLASS_PAIRS, "one tile per class pair");
+// (one row per class pair, and one per merged orientation that differs)
+static_assert(sizeof(kTileDefaults) == sizeof(kTileDefaultsMulti), "the same class pairs in both tables");
 
-const TileDefault* tile_default(const cq_ctx* c, const ClassKernels& ck) {
-  const TileDefault* tab = c->nmol > 1 ? kTileDefaultsMulti : kTileDefaults;
-  for (int i = 0; i < CQ_NUM_CLASS_PAIRS; ++i)
-    if (std::strcmp(tab[i].name, ck.name) == 0) return &tab[i];
-  return nullptr;
+const TileDefault* tile_default(const cq_ctx* c, const ClassShape& ck) {
+  auto find = [&](const TileDefault* tab, size_t n) -> const TileDefault* {
+    for (size_t i = 0; i < n; ++i)
+      if (std::strcmp(tab[i].name, ck.name) == 0) return &tab[i];
+    return nullptr;
+  };
+  return c->nmol > 1 ? find(kTileDefaultsMulti, sizeof(kTileDefaultsMulti) / sizeof(TileDefault))
+                     : find(kTileDefaults, sizeof(kTileDefaults) / sizeof(TileDefault));
 }
 
-int default_union_bound(const cq_ctx* c, const ClassKernels& ck, size_t jside) {
+int default_union_bound(const cq_ctx* c, const ClassShape& ck, size_t jside) {
   if (const TileDefault* t = tile_default(c, ck)) return t->ub;
   return (int)std::min<size_t>(UNION_MAX, std::max<size_t>(64, (16 * 1024) / (jside * sizeof(double)) / 64 * 64));
 }
 
-// Chunks per work item of class pair k: the caller's choice, else the built-in table's; always
-// a divisor of the chunk count.
-int class_chunks_per_item(const cq_ctx* c, int k) {
-  const int nch = kClassKernels[k].nchunk;
-  if (c->class_cpi[k] > 0) return c->class_cpi[k];
-  const TileDefault* t = tile_default(c, kClassKernels[k]);
-  int d = (!t || t->cpi == 0) ? nch : std::min(t->cpi, nch);
+// Chunks per work item of class pair k in an orientation: the caller's choice, else the built-in
+// table's; always a divisor of the chunk count.
+int class_chunks_per_item(const cq_ctx* c, int k, const ClassShape& ck) {
+  const int nch = ck.nchunk;
+  const TileDefault* t = tile_default(c, ck);
+  int d = c->class_cpi[k] > 0 ? std::min(c->class_cpi[k], nch) : (!t || t->cpi == 0) ? nch : std::min(t->cpi, nch);
   while (d > 1 && nch % d != 0) --d;
   return std::max(1, d);
 }
 
-void class_tile(const cq_ctx* c, int k, int variant, int& mmax, int& ub) {
-  const ClassKernels& ck = kClassKernels[k];
+void class_tile(const cq_ctx* c, int k, const ClassShape& ck, int variant, int& mmax, int& ub) {
   const size_t jside = variant == 2 ? (size_t)ck.nc * ck.nd : (size_t)ck.na * ck.nb;
   ub = default_union_bound(c, ck, jside);
   if (c->tile_ub[k] > 0) ub = std::max(64, std::min(c->tile_ub[k], UNION_MAX));
@@ -1153,18 +1147,16 @@ void plan_tasks(cq_ctx* c) {
   const int nm = c->nmol;
   const std::vector<int>& pair_mol = c->pair_mol_h;
   const bool own = c->own_blocks();
-  // bra-keyed in table 1: few bra pairs, and the bra-keyed LDS rows fit
-  auto bra_keyed = [&](int k) {
+  // bra-keyed: in table 1 where the bra class has few pairs and the bra-keyed LDS rows fit, in
+  // table 2 by the one form the class pair's merged kernel has
+  auto bra_keyed = [&](int k, int t) {
     const ClassKernels& ck = kClassKernels[k];
+    if (t != 1 || !ck.grp[0][2]) return t == 2 && ck.merged == 2;
     const long long nb = c->class_start[ck.bi + 1] - c->class_start[ck.bi], nk = c->class_start[ck.ki + 1] - c->class_start[ck.ki];
     int mm2 = 0, ub2 = 64;
-    if (ck.grp[0][2]) class_tile(c, k, 2, mm2, ub2);
+    class_tile(c, k, ck, 2, mm2, ub2);
     return ck.i != ck.j && mm2 > 0 && 2 * nb <= nk;
   };
-  c->merge_tab = own ? 2 : 1;
-  for (int k = 0; k < kNumClassPairs; ++k)
-    if (!(kClassKernels[k].merged >> (bra_keyed(k) ? 1 : 0) & 1)) c->merge_tab = 2;
-  const int ntab = c->merge_tab + 1;
   for (int t = 0; t < 3; ++t) {
     c->cps[t].clear();
     c->groups_h[t].clear();
@@ -1172,23 +1164,24 @@ void plan_tasks(cq_ctx* c) {
     c->batch_slots[t].assign(kNumClassPairs, std::vector<int>());
   }
   const long long budget = c->task_budget;
-  long long off = 0, off_m = 0, seg_total[3] = {0, 0, 0};
+  // every class pair has its own part of the task and segment lists, as large as the largest of
+  // its tables needs (a call runs a class pair from one table, and different class pairs from
+  // different ones)
+  long long off = 0, seg_off = 0;
   for (int k = 0; k < kNumClassPairs; ++k) {
     const ClassKernels& ck = kClassKernels[k];
-    CPMeta m{};
-    m.bra_start = c->class_start[ck.bi];
-    m.nbra = c->class_start[ck.bi + 1] - c->class_start[ck.bi];
-    m.ket_start = c->class_start[ck.ki];
-    m.nket = c->class_start[ck.ki + 1] - c->class_start[ck.ki];
-    m.same = ck.i == ck.j;
-    m.bra_class = ck.bi;
-    m.ket_class = ck.ki;
-    int mm2 = 0, ub2 = 64;
-    if (ck.grp[0][2]) class_tile(c, k, 2, mm2, ub2);
-    const int flip = bra_keyed(k);
-    CPMeta mt[3] = {m, m, m};
-    long long region = 0;
-    for (int t = 0; t < ntab; ++t) {
+    CPMeta mt[3];
+    long long region = 0, seg_region = 0;
+    for (int t = 0; t < 3; ++t) {
+      const ClassShape& sh = t == 2 ? ck.mrg : ck;
+      CPMeta m{};
+      m.bra_start = c->class_start[sh.bi];
+      m.nbra = c->class_start[sh.bi + 1] - c->class_start[sh.bi];
+      m.ket_start = c->class_start[sh.ki];
+      m.nket = c->class_start[sh.ki + 1] - c->class_start[sh.ki];
+      m.same = ck.i == ck.j;
+      m.bra_class = sh.bi;
+      m.ket_class = sh.ki;
       const std::vector<unsigned char>& nblk = t < 2 || !own ? c->nblk_h : c->nblk_m;
       const std::vector<unsigned char>& nublk = t < 2 || !own ? c->nublk_h : c->nublk_m;
       const std::vector<int>& uorder = t < 2 || !own ? c->uorder_h : c->uorder_m;
@@ -1197,18 +1190,15 @@ void plan_tasks(cq_ctx* c) {
       for (int i = 0; i < m.nbra; ++i) { bp_m[pair_mol[m.bra_start + i]] += 1; bb_m[pair_mol[m.bra_start + i]] += nblk[m.bra_start + i]; }
       for (int i = 0; i < m.nket; ++i) { kp_m[pair_mol[m.ket_start + i]] += 1; kb_m[pair_mol[m.ket_start + i]] += nblk[m.ket_start + i]; }
       CPMeta& mc = mt[t];
-      mc.flip = t == 0 ? 0 : t == 1 || ck.merged == 3 ? flip : ck.merged == 2;
+      mc = m;
+      mc.flip = bra_keyed(k, t);
       int mmax = 0, ub = 64;
-      if (mc.flip) {
-        mmax = mm2;
-        ub = ub2;
-      } else {
-        class_tile(c, k, 1, mmax, ub);
-        if (mmax == 0) class_tile(c, k, 0, mmax, ub);   // K columns do not fit: HBM K atomics
-        if (mmax == 0) throw std::invalid_argument(std::string("class pair ") + ck.name + ": no tile fits the device's LDS");
-      }
-      mc.mmax = mmax;
+      class_tile(c, k, sh, mc.flip ? 2 : 1, mmax, ub);
+      if (!mc.flip && mmax == 0 && t < 2) class_tile(c, k, sh, 0, mmax, ub);   // K columns do not fit: HBM K atomics
+      if (mmax == 0 && t < 2) throw std::invalid_argument(std::string("class pair ") + ck.name + ": no tile fits the device's LDS");
+      mc.mmax = mmax;   // (0 in table 2: the class pair keeps its own launch)
       mc.ub = ub;
+      mmax = std::max(mmax, 1);
       const int ucls = mc.flip ? m.bra_class : m.ket_class;
       const int uni_start = mc.flip ? m.bra_start : m.ket_start;
       // groups: runs of the class's uniform order with one molecule, one primitive-block count
@@ -1283,28 +1273,24 @@ void plan_tasks(cq_ctx* c) {
       close(mc.ngrp);
       mc.task_cap = cap;
       mc.seg_cap = seg_cap;
-      mc.seg_off = seg_total[t];
-      seg_total[t] += seg_cap;
-      if (t < 2) region = std::max(region, cap);
+      region = std::max(region, cap);
+      seg_region = std::max(seg_region, seg_cap);
     }
-    for (int t = 0; t < ntab; ++t) {
-      mt[t].task_off = t < 2 ? off : off_m;
+    for (int t = 0; t < 3; ++t) {
+      mt[t].task_off = off;
+      mt[t].seg_off = seg_off;
       c->cps[t].push_back(mt[t]);
     }
     off += region;
-    if (ntab > 2) off_m += mt[2].task_cap;
+    seg_off += seg_region;
   }
   c->task_capacity = off;
-  // one call may take table 0 for some class pairs and table 1 for others (per-class digestion
-  // variants): table 1's segments live after table 0's
-  for (auto& mt : c->cps[1]) mt.seg_off += seg_total[0];
-  for (int t = 0; t < ntab; ++t) {
+  for (int t = 0; t < 3; ++t) {
     c->d_cps[t].upload(c->cps[t], c->stream);
     c->d_groups[t].upload(c->groups_h[t], c->stream);
   }
-  // (a call uses tables 0 and 1 or table 2: they share the buffers)
-  c->d_tasks.ensure((size_t)std::max<long long>({1, off, off_m}));
-  c->d_segs.ensure((size_t)std::max<long long>({1, seg_total[0] + seg_total[1], seg_total[2]}));
+  c->d_tasks.ensure((size_t)std::max<long long>(1, off));
+  c->d_segs.ensure((size_t)std::max<long long>(1, seg_off));
   HIPCHK(hipStreamSynchronize(c->stream));
   c->plan_ok = true;
 }
@@ -1968,16 +1954,14 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   // class pairs one by one (their variant or stream, profiling, the screening mode, one stream)
   // and class pairs in several batches keep a launch per class pair.  (H2O)16/cc-pVDZ 3638 us with
   // a launch per class pair, 3544 merged; smaller systems gain more (choose_merge_blocks).
-  static_assert(CQ_NUM_TIERS == cq_ctx::kAux + 1, "one stream per merged tier");
-  const int mt = c->merge_tab;
   const bool can_merge = nround == 1 && !profiling && c->n_streams == cq_ctx::kAux + 1 &&
                          c->screen_mode == CQ_SCREEN_PER_STREAM && c->lds_mode == 2;
   std::vector<char> merged(kNumClassPairs, 0);
   for (int k = 0; k < kNumClassPairs && can_merge; ++k) {
-    const CPMeta& m = c->cps[mt][k];
+    const CPMeta& m = c->cps[2][k];
     merged[k] = c->class_variant[k] < 0 && c->class_stream[k] < 0 && stream_of[k] >= 0 && m.ngrp > 0 &&
-                c->batch_start[mt][k].size() == 2 && m.mmax >= 1 &&
-                group_lds(c, kClassKernels[k], m.flip ? 2 : 1, m.mmax, m.ub) <= c->max_dyn_lds;
+                c->batch_start[2][k].size() == 2 && m.mmax >= 1 &&
+                group_lds(c, kClassKernels[k].mrg, m.flip ? 2 : 1, m.mmax, m.ub) <= c->max_dyn_lds;
   }
   std::vector<char> fused(kNumClassPairs, 0);
   std::vector<int> once[cq_ctx::kAux + 1];   // per stream, in launch order
@@ -1992,7 +1976,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   auto screen_of = [&](const int* ks, int n, bool merge) {
     ScreenList sl = screen_list_base();
     for (int i = 0; i < n; ++i) {
-      const int k = ks[i], tb = merge ? mt : variant_of(k) >= 2 ? 1 : 0;
+      const int k = ks[i], tb = merge ? 2 : variant_of(k) >= 2 ? 1 : 0;
       const std::vector<int>& bs = c->batch_start[tb][k];
       add_screen_entry(sl, k, tb, bs[0], bs[1] - bs[0], c->batch_slots[tb][k][0]);
     }
@@ -2000,35 +1984,31 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   };
   auto launch_tier = [&](int t, hipStream_t st) {
     MergedArgs ma{};
-    std::vector<int> ks;
     size_t lds = 0;
     int nblk = 0;
     for (int kk = kNumClassPairs - 1; kk >= 0; --kk) {   // highest angular momentum first
       const int k = c->launch_order[kk];
       const ClassKernels& ck = kClassKernels[k];
       if (ck.tier != t || !merged[k]) continue;
-      const CPMeta& m = c->cps[mt][k];
+      const CPMeta& m = c->cps[2][k];
       const int kv = m.flip ? 2 : 1;
-      c->last_table[k] = mt;
-      ks.push_back(k);
+      c->last_table[k] = 2;
       MergedEntry& e = ma.e[ma.n++];
       e.k = k;
-      e.bra = m.flip;
       e.blk0 = nblk;
-      e.cpi = class_chunks_per_item(c, k);
-      e.nblk = (int)std::max<long long>(1, std::min<long long>(persistent_grid() / 4, m.seg_cap * (ck.nchunk / e.cpi)));
+      e.cpi = class_chunks_per_item(c, k, ck.mrg);
+      e.nblk = (int)std::max<long long>(1, std::min<long long>(persistent_grid() / 4, m.seg_cap * (ck.mrg.nchunk / e.cpi)));
       nblk += e.nblk;
-      e.nres = c->batch_slots[mt][k][0];
+      e.nres = c->batch_slots[2][k][0];
       e.mmax = m.mmax;
       e.ub = m.ub;
-      e.lds_n = lds_rows(c, ck, kv);
-      e.rowfn = (kv == 2 ? ck.ki : ck.bi) * c->ncart;
+      e.lds_n = lds_rows(c, ck.mrg, kv);
+      e.rowfn = (kv == 2 ? ck.mrg.ki : ck.mrg.bi) * c->ncart;
       e.task_off = m.task_off;
       e.seg_off = m.seg_off;
-      lds = std::max(lds, group_lds(c, ck, kv, m.mmax, m.ub));
+      lds = std::max(lds, group_lds(c, ck.mrg, kv, m.mmax, m.ub));
     }
-    if (ks.empty()) return;
-    launch_screen(screen_of(ks.data(), (int)ks.size(), true), st, c->prof_screen_events[kNumClassPairs], true);
+    if (ma.n == 0) return;
     ma.slot_words = (long long)slot_words;
     JKArgs jk{};
     jk.ncart = c->ncart;
@@ -2049,8 +2029,8 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
     }
     hipLaunchKernelGGL(kMergedTiers[t].kernel, dim3(nblk, nslot), dim3(kMergedTiers[t].wgs), lds, st, ma, c->d_tasks.p,
                        c->d_segs.p, c->d_ovf.p, c->d_work_q.p, c->d_pairs.p, c->d_prims.p, c->d_boys.p, jk,
-                       c->d_groups[mt].p,
-                       (mt == 2 && c->own_blocks() ? c->d_uorder_m : c->d_uorder).p);
+                       c->d_groups[2].p,
+                       (c->own_blocks() ? c->d_uorder_m : c->d_uorder).p);
     HIPCHK(hipGetLastError());
   };
   if (c->screen_mode == CQ_SCREEN_ONE) {
@@ -2060,8 +2040,15 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   }
   HIPCHK(hipEventRecord(c->ev_fork, s));
   for (int a = 0; a < cq_ctx::kAux; ++a) HIPCHK(hipStreamWaitEvent(c->aux[a], c->ev_fork, 0));
-  if (can_merge)
-    for (int t = 0; t < CQ_NUM_TIERS; ++t) launch_tier(t, stream_at(t));
+  for (int si = 0; can_merge && si <= cq_ctx::kAux; ++si) {
+    std::vector<int> ks;
+    for (int k = 0; k < kNumClassPairs; ++k)
+      if (merged[k] && kMergedTiers[kClassKernels[k].tier].stream == si) ks.push_back(k);
+    if (ks.empty()) continue;
+    launch_screen(screen_of(ks.data(), (int)ks.size(), true), stream_at(si), c->prof_screen_events[kNumClassPairs], true);
+    for (int t = CQ_NUM_TIERS - 1; t >= 0; --t)
+      if (kMergedTiers[t].stream == si) launch_tier(t, stream_at(si));
+  }
   if (c->screen_mode == CQ_SCREEN_PER_STREAM)
     for (int si = 0; si < c->n_streams; ++si)
       if (!once[si].empty())
@@ -2106,7 +2093,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
       JKArgs jkk = jk;   // the LDS rows of this class pair's swept side
       jkk.lds_n = lds_rows(c, ck, kv);
       jkk.rowfn = c->d_rowfn.p + (size_t)(kv == 2 ? ck.ki : ck.bi) * c->ncart;
-      const int cpi = class_chunks_per_item(c, k);
+      const int cpi = class_chunks_per_item(c, k, ck);
       unsigned* wq = c->d_work_q.p + ((size_t)s0 * kNumClassPairs + k) * WORK_QUEUES;
       // batches of groups, in order on this class pair's stream: a class pair in one batch
       // screens once and keeps its lists for every slot pass; a batched one clears its counters
@@ -2763,7 +2750,8 @@ int cq_get_work_stats(cq_ctx_t* c, double* out, int max_n) {
       hipLaunchKernelGGL(work_stats_kernel, dim3(persistent_grid()), dim3(WG), 0, c->stream,
                          c->d_tasks.p + m.task_off, c->d_segs.p + m.seg_off, c->batch_slots[tb][k][0], c->d_ovf.p + k,
                          c->d_groups[tb].p,
-                         (tb == 2 && c->own_blocks() ? c->d_uorder_m : c->d_uorder).p, m.flip, c->d_pairs.p,
+                         (tb == 2 && c->own_blocks() ? c->d_uorder_m : c->d_uorder).p,
+                         m.flip ^ (tb == 2 && kClassKernels[k].bi != kClassKernels[k].mrg.bi), c->d_pairs.p,
                          tb == 2 ? c->mpblk : PRIM_BLOCK, tb == 2 ? c->mublk : UNI_BLOCK, c->d_shells.p, acc.p + 4 * k);
       HIPCHK(hipGetLastError());
     }

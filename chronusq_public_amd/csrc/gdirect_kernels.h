@@ -114,6 +114,7 @@ __device__ __forceinline__ int take_item(unsigned* __restrict__ work, unsigned b
 // task lists and running block counts in LDS.
 struct ItemLds {
   int next;                      // the item after this one, taken while this one runs
+  int unit;                      // next unit to hand out
   int sh[MAX_GROUP];             // first function of each member's own (second) shell
   int joff[MAX_GROUP];           // its Coulomb block
   int moff[MAX_GROUP], mcnt[MAX_GROUP];
@@ -142,6 +143,13 @@ __device__ __forceinline__ void stage_members(ItemLds& it, const GroupRec& gr, c
     }
     if (m < gr.n) it.mblk[m] = nb;
   }
+}
+
+// Hands the calling wavefront the next unit of the item (beyond the wavefronts' first ones).
+__device__ __forceinline__ int next_unit(ItemLds& it) {
+  int u = 0;
+  if ((threadIdx.x & 63) == 0) u = atomicAdd(&it.unit, 1);
+  return __builtin_amdgcn_readfirstlane(u);
 }
 
 // Unit u of the item: chunk, member (wavefront-uniform) and 64-entry block of its list; units are
@@ -218,16 +226,18 @@ __device__ __forceinline__ void group_body(
     const int n = gr.n;
     const uint2* reg = tasks + sg.off;
     int U = 0;
+    if (threadIdx.x == 0) s_it.unit = WGS / 64;
     if (filled) {
       U = (int)reg[0].y;
       stage_members(s_it, gr, reg, pairs, uorder);
     }
     __syncthreads();
     if (filled) {
-      // units (chunk, member, 64-entry block of the member's list), chunk-major, over the
-      // workgroup's wavefronts: the member is wavefront-uniform
+      // units (chunk, member, 64-entry block of the member's list), chunk-major, handed to the
+      // workgroup's wavefronts as they come free (a member's list runs from heavily contracted to
+      // single primitives): the member is wavefront-uniform
       const int nbt = __builtin_amdgcn_readfirstlane(s_it.mblk[n - 1]);
-      for (int u = wid; u < nbt * cpi; u += WGS / 64) {
+      for (int u = wid; u < nbt * cpi; u = next_unit(s_it)) {
         int dch, mu, eb;
         locate_unit(s_it, n, nbt, cpi, u, dch, mu, eb);
         const int b0 = eb << 6, t = b0 + lane;
@@ -345,7 +355,7 @@ __device__ __forceinline__ void group_body(
 // series, 243 us merged.  A merged launch runs all class pairs of one tier (similar register
 // counts) side by side, one range of blocks per class pair, and one grid row (y) per density slot.
 struct MergedEntry {
-  int k, bra;                    // class pair; 1: bra-keyed groups, 0: ket-keyed
+  int k;                         // class pair
   int blk0, nblk;                // its blocks
   int nres, mmax, ub, cpi, lds_n, rowfn;
   long long task_off, seg_off;
@@ -389,15 +399,21 @@ typedef void (*GroupKernel)(const uint2*, const Segment*, int, const unsigned*, 
 typedef void (*MergedKernel)(MergedArgs, const uint2*, const Segment*, const unsigned*, unsigned*, const PairInfo*,
                              const PrimPair*, const double*, JKArgs, const GroupRec*, const int*);
 
-struct ClassKernels {
-  int i, j, bi, ki, L, nchunk;
+// Bra and ket class, chunks, name and sizes of a class pair in one orientation.
+struct ClassShape {
+  int bi, ki, nchunk;
   const char* name;
+  int nc, nd, na, nb;
+};
+
+struct ClassKernels : ClassShape {
+  int i, j, L;
   BlockKernel block;
   // grp[precision][variant]: precision 0 FP64 / 1 FP32 integrals; variant 0 ket-keyed with HBM K
   // atomics, 1 ket-keyed with LDS K columns, 2 bra-keyed with LDS K rows (null where the class
   // pair has no bra-keyed form)
   GroupKernel grp[2][3];
-  int nc, nd, na, nb;
   int seg_wg;         // workgroup size of the ket-keyed kernels
-  int tier, merged;   // merged launch the class pair belongs to, forms it has there (1 ket-keyed, 2 bra-keyed)
+  int tier, merged;   // merged launch the class pair belongs to, its form there (1 ket-keyed, 2 bra-keyed)
+  ClassShape mrg;     // its orientation there
 };

@@ -614,21 +614,37 @@ def orientation(X, Y):
     return (X, Y) if w1 <= w2 else (Y, X)
 
 
-# Merged launches: (workgroup size, wavefronts per SIMD, class pairs).  A tier's kernel needs the
-# registers of its largest class pair, so the tiers follow the register counts.
+def merged_orientation(X, Y):
+    """Bra and ket of a class pair's merged kernel: as orientation, but an (ss) class is the ket of
+    every class above (ps).  A primitive quartet's ket transform is then one term per Hermite
+    integral and the bra's coefficients are formed once per bra primitive: (ss|dp) 319 vector
+    instructions per primitive quartet, (dp|ss) 102; (ss|pp) 147 and 82, (ss|ds) 124 and 80.  (ss|ps)
+    57 and 55 gain nothing, and its swept (ss) pairs fill the lanes better ((H2O)11/6-31G 780 us
+    against 810).  The launches per class pair keep orientation: their FP32 forms would round
+    differently."""
+    bra, ket = orientation(X, Y)
+    return (ket, bra) if bra == (0, 0) and sum(ket) > 1 else (bra, ket)
+
+
+# Merged launches: (workgroup size, wavefronts per SIMD, stream, class pairs).  A tier's kernel needs
+# the registers of its largest class pair, so the tiers follow the register counts.  Tiers that
+# share a stream run in reverse order (the higher angular momentum first).
 TIERS = [
-    (512, 4, ["ssss", "ssps", "psps", "sspp", "ssds"]),
-    (256, 2, ["psds", "ssdp", "ppps", "pppp", "ppds", "dsds", "dpps"]),
-    (256, 2, ["dppp", "dpds", "dpdp", "ddss", "ddps"]),
-    (256, 1, ["ddpp", "ddds", "dddp", "dddd"]),
+    (512, 6, 0, ["ssss", "ssps"]),
+    (512, 4, 1, ["psps", "ppss", "dsss"]),
+    (256, 2, 2, ["psds", "dpss", "ppps", "pppp", "ppds", "dsds", "dpps"]),
+    (256, 2, 3, ["dppp", "dpds", "dpdp", "ddss", "ddps"]),
+    (256, 1, 0, ["ddpp", "ddds", "dddp", "dddd"]),
 ]
 
 
-def merged_forms(name, segb):
-    """Digestion forms (1 ket-keyed, 2 bra-keyed) of a class pair's merged kernel: both where
-    either side can have fewer pairs; the bra-keyed one alone for the other class pairs that have
-    it (few pairs of the higher class, many lanes of the lower), which halves their code."""
-    return (1, 2) if name in ("psds", "ppds") else (2,) if segb else (1,)
+def merged_form(name, segb):
+    """Digestion form (1 ket-keyed, 2 bra-keyed) of a class pair's merged kernel: bra-keyed where the
+    bra class has few pairs and the ket class many (a list holds one lane task per swept pair), except
+    against an (ss) ket below (dd), where the swept (ss) rows are few and the bra sweep fills the lanes
+    ((H2O)4/cc-pVDZ 474 us against 509 bra-keyed, one water and (H2O)16 the same).  One form each
+    also halves the merged kernels' code."""
+    return 2 if segb and not (name[2:] == "ss" and name[:2] != "dd") else 1
 
 
 def main(out_dir: str, maxl: int = 2):
@@ -638,7 +654,7 @@ def main(out_dir: str, maxl: int = 2):
     os.makedirs(out_dir, exist_ok=True)
     pcl = class_list(maxl)
     table = []
-    segbs = {}
+    merged, register = {}, []
     for i, X in enumerate(pcl):
         for j, Y in enumerate(pcl):
             if j > i:
@@ -661,30 +677,40 @@ def main(out_dir: str, maxl: int = 2):
             # bra-uniform groups pay off where the bra class has far fewer pairs than the ket
             # class (few bras survive per ket): different pair classes and a bra above (ss)
             segb = i != j and (LA, LB) != (0, 0)
-            segbs[name] = segb
             if segb:
                 src.append(f"DEFINE_CLASS_SEGB({name})")
             # ket-keyed groups of an (ss) or (ps) bra class hold many bras per ket: 512-thread
             # workgroups share one Boys table and one set of K columns over 8 wavefronts
             seg_wg = 512 if (LA, LB) in ((0, 0), (1, 0)) else 256
-            tier = [t for t, (_, _, names) in enumerate(TIERS) if name in names][0]
+            mbra, mket = merged_orientation(X, Y)
+            mname = "".join(CLS_NAME[l] for l in mbra + mket)
+            if mname != name:
+                hdr[-1] = gen_class(*mbra, *mket, "jk")
+                _write_if_changed(os.path.join(out_dir, f"cls_{mname}.h"), "\n".join(hdr) + "\n")
+            msegb = i != j and mbra != (0, 0)
+            mform = merged_form(mname, msegb)
+            merged[mname] = (len(table), mform)
+            tier = [t for t, (_, _, _, names) in enumerate(TIERS) if mname in names][0]
             gb = (lambda R: f"eri_grpb_{name}<{R}>") if segb else (lambda R: "nullptr")
-            f32 = src + [f"void cq_f32_{name}(GroupKernel* g) {{",
-                         f"  g[0] = eri_grp_{name}<{seg_wg}, 0, float>;",
-                         f"  g[1] = eri_grp_{name}<{seg_wg}, 1, float>;",
-                         f"  g[2] = {gb('float')};", "}"]
-            _write_if_changed(os.path.join(out_dir, f"f32_{name}.hip"), "\n".join(f32) + "\n")
-            src += [f"BlockKernel cq_block_{name}();", f"void cq_f32_{name}(GroupKernel* g);"]
-            src.append(f"void cq_register_{name}(ClassKernels& ck) {{")
-            src.append(f"  ck = ClassKernels{{{i}, {j}, {pcl.index(bra)}, {pcl.index(ket)}, {L}, Cls_{name}::NCH, \"{name}\", "
-                       f"cq_block_{name}(), "
-                       f"{{{{eri_grp_{name}<{seg_wg}, 0, double>, eri_grp_{name}<{seg_wg}, 1, double>, {gb('double')}}}, {{}}}}, "
-                       f"Cls_{name}::NC, Cls_{name}::ND, Cls_{name}::NA, Cls_{name}::NB, {seg_wg}, {tier}, {sum(merged_forms(name, segb))}}};")
-            src.append(f"  cq_f32_{name}(ck.grp[1]);")
-            src.append("}")
-            _write_if_changed(os.path.join(out_dir, f"eri_{name}.hip"), "\n".join(src) + "\n")
+            for pre, R in (("eri", "double"), ("f32", "float")):
+                fn = "cq_f64" if R == "double" else "cq_f32"
+                unit = src + [f"void {fn}_{name}(GroupKernel* g) {{",
+                              f"  g[0] = eri_grp_{name}<{seg_wg}, 0, {R}>;",
+                              f"  g[1] = eri_grp_{name}<{seg_wg}, 1, {R}>;",
+                              f"  g[2] = {gb(R)};", "}"]
+                _write_if_changed(os.path.join(out_dir, f"{pre}_{name}.hip"), "\n".join(unit) + "\n")
+
+            def shape(b, k):
+                chunks, persist = plan_class(*b, *k)
+                nm = "".join(CLS_NAME[l] for l in b + k)
+                return (f"ClassShape{{{pcl.index(b)}, {pcl.index(k)}, {1 if persist else len(chunks)}, \"{nm}\", "
+                        f"{ncart(k[0])}, {ncart(k[1])}, {ncart(b[0])}, {ncart(b[1])}}}")
+            register.append(f"  t[{len(table)}] = ClassKernels{{{shape(bra, ket)}, {i}, {j}, {L}, cq_block_{name}(), {{}}, "
+                            f"{seg_wg}, {tier}, {mform}, {shape(mbra, mket)}}};")
+            register.append(f"  cq_f64_{name}(t[{len(table)}].grp[0]);")
+            register.append(f"  cq_f32_{name}(t[{len(table)}].grp[1]);")
             table.append(name)
-    for t, (wgs, waves, names) in enumerate(TIERS):
+    for t, (wgs, waves, _, names) in enumerate(TIERS):
         src = ["// GENERATED by gen_eri.py -- do not edit."]
         src += [f'#include "cls_{n}.h"' for n in names]
         src += [f"__global__ void __launch_bounds__({wgs}, {waves}) eri_merged_{t}(MERGED_KERNEL_PARAMS) {{",
@@ -695,13 +721,13 @@ def main(out_dir: str, maxl: int = 2):
                 "  const MergedEntry& e = merged_entry(ma, jk0, jk);",
                 "  unsigned* const wq = work + ((size_t)blockIdx.y * CQ_NUM_CLASS_PAIRS + e.k) * WORK_QUEUES;",
                 "  const unsigned blk = blockIdx.x - (unsigned)e.blk0;",
-                "  switch (2 * e.k + e.bra) {"]
+                "  switch (e.k) {"]
         for n in names:
-            for dig in merged_forms(n, segbs[n]):
-                src += [f"    case {2 * table.index(n) + (dig == 2)}:",
-                        f"      group_body<Cls_{n}, {wgs}, {dig}, double>(tasks + e.task_off, segs + e.seg_off, e.nres, ovf + e.k, wq, pairs,",
-                        "          prims, boys, jk, groups, uorder, e.mmax, e.ub, e.cpi, blk, (unsigned)e.nblk, boys_lds, s_it, dyn_lds);",
-                        "      break;"]
+            k, dig = merged[n]
+            src += [f"    case {k}:",
+                    f"      group_body<Cls_{n}, {wgs}, {dig}, double>(tasks + e.task_off, segs + e.seg_off, e.nres, ovf + e.k, wq, pairs,",
+                    "          prims, boys, jk, groups, uorder, e.mmax, e.ub, e.cpi, blk, (unsigned)e.nblk, boys_lds, s_it, dyn_lds);",
+                    "      break;"]
         src += ["    default: break;", "  }", "}",
                 f"MergedKernel cq_merged_{t}() {{ return eri_merged_{t}; }}"]
         _write_if_changed(os.path.join(out_dir, f"merged_{t}.hip"), "\n".join(src) + "\n")
@@ -710,17 +736,18 @@ def main(out_dir: str, maxl: int = 2):
     _write_if_changed(os.path.join(out_dir, "eri_counts.inc"), "\n".join(cnt) + "\n")
     reg = ["// GENERATED by gen_eri.py -- do not edit."]
     for name in table:
-        reg.append(f"void cq_register_{name}(ClassKernels& ck);")
+        reg.append(f"BlockKernel cq_block_{name}();")
+        reg.append(f"void cq_f64_{name}(GroupKernel* g);")
+        reg.append(f"void cq_f32_{name}(GroupKernel* g);")
     reg.append("static inline void cq_register_all(ClassKernels* t) {")
-    for k, name in enumerate(table):
-        reg.append(f"  cq_register_{name}(t[{k}]);")
+    reg += register
     reg.append("}")
     for t in range(len(TIERS)):
         reg.append(f"MergedKernel cq_merged_{t}();")
-    reg.append("struct MergedTier { MergedKernel kernel; int wgs; };")
+    reg.append("struct MergedTier { MergedKernel kernel; int wgs, stream; };")
     reg.append("static inline void cq_merged_all(MergedTier* t) {")
-    for t, (wgs, _, _) in enumerate(TIERS):
-        reg.append(f"  t[{t}] = MergedTier{{cq_merged_{t}(), {wgs}}};")
+    for t, (wgs, _, stream, _) in enumerate(TIERS):
+        reg.append(f"  t[{t}] = MergedTier{{cq_merged_{t}(), {wgs}, {stream}}};")
     reg.append("}")
     _write_if_changed(os.path.join(out_dir, "eri_registry.inc"), "\n".join(reg) + "\n")
 
