@@ -28,6 +28,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <memory>
 #include <mutex>
 #include <cmath>
 #include <cstdio>
@@ -661,44 +662,66 @@ __global__ void sph_transform_kernel(const double* __restrict__ Mc, OutList out,
 
 // Schwarz: Q(P) = sqrt(max_{ij} |(ij|ij)|) in the shells' own (pure or Cartesian) basis,
 // from the Cartesian diagonal block (ab|ab) of each pair.
-__global__ void schwarz_kernel(const double* __restrict__ blocks, const int* __restrict__ pair_ids, int npair,
+// A power-of-two run of lanes per pair, one diagonal element (ij|ij) per lane, over the at most three
+// Cartesian functions of a d, p or s function that count: with one lane per pair and the six of a
+// shell tested in turn, the 25 elements of a (dd) pair ran in series ((H2O)16/cc-pVDZ, (dd):
+// 299 us; 19 so).
+__global__ void schwarz_kernel(const double* __restrict__ blocks, const int* __restrict__ pair_ids, int npair, int lanes,
                                const PairInfo* __restrict__ pairs, const ShellMeta* __restrict__ sh,
                                const double* __restrict__ tco, const int* __restrict__ tco_off,
                                double* __restrict__ pairQ) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= npair) return;
-  const int P = pair_ids[k];
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = (int)(t / lanes), f0 = (int)(t % lanes);
+  const bool active = k < npair;
+  const int P = pair_ids[active ? k : npair - 1];
   const PairInfo pi = pairs[P];
   const ShellMeta A = sh[pi.a], B = sh[pi.b];
   const int nca = (A.l + 1) * (A.l + 2) / 2, ncb = (B.l + 1) * (B.l + 2) / 2;
   const int nab = nca * ncb;
   const int na = A.pure ? 2 * A.l + 1 : nca;
   const int nb = B.pure ? 2 * B.l + 1 : ncb;
-  const double* blk = blocks + (long)k * nab * nab;
-  double mx = 0.0;
-  for (int i = 0; i < na; ++i)
-    for (int j = 0; j < nb; ++j) {
-      double s = 0.0;
-      for (int a = 0; a < nca; ++a) {
-        const double ta = tcoef(A, i, a, tco, tco_off);
-        if (ta == 0.0) continue;
-        for (int b = 0; b < ncb; ++b) {
-          const double tb = tcoef(B, j, b, tco, tco_off);
-          if (tb == 0.0) continue;
-          for (int c = 0; c < nca; ++c) {
-            const double tc = tcoef(A, i, c, tco, tco_off);
-            if (tc == 0.0) continue;
-            for (int d = 0; d < ncb; ++d) {
-              const double td = tcoef(B, j, d, tco, tco_off);
-              if (td == 0.0) continue;
-              s += ta * tb * tc * td * blk[(long)(a * ncb + b) * nab + c * ncb + d];
-            }
-          }
-        }
-      }
-      mx = fmax(mx, fabs(s));
+  const double* blk = blocks + (long)(active ? k : npair - 1) * nab * nab;
+  // the Cartesian functions (in order) and coefficients of function f of a shell; 0: none
+  auto terms = [&](const ShellMeta& S, int f, int nc, int (&id)[3], double (&co)[3]) {
+    int n = 0;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) { id[x] = 0; co[x] = 0.0; }
+#pragma unroll
+    for (int x = 0; x < 6; ++x) {
+      const double v = x < nc ? tcoef(S, f, x, tco, tco_off) : 0.0;
+      if (v == 0.0) continue;
+#pragma unroll
+      for (int y = 0; y < 3; ++y)
+        if (n == y) { id[y] = x; co[y] = v; }
+      ++n;
     }
-  pairQ[P] = sqrt(mx);
+  };
+  double mx = 0.0;
+  for (int f = f0; f < na * nb; f += lanes) {
+    int ia[3], ib[3];
+    double ca[3], cb[3];
+    terms(A, f / nb, nca, ia, ca);
+    terms(B, f % nb, ncb, ib, cb);
+    double s = 0.0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = 0; b < 3; ++b) {
+        const double tab = ca[a] * cb[b];
+        if (tab == 0.0) continue;
+        const double* row = blk + (long)(ia[a] * ncb + ib[b]) * nab;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            const double v = row[ia[c] * ncb + ib[d]];
+            s = ca[c] == 0.0 || cb[d] == 0.0 ? s : s + tab * ca[c] * cb[d] * v;
+          }
+      }
+    mx = fmax(mx, fabs(s));
+  }
+  for (int o = lanes / 2; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  if (active && f0 == 0) pairQ[P] = sqrt(mx);
 }
 
 // Work sums over one class pair's task regions, for the algorithmic FLOP model (kernel
@@ -857,27 +880,84 @@ std::vector<double> boys_table() {
     }                                                                                       \
   } while (0)
 
+// Device memory of a context's small buffers, in one slab instead of some forty allocations (and
+// frees) of about 10 us each, and their first contents in as few copies as their neighbourhoods allow:
+// stage() writes the slab's host image, flush() copies what was staged since the last one.  Given
+// back with the context.
+struct Arena {
+  static constexpr size_t kSlab = 1 << 20, kLargest = 256 << 10, kAlign = 256;
+  struct Slab { char* dev; size_t size, used; std::unique_ptr<char[]> host; };
+  struct Range { size_t slab, lo, hi; };
+  std::vector<Slab> slabs;
+  std::vector<Range> dirty;
+  char* take(size_t bytes) {
+    bytes = (bytes + kAlign - 1) / kAlign * kAlign;
+    if (slabs.empty() || slabs.back().size - slabs.back().used < bytes) {
+      slabs.push_back(Slab{nullptr, std::max(bytes, kSlab), 0, nullptr});
+      HIPCHK(hipMalloc(&slabs.back().dev, slabs.back().size));
+      slabs.back().host.reset(new char[slabs.back().size]);
+    }
+    Slab& b = slabs.back();
+    b.used += bytes;
+    return b.dev + b.used - bytes;
+  }
+  void stage(const void* at, const void* src, size_t bytes) {
+    for (size_t k = slabs.size(); k-- > 0;) {
+      Slab& b = slabs[k];
+      if ((const char*)at < b.dev || (const char*)at >= b.dev + b.size) continue;
+      const size_t lo = (const char*)at - b.dev, hi = lo + bytes;
+      std::memcpy(b.host.get() + lo, src, bytes);
+      Range* r = dirty.empty() ? nullptr : &dirty.back();
+      if (r && r->slab == k && r->hi <= lo && lo - r->hi < kAlign) r->hi = hi;
+      else dirty.push_back(Range{k, lo, hi});
+      return;
+    }
+  }
+  void flush(hipStream_t s) {
+    for (const Range& r : dirty)
+      HIPCHK(hipMemcpyAsync(slabs[r.slab].dev + r.lo, slabs[r.slab].host.get() + r.lo, r.hi - r.lo, hipMemcpyHostToDevice, s));
+    dirty.clear();
+  }
+  void release() {
+    for (Slab& b : slabs)
+      if (b.dev) (void)hipFree(b.dev);
+    slabs.clear();
+  }
+};
+
 template <typename T>
 struct DevBuf {
   T* p = nullptr;
   size_t n = 0;
-  void ensure(size_t need) {
+  bool own = true;   // false: in an arena
+  void ensure(size_t need, Arena* a = nullptr) {
     if (need <= n && p) return;
-    if (p) HIPCHK(hipFree(p));
+    const bool first = !p;
+    if (p && own) HIPCHK(hipFree(p));
     p = nullptr;
     n = 0;
+    own = true;
     if (need == 0) return;
-    HIPCHK(hipMalloc(&p, need * sizeof(T)));
+    if (a && first && need * sizeof(T) <= Arena::kLargest) {
+      p = (T*)a->take(need * sizeof(T));
+      own = false;
+    } else {
+      HIPCHK(hipMalloc(&p, need * sizeof(T)));
+    }
     n = need;
   }
-  void upload(const std::vector<T>& v, hipStream_t s) {
-    ensure(v.size());
-    if (!v.empty()) HIPCHK(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s));
+  // with an arena: staged there (until its flush) where the buffer is
+  void upload(const std::vector<T>& v, hipStream_t s, Arena* a = nullptr) {
+    ensure(v.size(), a);
+    if (v.empty()) return;
+    if (a && !own) a->stage(p, v.data(), v.size() * sizeof(T));
+    else HIPCHK(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s));
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p && own) (void)hipFree(p);
     p = nullptr;
     n = 0;
+    own = true;
   }
 };
 
@@ -894,7 +974,9 @@ struct cq_ctx {
   std::vector<double> pairQ;
   std::vector<int> class_start;      // npc + 1 (two-electron pair list)
   std::vector<int> class_start_1e;   // npc + 1 (every shell pair, one-electron integrals)
-  std::vector<PrimPair> prims;
+  size_t nprim_pair = 0;
+  Arena arena;
+  Arena* building = nullptr;         // the arena while the context is built
   std::vector<double> Q;             // nshell x nshell
   double tau = 1e-14;                // include/aointegrals.h:334
   int precision_mode = 0;
@@ -1018,6 +1100,7 @@ struct cq_ctx {
     }
     if (ev_fork) (void)hipEventDestroy(ev_fork);
     d_s12.release(); d_grp.release(); d_cls_grp_off.release(); d_pair_mol.release(); d_cmg.release();
+    arena.release();
     if (stream && own_stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -1025,6 +1108,23 @@ struct cq_ctx {
 namespace {
 
 int pair_class(int la, int lb) { return la * (la + 1) / 2 + lb; }
+
+// Stable ascending order of ids by key[id] (bytewise, from the lowest byte that differs up): a few
+// linear passes where a comparison sort of the same ids costs an indirect compare per step.
+void radix_order(const std::vector<unsigned long long>& key, int* ids, size_t n, std::vector<int>& tmp) {
+  if (n < 2) return;
+  unsigned long long diff = 0;
+  for (size_t i = 1; i < n; ++i) diff |= key[ids[i]] ^ key[ids[0]];
+  tmp.resize(std::max(tmp.size(), n));
+  for (int sh = 0; sh < 64; sh += 8) {
+    if (!((diff >> sh) & 255)) continue;
+    size_t at[257] = {0};
+    for (size_t i = 0; i < n; ++i) ++at[((key[ids[i]] >> sh) & 255) + 1];
+    for (int b = 0; b < 256; ++b) at[b + 1] += at[b];
+    for (size_t i = 0; i < n; ++i) tmp[at[(key[ids[i]] >> sh) & 255]++] = ids[i];
+    std::copy(tmp.begin(), tmp.begin() + n, ids);
+  }
+}
 
 int grid_for(long n, int block) { return (int)std::max<long>(1, (n + block - 1) / block); }
 
@@ -1164,6 +1264,17 @@ void plan_tasks(cq_ctx* c) {
     c->batch_slots[t].assign(kNumClassPairs, std::vector<int>());
   }
   const long long budget = c->task_budget;
+  // pairs and primitive blocks (of the launches per class pair, of the merged ones) per class and molecule
+  std::vector<long long> pairs_m((size_t)c->npc * nm, 0), blocks_m[2];
+  for (int o = 0; o < (own ? 2 : 1); ++o) {
+    blocks_m[o].assign((size_t)c->npc * nm, 0);
+    const std::vector<unsigned char>& nblk = o ? c->nblk_m : c->nblk_h;
+    for (int X = 0; X < c->npc; ++X)
+      for (int k = c->class_start[X]; k < c->class_start[X + 1]; ++k) {
+        blocks_m[o][(size_t)X * nm + pair_mol[k]] += nblk[k];
+        if (o == 0) pairs_m[(size_t)X * nm + pair_mol[k]] += 1;
+      }
+  }
   // every class pair has its own part of the task and segment lists, as large as the largest of
   // its tables needs (a call runs a class pair from one table, and different class pairs from
   // different ones)
@@ -1186,9 +1297,9 @@ void plan_tasks(cq_ctx* c) {
       const std::vector<unsigned char>& nublk = t < 2 || !own ? c->nublk_h : c->nublk_m;
       const std::vector<int>& uorder = t < 2 || !own ? c->uorder_h : c->uorder_m;
       // swept-side pairs and primitive blocks per molecule
-      std::vector<long long> bp_m(nm, 0), kp_m(nm, 0), bb_m(nm, 0), kb_m(nm, 0);
-      for (int i = 0; i < m.nbra; ++i) { bp_m[pair_mol[m.bra_start + i]] += 1; bb_m[pair_mol[m.bra_start + i]] += nblk[m.bra_start + i]; }
-      for (int i = 0; i < m.nket; ++i) { kp_m[pair_mol[m.ket_start + i]] += 1; kb_m[pair_mol[m.ket_start + i]] += nblk[m.ket_start + i]; }
+      const std::vector<long long>& blk_m = blocks_m[t == 2 && own];
+      const long long *bp_m = &pairs_m[(size_t)sh.bi * nm], *kp_m = &pairs_m[(size_t)sh.ki * nm];
+      const long long *bb_m = &blk_m[(size_t)sh.bi * nm], *kb_m = &blk_m[(size_t)sh.ki * nm];
       CPMeta& mc = mt[t];
       mc = m;
       mc.flip = bra_keyed(k, t);
@@ -1286,12 +1397,12 @@ void plan_tasks(cq_ctx* c) {
   }
   c->task_capacity = off;
   for (int t = 0; t < 3; ++t) {
-    c->d_cps[t].upload(c->cps[t], c->stream);
-    c->d_groups[t].upload(c->groups_h[t], c->stream);
+    c->d_cps[t].upload(c->cps[t], c->stream, c->building);
+    c->d_groups[t].upload(c->groups_h[t], c->stream, c->building);
   }
   c->d_tasks.ensure((size_t)std::max<long long>(1, off));
   c->d_segs.ensure((size_t)std::max<long long>(1, seg_off));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  if (!c->building) HIPCHK(hipStreamSynchronize(c->stream));
   c->plan_ok = true;
 }
 
@@ -1313,6 +1424,7 @@ void choose_merge_blocks(cq_ctx* c, int npair, int np_max) {
 
 void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const int* nprim, const double* alpha,
                    const double* coef, const double* origin, const int* mol = nullptr) {
+  c->building = &c->arena;
   HIPCHK(hipGetDevice(&c->device));
   HIPCHK(hipStreamCreate(&c->stream));
   for (int k = 0; k < cq_ctx::kAux; ++k) {
@@ -1392,7 +1504,7 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
           c->lds_n_set[pc] = std::max(c->lds_n_set[pc], r);
         }
       }
-    c->d_rowfn.upload(rowfn, c->stream);
+    c->d_rowfn.upload(rowfn, c->stream, c->building);
   }
   // solid-harmonic tables for l = 0..2
   c->tco_off.assign(5, 0);
@@ -1405,10 +1517,10 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
   }
   // shell pairs (canonical s1 >= s2) and their primitive pairs, built by up to 16 host threads
   // over ranges of s1 (equal shares of the canonical pairs) and joined in s1 order, so the
-  // list is the same as a serial build's; a pair's primitive pairs are allprim[off, off + n)
+  // list is the same as a serial build's; a pair's primitive pairs are [off, off + n) of the parts end to end
   struct HostPair { PairInfo info; int cls; long off; int n; };
   std::vector<HostPair> hp;
-  std::vector<PrimPair> allprim;
+  std::vector<std::vector<PrimPair>> pparts;   // one part per thread, uploaded as they are
   const double pi = 3.14159265358979323846;
   const double q_num = 2.0 * std::pow(pi, 2.5), q_half = std::sqrt(q_num);
   auto build_range = [&](int s1_lo, int s1_hi, std::vector<HostPair>& out, std::vector<PrimPair>& prims) {
@@ -1458,7 +1570,7 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     for (int t = 1; t < nthr; ++t)   // s1 < cut[t] holds about t / nthr of the canonical pairs
       cut[t] = std::max(cut[t - 1], std::min(nshell, (int)std::lround(nshell * std::sqrt((double)t / nthr))));
     std::vector<std::vector<HostPair>> parts(nthr);
-    std::vector<std::vector<PrimPair>> pparts(nthr);
+    pparts.resize(nthr);
     std::vector<std::exception_ptr> errs(nthr);
     std::vector<std::thread> pool;
     for (int t = 1; t < nthr; ++t)
@@ -1469,52 +1581,38 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     for (auto& th : pool) th.join();
     for (auto& e : errs)
       if (e) std::rethrow_exception(e);
-    size_t total = 0, ptotal = 0;
-    for (int t = 0; t < nthr; ++t) { total += parts[t].size(); ptotal += pparts[t].size(); }
+    size_t total = 0;
+    for (int t = 0; t < nthr; ++t) total += parts[t].size();
     hp.reserve(total);
-    allprim.reserve(ptotal);
     for (int t = 0; t < nthr; ++t) {
-      const long base = (long)allprim.size();
-      allprim.insert(allprim.end(), pparts[t].begin(), pparts[t].end());
-      for (HostPair h : parts[t]) { h.off += base; hp.push_back(h); }
+      for (HostPair h : parts[t]) { h.off += (long)c->nprim_pair; hp.push_back(h); }
+      c->nprim_pair += pparts[t].size();
     }
   }
-  // the one-electron integrals cover every shell pair; the two-electron lists drop the pairs
-  // without a primitive pair above the threshold (Q = 0: none of their quartets can pass)
-  {
-    std::vector<PairInfo> all;
-    std::vector<int> cls_all;
-    for (auto& h : hp) { all.push_back(h.info); cls_all.push_back(h.cls); }
-    std::vector<int> order(all.size());
-    std::iota(order.begin(), order.end(), 0);
-    // (inside a class the most contracted pairs first: the lanes of a wavefront stay in step)
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-      if (cls_all[x] != cls_all[y]) return cls_all[x] < cls_all[y];
-      return nprim[all[x].a] * nprim[all[x].b] > nprim[all[y].a] * nprim[all[y].b];
-    });
-    std::vector<PairInfo>& sorted_all = c->pairs_1e_h;
-    sorted_all.clear();
-    sorted_all.reserve(all.size());
-    c->class_start_1e.assign(c->npc + 1, 0);
-    for (int k : order) { sorted_all.push_back(all[k]); c->class_start_1e[cls_all[k] + 1]++; }
-    for (int k = 0; k < c->npc; ++k) c->class_start_1e[k + 1] += c->class_start_1e[k];
-    c->d_pairs_1e.upload(sorted_all, c->stream);
-  }
-  hp.erase(std::remove_if(hp.begin(), hp.end(), [](const HostPair& h) { return h.n == 0; }), hp.end());
-  // group by class (stable)
-  std::stable_sort(hp.begin(), hp.end(), [](const HostPair& x, const HostPair& y) { return x.cls < y.cls; });
+  // the two-electron lists drop the pairs without a primitive pair above the threshold (Q = 0: none
+  // of their quartets can pass); at: pairs of hp grouped by class (stable)
+  std::vector<int> at, tmp;
+  std::vector<unsigned long long> key;
   c->class_start.assign(c->npc + 1, 0);
-  for (auto& h : hp) c->class_start[h.cls + 1]++;
+  for (auto& h : hp)
+    if (h.n) c->class_start[h.cls + 1]++;
   for (int k = 0; k < c->npc; ++k) c->class_start[k + 1] += c->class_start[k];
-  // the pair list in hp's order; every pair's primitive pairs stay where the build put them
-  // (allprim, uploaded once), the pair pointing at its range
+  at.resize(c->class_start[c->npc]);
+  {
+    std::vector<int> next(c->class_start.begin(), c->class_start.end() - 1);
+    for (size_t k = 0; k < hp.size(); ++k)
+      if (hp[k].n) at[next[hp[k].cls]++] = (int)k;
+  }
+  // the pair list in the order of at; every pair's primitive pairs stay where the build put them
+  // (uploaded once), the pair pointing at its range
   auto flatten = [&]() {
-    c->pairs.resize(hp.size());
+    c->pairs.resize(at.size());
     int joff = 0;   // at most ncart^2 < 2^31 elements: each ordered shell pair at most once
-    for (size_t k = 0; k < hp.size(); ++k) {
-      PairInfo pi_ = hp[k].info;
-      pi_.p0 = (int)hp[k].off;
-      pi_.p1 = (int)(hp[k].off + hp[k].n);
+    for (size_t k = 0; k < at.size(); ++k) {
+      const HostPair& h = hp[at[k]];
+      PairInfo pi_ = h.info;
+      pi_.p0 = (int)h.off;
+      pi_.p1 = (int)(h.off + h.n);
       pi_.joff = joff;
       joff += ncart_l(l[pi_.a]) * ncart_l(l[pi_.b]);
       c->pairs[k] = pi_;
@@ -1527,22 +1625,29 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
   c->alpha_host.assign(alpha, alpha + poff[nshell]);
   c->coef_host.assign(coef, coef + poff[nshell]);
   c->origin_host.assign(origin, origin + 3 * nshell);
-  c->d_prim_off.upload(c->prim_off_host, c->stream);
-  c->d_alpha.upload(c->alpha_host, c->stream);
-  c->d_coef.upload(c->coef_host, c->stream);
-  c->d_origin.upload(c->origin_host, c->stream);
-  c->d_shells.upload(c->shells, c->stream);
-  c->d_cart2shell.upload(c->cart2shell, c->stream);
-  c->d_sph2shell.upload(c->sph2shell, c->stream);
-  c->d_tco.upload(c->tco, c->stream);
-  c->d_tco_off.upload(c->tco_off, c->stream);
+  c->d_prim_off.upload(c->prim_off_host, c->stream, c->building);
+  c->d_alpha.upload(c->alpha_host, c->stream, c->building);
+  c->d_coef.upload(c->coef_host, c->stream, c->building);
+  c->d_origin.upload(c->origin_host, c->stream, c->building);
+  c->d_shells.upload(c->shells, c->stream, c->building);
+  c->d_cart2shell.upload(c->cart2shell, c->stream, c->building);
+  c->d_sph2shell.upload(c->sph2shell, c->stream, c->building);
+  c->d_tco.upload(c->tco, c->stream, c->building);
+  c->d_tco_off.upload(c->tco_off, c->stream, c->building);
   c->boys_host = boys_table();   // stays alive until the stream is synchronised
-  c->d_boys.upload(c->boys_host, c->stream);
-  c->d_pairs.upload(c->pairs, c->stream);
-  if (allprim.size() > (size_t)INT32_MAX) throw std::invalid_argument("too many primitive pairs");
-  c->prims.swap(allprim);
-  c->d_prims.upload(c->prims, c->stream);
-  c->d_pairQ.ensure(npair);
+  c->d_boys.upload(c->boys_host, c->stream, c->building);
+  c->d_pairs.upload(c->pairs, c->stream, c->building);
+  if (c->nprim_pair > (size_t)INT32_MAX) throw std::invalid_argument("too many primitive pairs");
+  c->d_prims.ensure(c->nprim_pair);
+  {
+    size_t base = 0;
+    for (const auto& part : pparts) {
+      if (!part.empty())
+        HIPCHK(hipMemcpyAsync(c->d_prims.p + base, part.data(), part.size() * sizeof(PrimPair), hipMemcpyHostToDevice, c->stream));
+      base += part.size();
+    }
+  }
+  c->d_pairQ.ensure(npair, c->building);
   // Schwarz bounds: diagonal quartets (P|P) per class on the device, the classes on the
   // auxiliary streams; a pair with more than PRIM_BLOCK primitive pairs is split into
   // (block i | block j) tasks that add into the pair's output slot
@@ -1552,7 +1657,7 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     struct Launch { int k; long t0, nt; int s0, ns, nab; size_t out0; };
     std::vector<Launch> launches;
     size_t out_total = 0;
-    for (int k = 0; k < kNumClassPairs; ++k) {
+    for (int k = kNumClassPairs - 1; k >= 0; --k) {   // the longest kernels first
       const ClassKernels& ck = kClassKernels[k];
       if (ck.i != ck.j) continue;
       const int X = ck.i;
@@ -1581,13 +1686,18 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
       out_total += (size_t)n * nab * nab;
       launches.push_back(L);
     }
-    DevBuf<uint2> dt;
-    DevBuf<int> dslot, di;
+    DevBuf<char> lists;   // tasks, their output slots, the pairs
     DevBuf<double> dblk;
-    dt.upload(tasks, c->stream);
-    dslot.upload(slots, c->stream);
-    di.upload(ids, c->stream);
+    std::vector<char> lists_h(tasks.size() * sizeof(uint2) + (slots.size() + ids.size()) * sizeof(int));
+    char* const lh = lists_h.data();
+    std::copy(tasks.begin(), tasks.end(), (uint2*)lh);
+    std::copy(slots.begin(), slots.end(), (int*)(lh + tasks.size() * sizeof(uint2)));
+    std::copy(ids.begin(), ids.end(), (int*)(lh + tasks.size() * sizeof(uint2)) + slots.size());
+    lists.upload(lists_h, c->stream);
+    const uint2* const dt = (const uint2*)lists.p;
+    const int *const dslot = (const int*)(dt + tasks.size()), *const di = dslot + slots.size();
     dblk.ensure(std::max<size_t>(1, out_total));
+    c->arena.flush(c->stream);
     HIPCHK(hipMemsetAsync(dblk.p, 0, std::max<size_t>(1, out_total) * sizeof(double), c->stream));
     HIPCHK(hipEventRecord(c->ev_fork, c->stream));
     for (int a = 0; a < cq_ctx::kAux; ++a) HIPCHK(hipStreamWaitEvent(c->aux[a], c->ev_fork, 0));
@@ -1596,41 +1706,70 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
       const ClassKernels& ck = kClassKernels[L.k];
       hipStream_t sa = c->aux[li++ % cq_ctx::kAux];
       // slots are per class: the slot array entries count from the class's first pair
-      hipLaunchKernelGGL(ck.block, dim3(grid_for(L.nt, WG)), dim3(WG), 0, sa, dt.p + L.t0, L.nt, c->d_pairs.p,
-                         c->d_prims.p, c->d_boys.p, dblk.p + L.out0, L.nab * L.nab, dslot.p + L.t0);
+      hipLaunchKernelGGL(ck.block, dim3(grid_for(L.nt, WG)), dim3(WG), 0, sa, dt + L.t0, L.nt, c->d_pairs.p,
+                         c->d_prims.p, c->d_boys.p, dblk.p + L.out0, L.nab * L.nab, dslot + L.t0);
       HIPCHK(hipGetLastError());
-      hipLaunchKernelGGL(schwarz_kernel, dim3(grid_for(L.ns, 128)), dim3(128), 0, sa, dblk.p + L.out0, di.p + L.s0,
-                         L.ns, c->d_pairs.p, c->d_shells.p, c->d_tco.p, c->d_tco_off.p, c->d_pairQ.p);
+      int lanes = 1;
+      while (lanes < L.nab && lanes < 64) lanes *= 2;
+      hipLaunchKernelGGL(schwarz_kernel, dim3(grid_for((long)L.ns * lanes, 128)), dim3(128), 0, sa, dblk.p + L.out0, di + L.s0,
+                         L.ns, lanes, c->d_pairs.p, c->d_shells.p, c->d_tco.p, c->d_tco_off.p, c->d_pairQ.p);
       HIPCHK(hipGetLastError());
+    }
+    // meanwhile: the one-electron list, of every shell pair by class (inside a class the most
+    // contracted pairs first: the lanes of a wavefront stay in step)
+    {
+      std::vector<int> order(hp.size());
+      std::iota(order.begin(), order.end(), 0);
+      key.resize(hp.size());
+      c->class_start_1e.assign(c->npc + 1, 0);
+      for (size_t k = 0; k < hp.size(); ++k) {
+        const unsigned np = (unsigned)nprim[hp[k].info.a] * (unsigned)nprim[hp[k].info.b];
+        key[k] = (unsigned long long)hp[k].cls << 32 | (0xffffffffu - np);
+        c->class_start_1e[hp[k].cls + 1]++;
+      }
+      for (int k = 0; k < c->npc; ++k) c->class_start_1e[k + 1] += c->class_start_1e[k];
+      radix_order(key, order.data(), order.size(), tmp);
+      c->pairs_1e_h.clear();
+      c->pairs_1e_h.reserve(hp.size());
+      for (int k : order) c->pairs_1e_h.push_back(hp[k].info);
+      c->d_pairs_1e.upload(c->pairs_1e_h, c->stream);
     }
     for (int a = 0; a < cq_ctx::kAux; ++a) HIPCHK(hipStreamSynchronize(c->aux[a]));
     HIPCHK(hipStreamSynchronize(c->stream));
-    dt.release(); dslot.release(); di.release(); dblk.release();
+    lists.release(); dblk.release();
   }
   c->pairQ.resize(npair);
   HIPCHK(hipMemcpy(c->pairQ.data(), c->d_pairQ.p, npair * sizeof(double), hipMemcpyDeviceToHost));
   // sort within class by primitive-pair count (descending), then Schwarz bound (descending):
   // equal counts side by side keep the lanes of a wavefront in step, and inside each count
   // group the bound order lets screening stop early
+  // (bounds are not negative: their bits are ordered as they are; by bound first, then, stable,
+  // by molecule and count)
   std::vector<int> order(npair);
   std::iota(order.begin(), order.end(), 0);
+  key.resize(npair);
+  for (int k = 0; k < npair; ++k) {
+    unsigned long long bits;
+    std::memcpy(&bits, &c->pairQ[k], sizeof(bits));
+    key[k] = ~bits;
+  }
   for (int X = 0; X < c->npc; ++X)
-    std::stable_sort(order.begin() + c->class_start[X], order.begin() + c->class_start[X + 1], [&](int x, int y) {
-      const int mx = c->shell_mol[hp[x].info.s1], my = c->shell_mol[hp[y].info.s1];
-      if (mx != my) return mx < my;
-      const int nx = hp[x].n, ny = hp[y].n;
-      if (nx != ny) return nx > ny;
-      return c->pairQ[x] > c->pairQ[y];
-    });
-  std::vector<HostPair> hp2;
-  std::vector<double> q2;
-  hp2.reserve(npair);
-  for (int k : order) { hp2.push_back(hp[k]); q2.push_back(c->pairQ[k]); }
-  hp.swap(hp2);
-  c->pairQ.swap(q2);
+    radix_order(key, order.data() + c->class_start[X], c->class_start[X + 1] - c->class_start[X], tmp);
+  for (int k = 0; k < npair; ++k)
+    key[k] = (unsigned long long)c->shell_mol[hp[at[k]].info.s1] << 32 | (0xffffffffu - (unsigned)hp[at[k]].n);
+  for (int X = 0; X < c->npc; ++X)
+    radix_order(key, order.data() + c->class_start[X], c->class_start[X + 1] - c->class_start[X], tmp);
+  {
+    std::vector<int> at2(npair);
+    std::vector<double> q2(npair);
+    for (int k = 0; k < npair; ++k) { at2[k] = at[order[k]]; q2[k] = c->pairQ[order[k]]; }
+    at.swap(at2);
+    c->pairQ.swap(q2);
+  }
   flatten();
-  c->d_pairs.upload(c->pairs, c->stream);
-  c->d_pairQ.upload(c->pairQ, c->stream);
+  c->d_pairs.upload(c->pairs, c->stream, c->building);
+  c->d_pairQ.upload(c->pairQ, c->stream, c->building);
+  c->arena.flush(c->stream);
   {
     const long ns2 = (long)nshell * nshell;
     c->d_jtab.ensure((size_t)ns2);
@@ -1667,16 +1806,16 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     while (next_m <= nm) cm[next_m++] = (int)c->grp.size();
   }
   c->cls_grp_off[c->npc] = (int)c->grp.size();
-  c->d_grp.upload(c->grp, c->stream);
-  c->d_cls_grp_off.upload(c->cls_grp_off, c->stream);
-  c->d_cmg.upload(c->cmg, c->stream);
-  c->d_pair_mol.upload(pair_mol, c->stream);
+  c->d_grp.upload(c->grp, c->stream, c->building);
+  c->d_cls_grp_off.upload(c->cls_grp_off, c->stream, c->building);
+  c->d_cmg.upload(c->cmg, c->stream, c->building);
+  c->d_pair_mol.upload(pair_mol, c->stream, c->building);
   c->pair_mol_h = pair_mol;
   {
     std::vector<int2> s12(npair);
     for (int k = 0; k < npair; ++k) s12[k] = make_int2(c->pairs[k].s1, c->pairs[k].s2);
-    c->d_s12.upload(s12, c->stream);
-    HIPCHK(hipStreamSynchronize(c->stream));
+    c->d_s12.upload(s12, c->stream, c->building);
+    if (c->d_s12.own) HIPCHK(hipStreamSynchronize(c->stream));   // the copy reads s12
   }
   c->Q.assign((size_t)nshell * nshell, 0.0);
   for (int k = 0; k < npair; ++k) {
@@ -1703,10 +1842,10 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     c->nublk_m[k] = (unsigned char)((np + c->mublk - 1) / c->mublk);
   }
   if ((unsigned)npair > PAIR_MASK) throw std::invalid_argument("too many shell pairs");
-  c->d_pair_nblk.upload(nblk, c->stream);
-  c->d_pair_nublk.upload(nublk, c->stream);
   c->nblk_h.swap(nblk);
   c->nublk_h.swap(nublk);
+  c->d_pair_nblk.upload(c->nblk_h, c->stream, c->building);
+  c->d_pair_nublk.upload(c->nublk_h, c->stream, c->building);
   // uniform order of every class: by molecule, primitive blocks and the first shell's contraction
   // (most first: work items are handed out in this order, and a heavily contracted group's items
   // take up to 100 us, so they must not be the last ones), first and second shell (groups are cut
@@ -1714,32 +1853,32 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
   auto uniform_order = [&](std::vector<int>& ord, const std::vector<unsigned char>& nub) {
     ord.resize(npair);
     std::iota(ord.begin(), ord.end(), 0);
+    // 16 bits of molecule and of each shell (a context has at most 46340 functions), 6 of the 1 to 64
+    // blocks, 10 of the contraction (beyond 1023 primitives by shell alone)
+    for (int k = 0; k < npair; ++k) {
+      const unsigned long long a = (unsigned)c->pairs[k].a, b = (unsigned)c->pairs[k].b;
+      key[k] = (unsigned long long)c->pair_mol_h[k] << 48 | (unsigned long long)(64 - nub[k]) << 42 |
+               (unsigned long long)(1023 - std::min(nprim[a], 1023)) << 32 | a << 16 | b;
+    }
     for (int X = 0; X < c->npc; ++X)
-      std::stable_sort(ord.begin() + c->class_start[X], ord.begin() + c->class_start[X + 1], [&](int x, int y) {
-        if (c->pair_mol_h[x] != c->pair_mol_h[y]) return c->pair_mol_h[x] < c->pair_mol_h[y];
-        if (nub[x] != nub[y]) return nub[x] > nub[y];
-        const int ax = c->pairs[x].a, ay = c->pairs[y].a;
-        if (nprim[ax] != nprim[ay]) return nprim[ax] > nprim[ay];
-        if (ax != ay) return ax < ay;
-        return c->pairs[x].b < c->pairs[y].b;
-      });
+      radix_order(key, ord.data() + c->class_start[X], c->class_start[X + 1] - c->class_start[X], tmp);
   };
   uniform_order(c->uorder_h, c->nublk_h);
   if (c->own_blocks()) {
     uniform_order(c->uorder_m, c->nublk_m);
-    c->d_uorder_m.upload(c->uorder_m, c->stream);
-    c->d_pair_nblk_m.upload(c->nblk_m, c->stream);
+    c->d_uorder_m.upload(c->uorder_m, c->stream, c->building);
+    c->d_pair_nblk_m.upload(c->nblk_m, c->stream, c->building);
   }
-  c->d_uorder.upload(c->uorder_h, c->stream);
+  c->d_uorder.upload(c->uorder_h, c->stream, c->building);
   plan_tasks(c);
   c->scratch = scratch_address();
   // WORK_QUEUES work queues per class pair and slot pass; one overflow-slot counter per class pair
-  c->d_work_q.ensure((size_t)kNumClassPairs * MAX_MATS * WORK_QUEUES);
-  c->d_ovf.ensure(kNumClassPairs);
-  c->d_qcounts.ensure(2 * kNumClassPairs);   // surviving quartets: FP64 window, then FP32 window
-  c->d_nglob.ensure(2 + MAX_MATS);   // largest |X| of the call, of each matrix, norm asymmetry flag
-  c->d_Nmax.ensure((size_t)nshell * nshell);
-  c->d_Npair.ensure(std::max(1, npair));
+  c->d_work_q.ensure((size_t)kNumClassPairs * MAX_MATS * WORK_QUEUES, c->building);
+  c->d_ovf.ensure(kNumClassPairs, c->building);
+  c->d_qcounts.ensure(2 * kNumClassPairs, c->building);   // surviving quartets: FP64 window, then FP32 window
+  c->d_nglob.ensure(2 + MAX_MATS, c->building);   // largest |X| of the call, of each matrix, norm asymmetry flag
+  c->d_Nmax.ensure((size_t)nshell * nshell, c->building);
+  c->d_Npair.ensure(std::max(1, npair), c->building);
   c->last_counts.assign(kNumClassPairs, 0);
   c->prof_events.assign(kNumClassPairs, {});
   c->prof_screen_events.assign(kNumClassPairs + 1, {});   // the last: the fused screening launch
@@ -1751,7 +1890,10 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
                    [](int x, int y) { return kClassKernels[x].L < kClassKernels[y].L; });
   c->prof_ms.assign(kNumClassPairs, 0.0);
   c->prof_launches.assign(kNumClassPairs, 0);
+  c->arena.flush(c->stream);
   HIPCHK(hipStreamSynchronize(c->stream));
+  c->building = nullptr;
+  for (Arena::Slab& b : c->arena.slabs) b.host.reset();
 }
 
 struct Slot {
@@ -2370,7 +2512,7 @@ int cq_get_dims(const cq_ctx_t* c, int* nshell, int* nbf, int* ncart, int* npair
   if (nbf) *nbf = c->nsph;
   if (ncart) *ncart = c->ncart;
   if (npair) *npair = (int)c->pairs.size();
-  if (nprim_pair) *nprim_pair = (int)c->prims.size();
+  if (nprim_pair) *nprim_pair = (int)c->nprim_pair;
   return CQ_OK;
 }
 

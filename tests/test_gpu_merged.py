@@ -126,3 +126,16 @@ def test_one_electron_workgroup_edges(name):
     for g, w in zip(got, oracle.OracleBasis(bs).one_electron(mol)):
         g = g.cpu().numpy()
         assert np.isfinite(g).all() and np.abs(g - w).max() < TOL * max(1.0, np.abs(w).max())
+
+
+@pytest.mark.parametrize("name,basis", [("H/6-31g", None), ("NeH/cc-pvdz", None), ("NeH/cc-pvdz", "6-31g*"),
+                                        ("H2O 4/cc-pvdz", None), ("H2O 4/cc-pvdz", "6-31g*")])
+def test_schwarz_bounds_lane_groups(name, basis):
+    """Schwarz bounds with 1 to 64 lanes per pair, pure and Cartesian d, one pair and many per class,
+    against the oracle to 1e-12 of the largest."""
+    mol, bs = _build(name)
+    if basis:
+        bs = B.build_basis(basis, mol.Z, mol.coords_bohr)
+    Q, want = AOIntegrals(bs).computeSchwartz(), oracle.OracleBasis(bs).schwarz()
+    assert np.abs(Q - Q.T).max() == 0.0
+    assert np.abs(Q - want).max() <= 1e-12 * max(1.0, want.max())
