@@ -2096,7 +2096,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   // class pairs one by one (their variant or stream, profiling, the screening mode, one stream)
   // and class pairs in several batches keep a launch per class pair.  (H2O)16/cc-pVDZ 3638 us with
   // a launch per class pair, 3544 merged; smaller systems gain more (choose_merge_blocks).
-  const bool can_merge = nround == 1 && !profiling && c->n_streams == cq_ctx::kAux + 1 &&
+  const bool can_merge = !fp32 && !profiling && c->n_streams == cq_ctx::kAux + 1 &&
                          c->screen_mode == CQ_SCREEN_PER_STREAM && c->lds_mode == 2;
   std::vector<char> merged(kNumClassPairs, 0);
   for (int k = 0; k < kNumClassPairs && can_merge; ++k) {
