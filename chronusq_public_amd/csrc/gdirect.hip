@@ -1410,7 +1410,7 @@ void plan_tasks(cq_ctx* c) {
 // np_max primitive pairs each.  Few quartets leave most of the device idle, and then the longest
 // lane task (block x block primitive quartets in series) sets the time: smaller blocks.  More
 // quartets fill the device, and every block more digests its quartet once more.
-// Measured, G[D] in us with blocks (lane, uniform) 2,8 / 4,8 / 8,32:
+// Measured (before the tiles of today), G[D] in us with blocks (lane, uniform) 2,8 / 4,8 / 8,32:
 //   H2O/6-31G* (55 pairs) 243 / 286 / 412, O2/cc-pVDZ UHF (78) 255 / 302 / 543,
 //   (H2O)4/cc-pVDZ (1176) 548 / 496 / 598, (H2O)11/6-31G UHF (4851) 809 / 772 / 783,
 //   C12H26/6-31G* (7750) 2354 / 2121 / 2064, (H2O)16/cc-pVDZ (18528) 4116 / 3632 / 3544.
@@ -1648,8 +1648,8 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     }
   }
   c->d_pairQ.ensure(npair, c->building);
-  // Schwarz bounds: diagonal quartets (P|P) per class on the device, the classes on the
-  // auxiliary streams; a pair with more than PRIM_BLOCK primitive pairs is split into
+  // Schwarz bounds: diagonal quartets (P|P) per class on the device, the classes on four
+  // streams; a pair with more than PRIM_BLOCK primitive pairs is split into
   // (block i | block j) tasks that add into the pair's output slot
   {
     std::vector<uint2> tasks;
@@ -1704,7 +1704,10 @@ void build_context(cq_ctx* c, int nshell, const int* l, const int* pure, const i
     int li = 0;
     for (const Launch& L : launches) {
       const ClassKernels& ck = kClassKernels[L.k];
-      hipStream_t sa = c->aux[li++ % cq_ctx::kAux];
+      // (four streams: the longest class pairs side by side; on three, (H2O)16's (pp|pp) followed
+      // (dd|dd), 590 us in all instead of 400)
+      const int si = li++ % (cq_ctx::kAux + 1);
+      hipStream_t sa = si < cq_ctx::kAux ? c->aux[si] : c->stream;
       // slots are per class: the slot array entries count from the class's first pair
       hipLaunchKernelGGL(ck.block, dim3(grid_for(L.nt, WG)), dim3(WG), 0, sa, dt + L.t0, L.nt, c->d_pairs.p,
                          c->d_prims.p, c->d_boys.p, dblk.p + L.out0, L.nab * L.nab, dslot + L.t0);
@@ -2091,11 +2094,13 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   // its class pairs behind it, so the kernels start early and the bulk of the screening runs
   // beside other streams' kernels; with CQ_SCREEN_ONE one launch on s before the fork screens
   // them all
-  // merged launches (FP64, default settings): the class pairs of a tier that run in one batch, per
-  // tier one screening and one merged launch on a stream of its own.  Settings that address
-  // class pairs one by one (their variant or stream, profiling, the screening mode, one stream)
-  // and class pairs in several batches keep a launch per class pair.  (H2O)16/cc-pVDZ 3638 us with
-  // a launch per class pair, 3544 merged; smaller systems gain more (choose_merge_blocks).
+  // merged launches (FP64, also the FP64 window of a mixed call; default settings): the class pairs
+  // of a tier that run in one batch, per tier one merged launch on the tier's stream, per stream one
+  // screening launch before them.  Settings that address class pairs one by one (their variant or
+  // stream, profiling, the screening mode, one stream), class pairs in several batches and the FP32
+  // window keep a launch per class pair.  When the merged launches came in, (H2O)16/cc-pVDZ took
+  // 3638 us with a launch per class pair and 3544 merged; smaller systems gain more
+  // (choose_merge_blocks).  Mixed, threshold 1e-5: 3550 us with both windows apart, 3106 so.
   const bool can_merge = !fp32 && !profiling && c->n_streams == cq_ctx::kAux + 1 &&
                          c->screen_mode == CQ_SCREEN_PER_STREAM && c->lds_mode == 2;
   std::vector<char> merged(kNumClassPairs, 0);
