@@ -61,7 +61,7 @@ int cq_ctx_destroy(cq_ctx_t* ctx);
  * molecule per job): the shells of all molecules concatenated, molecule[s] = 0, 1, ...
  * nondecreasing over the shells.  Shell pairs and quartets are formed only within a molecule,
  * so one contraction over the block-diagonal N x N density (N = all molecules' functions)
- * gives every molecule's own G[D] in its diagonal block, with one launch per class pair for
+ * gives every molecule's own G[D] in its diagonal block, with the launches of one molecule for
  * the whole batch.  cq_one_electron rejects such a context. */
 int cq_ctx_create_batch(cq_ctx_t** ctx, int nshell, const int* l, const int* pure, const int* nprim,
                         const double* alpha, const double* coef, const double* origin, const int* molecule);
@@ -153,7 +153,10 @@ int cq_class_pair_info(int k, int* la, int* lb, int* lc, int* ld);
 int cq_set_lds_digestion(cq_ctx_t* ctx, int mode);
 
 /* Digestion variant of one class pair k (0 .. cq_num_class_pairs()-1): 0, 1 or 2 as in
- * cq_set_lds_digestion (capped by the context's mode), -1 to follow the context's mode.  Lets
+ * cq_set_lds_digestion (capped by the context's mode), -1 to follow the context's mode.  A class
+ * pair with a choice of its own (here or in cq_set_class_stream) has a launch of its own; the
+ * others share a few merged launches, except with profiling, fewer than four streams, another
+ * screening or digestion mode than the default, and in the FP32 window.  Lets
  * a tuner pick the fastest variant per class pair from cq_get_kernel_times; results agree to
  * rounding in every variant. */
 int cq_set_class_digestion(cq_ctx_t* ctx, int k, int mode);
@@ -218,7 +221,8 @@ int cq_get_screen_times(cq_ctx_t* ctx, double* ms, long long* launches, int max_
 
 /* How the class pairs that screen once per call are screened: one launch per class pair on
  * its own stream (CQ_SCREEN_PER_CLASS), one launch per stream for the class pairs that run on
- * it, ahead of their kernels (CQ_SCREEN_PER_STREAM, the default), or one launch for all class
+ * it, ahead of their kernels (CQ_SCREEN_PER_STREAM, the default, and the only mode with merged
+ * launches), or one launch for all class
  * pairs before any class kernel starts (CQ_SCREEN_ONE).  The surviving quartets are identical
  * in every mode.  No reference counterpart (the reference screens inside its quartet loop,
  * aointegrals_contract.h:96-131). */
