@@ -629,8 +629,9 @@ def merged_orientation(X, Y):
 # Merged launches: (workgroup size, wavefronts per SIMD, stream, class pairs).  A tier's kernel needs
 # the registers of its largest class pair, so the tiers follow the register counts.  Tiers that
 # share a stream run in reverse order (the higher angular momentum first).  Bound by the latency of
-# FP64 chains at the wavefronts the registers allow: (ss|ss) and (ss|ps) 59 % vector busy at 6 per SIMD
-# (3330 us a (H2O)16/cc-pVDZ contraction; 3505 at 4), the tiers above 25-45 %.  Against this split
+# FP64 chains at the wavefronts the registers allow: alone, on (H2O)16/cc-pVDZ, the tiers issue vector
+# instructions in 50, 30, 33, 26 and 18 % of the cycles (the first at 6 wavefronts per SIMD 3330 us a
+# contraction, at 4 3505, before the tiles of today).  Against this split
 # ((H2O)16 2895 us, C12H26/6-31G* 1783, 24 molecules 7790): the last tier at two wavefronts, spilling,
 # 3018, 1923, 8390; (pp|pp), which spills in the third tier, in the last 2970, 1894, 8000; (dp|dp), (dd|ss)
 # and (dd|ps) in the last 2953, 1848, 8045; the last tier on stream 1, 2 or 3 3106, 3022, 2937 and 2010 to
