@@ -52,6 +52,7 @@ static MergedTier kMergedTiers[CQ_NUM_TIERS];
 // dynamic LDS of the group kernels: what the 64 KiB per workgroup leaves beside the static
 // LDS (Boys table, 26064 B, the work item's members)
 static const size_t kStaticLds = BOYS_ROWS * BOYS_LDS_W * sizeof(double) + 512;
+static_assert(sizeof(ItemLds) <= 512, "the work item's members fit the static LDS set aside for them");
 static const size_t kMaxDynLds = 64 * 1024 - kStaticLds;
 
 // Dynamic LDS the group kernels may use on this device: the device's per-workgroup limit
