@@ -460,7 +460,8 @@ __global__ void pair_elements_kernel(const PairInfo* __restrict__ pairs, int npa
 }
 
 // The nonzero coefficients of one shell function or component in the solid-harmonic transform
-// (l <= 2: at most three Cartesian components per function, two functions per component).
+// (l <= 2: at most three Cartesian components per function, two functions per component).  A pure p
+// shell is transformed too: its functions m = -1, 0, 1 are y, z, x.
 struct TList {
   int n, idx[3];
   double c[3];
@@ -468,13 +469,13 @@ struct TList {
 __device__ __forceinline__ TList sph_to_cart(const ShellMeta& s, int mu, const double* __restrict__ tco,
                                              const int* __restrict__ tco_off) {
   TList t{1, {mu, 0, 0}, {1.0, 0.0, 0.0}};
-  if (s.pure && s.l >= 2) {
+  if (s.pure && s.l >= 1) {
     t.n = 0;
     const int nc = (s.l + 1) * (s.l + 2) / 2;
     const double* T = tco + tco_off[s.l] + mu * nc;
     double v[6];
 #pragma unroll
-    for (int a = 0; a < 6; ++a) v[a] = T[a];
+    for (int a = 0; a < 6; ++a) v[a] = a < nc ? T[a] : 0.0;
 #pragma unroll
     for (int a = 0; a < 6; ++a)
       if (v[a] != 0.0 && t.n < 3) { t.idx[t.n] = a; t.c[t.n] = v[a]; ++t.n; }
@@ -484,13 +485,13 @@ __device__ __forceinline__ TList sph_to_cart(const ShellMeta& s, int mu, const d
 __device__ __forceinline__ TList cart_to_sph(const ShellMeta& s, int a, const double* __restrict__ tco,
                                              const int* __restrict__ tco_off) {
   TList t{1, {a, 0, 0}, {1.0, 0.0, 0.0}};
-  if (s.pure && s.l >= 2) {
+  if (s.pure && s.l >= 1) {
     t.n = 0;
     const int nc = (s.l + 1) * (s.l + 2) / 2;
     const double* T = tco + tco_off[s.l] + a;
     double v[5];
 #pragma unroll
-    for (int m = 0; m < 5; ++m) v[m] = T[m * nc];
+    for (int m = 0; m < 5; ++m) v[m] = m < 2 * s.l + 1 ? T[m * nc] : 0.0;
 #pragma unroll
     for (int m = 0; m < 5; ++m)
       if (v[m] != 0.0 && t.n < 3) { t.idx[t.n] = m; t.c[t.n] = v[m]; ++t.n; }

@@ -1,0 +1,71 @@
+"""GPU: shells whose pure flag differs from the shipped bases' (Cartesian s and p, pure d), which the
+C ABI and ``basis.Shell`` accept: G[D] of symmetric and non-symmetric densities, S, T, V, multipoles
+and Schwarz bounds against the oracle, in the oracle's function order (a pure p shell's functions are
+m = -1, 0, 1, i.e. y, z, x)."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import oracle
+from chronusq_public_amd import basis as B
+from chronusq_public_amd import molecule as M
+from chronusq_public_amd.aointegrals import AOIntegrals, COULOMB, EXCHANGE
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-10
+
+# form: pure flag of shell number i with angular momentum l
+FORMS = {
+    "pure s and p": lambda i, l: True,
+    "every other p pure": lambda i, l: l > 1 or (l == 1 and i % 2 == 0),
+}
+
+
+def _build(basis, form):
+    mol = M.water_cluster(2, seed=9, box_ang=M.scaled_box(2))
+    bs = B.build_basis(basis, mol.Z, mol.coords_bohr)
+    flag = FORMS[form]
+    bs.shells = [dataclasses.replace(s, pure=flag(i, s.l)) for i, s in enumerate(bs.shells)]
+    return mol, bs
+
+
+def _density(N, seed, symmetric):
+    X = np.random.default_rng(seed).uniform(-1, 1, (N, N))
+    return np.asfortranarray(0.5 * (X + X.T) if symmetric else X)
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("basis", ["6-31g", "cc-pvdz"])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_contraction(form, basis, symmetric):
+    print(f"[forms] G[D] {form} {basis} symmetric={symmetric}", flush=True)
+    _, bs = _build(basis, form)
+    ob = oracle.OracleBasis(bs)
+    ao = AOIntegrals(bs)
+    ao.thresholdSchwartz = 1e-12
+    A, C = (_density(bs.nbasis, seed, symmetric) for seed in (3, 4))
+    Xs, types, scales = [A, A, C], [COULOMB, EXCHANGE, EXCHANGE], [1.0, -0.5, 0.25]
+    got = [np.zeros((bs.nbasis, bs.nbasis), order="F") for _ in Xs]
+    want = [np.zeros((ob.nbf, ob.nbf), order="F") for _ in Xs]
+    ao.newTwoEContract(Xs, got, types, scales)
+    n = ob.contract_direct(ao.computeSchwartz(), 1e-12, Xs, want, [0, 1, 1], scales)
+    assert sum(ao.quartet_counts().values()) == n
+    for g, w in zip(got, want):
+        assert np.abs(g - w).max() < TOL
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("basis", ["6-31g", "cc-pvdz"])
+def test_one_electron_and_multipoles(form, basis):
+    print(f"[forms] one-electron {form} {basis}", flush=True)
+    mol, bs = _build(basis, form)
+    ob = oracle.OracleBasis(bs)
+    ao = AOIntegrals(bs)
+    for g, w in zip(ao.computeAOOneE(mol), ob.one_electron(mol)):
+        assert np.abs(g.cpu().numpy() - w).max() < TOL * max(1.0, np.abs(w).max())
+    for g, w in zip(ao.computeMultipole(3, (0.4, -1.3, 0.9)), ob.multipole(3, (0.4, -1.3, 0.9))):
+        assert np.abs(g.cpu().numpy() - w).max() < 1e-12 * max(1.0, np.abs(w).max())
+    Q, want = ao.computeSchwartz(), ob.schwarz()
+    assert np.abs(Q - want).max() <= 1e-12 * max(1.0, want.max())
