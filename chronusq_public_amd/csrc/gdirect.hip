@@ -728,12 +728,14 @@ __global__ void schwarz_kernel(const double* __restrict__ blocks, const int* __r
 
 // Work sums over one class pair's task regions, for the algorithmic FLOP model (kernel
 // orientation: the bra is the (la lb) side): acc[0] += K_ab K_cd (primitive quartets),
-// acc[1] += K_ab, acc[2] += sequential Cartesian->spherical transform cost, acc[3] += output
-// integrals in the shells' basis.  One wavefront per segment.
+// acc[1] += K_ab once per block of kblk primitives of the ket (each digests the bra's primitives
+// anew), acc[2] += sequential Cartesian->spherical transform cost, acc[3] += output integrals in
+// the shells' basis.  kblk is the ket block of the launches per class pair whatever the lists'
+// own blocks are, so a merged launch's lists give the same sums.  One wavefront per segment.
 __global__ void work_stats_kernel(const uint2* __restrict__ tasks, const Segment* __restrict__ segs,
                                   int nres, const unsigned* __restrict__ ovf, const GroupRec* __restrict__ groups,
                                   const int* __restrict__ uorder, int flip, const PairInfo* __restrict__ pairs,
-                                  int pblk, int ublk, const ShellMeta* __restrict__ sh, double* __restrict__ acc) {
+                                  int kblk, const ShellMeta* __restrict__ sh, double* __restrict__ acc) {
   const long nseg = (long)nres + *ovf;
   const int lane = threadIdx.x & 63;
   const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) / 64;
@@ -741,27 +743,22 @@ __global__ void work_stats_kernel(const uint2* __restrict__ tasks, const Segment
   double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
   for (long si = wave; si < nseg; si += nwaves) {
     const Segment sg = segs[si];
-    if (sg.count == 0) continue;
+    // every sum is per quartet: entries other than a pair's first block are further primitive blocks
+    if (sg.count == 0 || sg.blk > 1) continue;
     const GroupRec gr = groups[sg.ket];
     const uint2* reg = tasks + sg.off;
     for (int m = 0; m < gr.n; ++m) {
       const PairInfo Up = pairs[uorder[gr.first + m]];
-      int up0, up1;
-      prim_range(Up, (unsigned)sg.blk, ublk, up0, up1);
       const uint2 hm = reg[1 + m];
       for (int t = lane; t < (int)hm.x; t += 64) {
         const uint2 e = reg[hm.y + t];
+        if (block_of(e.x) > 1) continue;
         const PairInfo Sp = pairs[pair_of(e.x)];
-        int sp0, sp1;
-        prim_range(Sp, block_of(e.x), pblk, sp0, sp1);
         const PairInfo& B = flip ? Up : Sp;
         const PairInfo& K = flip ? Sp : Up;
-        const double kab = flip ? up1 - up0 : sp1 - sp0, kcd = flip ? sp1 - sp0 : up1 - up0;
-        s0 += kab * kcd;
-        s1 += kab;
-        // per-quartet terms once per quartet: entries of a split pair other than its first
-        // block are further primitive blocks of the same quartet
-        if (block_of(e.x) > 1 || sg.blk > 1) continue;
+        const int kab = B.p1 - B.p0, kcd = K.p1 - K.p0;
+        s0 += (double)kab * kcd;
+        s1 += (double)kab * ((kcd + kblk - 1) / kblk);
         const int shl[4] = {B.a, B.b, K.a, K.b};
         double dims[4];
         int l4[4], p4[4];
@@ -2901,7 +2898,7 @@ int cq_get_work_stats(cq_ctx_t* c, double* out, int max_n) {
                          c->d_groups[tb].p,
                          (tb == 2 && c->own_blocks() ? c->d_uorder_m : c->d_uorder).p,
                          m.flip ^ (tb == 2 && kClassKernels[k].bi != kClassKernels[k].mrg.bi), c->d_pairs.p,
-                         tb == 2 ? c->mpblk : PRIM_BLOCK, tb == 2 ? c->mublk : UNI_BLOCK, c->d_shells.p, acc.p + 4 * k);
+                         c->cps[tb == 2 ? 1 : tb][k].flip ? PRIM_BLOCK : UNI_BLOCK, c->d_shells.p, acc.p + 4 * k);
       HIPCHK(hipGetLastError());
     }
     std::vector<double> h((size_t)4 * kNumClassPairs);
