@@ -49,3 +49,22 @@ def test_work_sums_do_not_depend_on_the_launches(m, basis):
         sums.append(np.array(w).reshape(nc, 4))
     assert sums[0][:, 0].sum() > 0
     assert np.array_equal(sums[0], sums[1])
+
+
+def test_plans_that_no_launch_uses_reserve_nothing():
+    """(H2O)100/cc-pVDZ: the merged tiles of class pairs with many d or p rows do not fit the LDS, and
+    the largest class pairs take several batches; neither plan may size the buffers.  Beside the task
+    lists (8 B per entry) a context holds their segments (16 B per region of at least 64 swept pairs'
+    entries and a header), the pair tables and matrices over shells: less than a twentieth of the lists."""
+    import torch
+    bs = _water(100, "cc-pvdz")
+    AOIntegrals(_water(1, "cc-pvdz")).close()   # the library's own first allocations
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    ao = AOIntegrals(bs)
+    used = free - torch.cuda.mem_get_info()[0]
+    entries, batches = ao.task_plan()
+    ao.close()
+    print(f"[plans] context {used / 2**30:.2f} GiB, task lists {entries * 8 / 2**30:.2f} GiB, {batches} batches", flush=True)
+    assert batches > 1
+    assert used - 8 * entries < 8 * entries / 20
