@@ -1165,7 +1165,8 @@ size_t group_lds(const cq_ctx* c, const ClassShape& ck, int variant, int mmax, i
 // pairs sharing a shell), the union bound (swept pairs per task region), the group size then lowered
 // until the LDS budget holds it, and the chunks of a split class pair per work item (0: all).  Few,
 // long work items cost balance; many short ones cost their start and flush, and a swept pair's J is
-// flushed once per group.  The rows come from a coordinate search over (1..16 members) x (128..1024)
+// flushed once per group.
+//   kMergedTiles, the merged launches': from a coordinate search over (1..16 members) x (128..1024)
 // on whole contractions of four molecules at once (water clusters and alkanes, 6-31G* and cc-pVDZ;
 // several molecules in one context: two mixed sets of 16 and 24), each row kept where it gained on
 // their mean: (H2O)16/cc-pVDZ 3320 -> 2890 us, C12H26/6-31G* 2000 -> 1795, (H2O)64/cc-pVDZ 90.3 ->
@@ -1173,60 +1174,77 @@ size_t group_lds(const cq_ctx* c, const ClassShape& ck, int variant, int mmax, i
 // and unions now that a wavefront takes its next unit when it is free: a workgroup's wavefronts
 // no longer wait for the one with the longest lists.  Chunks per item: (H2O)16 (dp|dp) 0.29 -> 0.17
 // ms at 3 ((dd|dd) 0.14 -> 0.08); several molecules G[D] 152 -> 118 ms with all.
+//   kTiles, a class pair's own launch.  Alone on the device it wants more, smaller items than beside
+// others ((ss|ds) of (H2O)16, 4 members x 256 against 16 x 512: 255 against 500 us).  Up to
+// kOwnTilePairs shell pairs the rows come from the same search with every class pair in its own
+// launch, on one stream and on four; above, the merged launches' rows serve here too.  (H2O)16 on one
+// stream 6450 -> 5450 us (four: 3540 -> 3530), C12H26 4900 -> 3780 (2400 -> 2110), (H2O)11/6-31G open
+// shell 2270 -> 2050 (1165 -> 1065), (H2O)16 mixed with both windows apart 8000 -> 7150 (3770 -> 3680).
+// The line: (H2O)24/cc-pVDZ (20500 pairs) on four streams 6.7 ms with the large rows and 6.85 with the
+// small ones, (H2O)64 (75100; class pairs in several batches beside the merged launches) 78.1 and 80.7.
 struct TileDefault { const char* name; int max_group, ub, cpi; };
-static const TileDefault kTileDefaults[] = {
-    {"ssss", 4, 512, 1}, {"ssps", 4, 512, 1}, {"psps", 4, 1024, 1}, {"sspp", 8, 512, 1}, {"ppps", 4, 512, 1},
-    {"pppp", 3, 256, 1}, {"ssds", 16, 512, 1}, {"psds", 8, 512, 1}, {"ppds", 4, 512, 1}, {"dsds", 8, 256, 1},
-    {"ssdp", 1, 512, 1}, {"dpps", 4, 512, 1}, {"dppp", 8, 512, 3}, {"dpds", 16, 256, 1}, {"dpdp", 8, 128, 3},
-    {"ddss", 1, 256, 1}, {"ddps", 1, 512, 1}, {"ddpp", 1, 512, 1}, {"ddds", 1, 512, 1}, {"dddp", 1, 512, 2},
-    {"dddd", 1, 256, 3},
-    {"ppss", 8, 512, 1}, {"dsss", 16, 512, 1}, {"dpss", 4, 128, 1}};
-static const TileDefault kTileDefaultsMulti[] = {
-    {"ssss", 4, 512, 0}, {"ssps", 4, 1024, 0}, {"psps", 16, 1024, 0}, {"sspp", 4, 512, 0}, {"ppps", 2, 512, 0},
-    {"pppp", 16, 512, 0}, {"ssds", 16, 512, 0}, {"psds", 16, 512, 0}, {"ppds", 16, 256, 0}, {"dsds", 16, 512, 0},
-    {"ssdp", 8, 256, 0}, {"dpps", 2, 1024, 0}, {"dppp", 8, 512, 0}, {"dpds", 16, 256, 0}, {"dpdp", 16, 256, 0},
-    {"ddss", 2, 1024, 0}, {"ddps", 2, 1024, 0}, {"ddpp", 1, 128, 0}, {"ddds", 16, 1024, 0}, {"dddp", 4, 1024, 0},
-    {"dddd", 4, 512, 0},
-    {"ppss", 16, 512, 0}, {"dsss", 16, 512, 0}, {"dpss", 8, 256, 0}};
+static const size_t kOwnTilePairs = 20000;
+static const TileDefault kTiles[3][CQ_NUM_CLASS_PAIRS] = {   // up to, above kOwnTilePairs pairs; several molecules
+    {{"ssss", 4, 256, 1}, {"ssps", 4, 384, 1}, {"psps", 4, 512, 1}, {"sspp", 4, 512, 1}, {"ppps", 4, 512, 1},
+     {"pppp", 3, 256, 1}, {"ssds", 4, 256, 1}, {"psds", 8, 512, 1}, {"ppds", 2, 512, 1}, {"dsds", 8, 256, 1},
+     {"ssdp", 1, 512, 1}, {"dpps", 2, 512, 1}, {"dppp", 1, 256, 3}, {"dpds", 4, 256, 1}, {"dpdp", 8, 128, 3},
+     {"ddss", 1, 256, 1}, {"ddps", 1, 512, 1}, {"ddpp", 1, 512, 1}, {"ddds", 1, 512, 1}, {"dddp", 1, 512, 2},
+     {"dddd", 1, 256, 3}},
+    {{"ssss", 4, 512, 1}, {"ssps", 4, 512, 1}, {"psps", 4, 1024, 1}, {"sspp", 8, 512, 1}, {"ppps", 4, 512, 1},
+     {"pppp", 3, 256, 1}, {"ssds", 16, 512, 1}, {"psds", 8, 512, 1}, {"ppds", 4, 512, 1}, {"dsds", 8, 256, 1},
+     {"ssdp", 1, 512, 1}, {"dpps", 4, 512, 1}, {"dppp", 8, 512, 3}, {"dpds", 16, 256, 1}, {"dpdp", 8, 128, 3},
+     {"ddss", 1, 256, 1}, {"ddps", 1, 512, 1}, {"ddpp", 1, 512, 1}, {"ddds", 1, 512, 1}, {"dddp", 1, 512, 2},
+     {"dddd", 1, 256, 3}},
+    {{"ssss", 4, 512, 0}, {"ssps", 4, 1024, 0}, {"psps", 16, 1024, 0}, {"sspp", 4, 512, 0}, {"ppps", 2, 512, 0},
+     {"pppp", 16, 512, 0}, {"ssds", 16, 256, 0}, {"psds", 16, 512, 0}, {"ppds", 16, 256, 0}, {"dsds", 16, 512, 0},
+     {"ssdp", 8, 256, 0}, {"dpps", 2, 1024, 0}, {"dppp", 8, 512, 0}, {"dpds", 16, 256, 0}, {"dpdp", 16, 256, 0},
+     {"ddss", 2, 1024, 0}, {"ddps", 2, 1024, 0}, {"ddpp", 1, 128, 0}, {"ddds", 16, 1024, 0}, {"dddp", 4, 1024, 0},
+     {"dddd", 4, 512, 0}}};
+static const TileDefault kMergedTiles[2][CQ_NUM_CLASS_PAIRS] = {
+    {{"ssss", 4, 512, 1}, {"ssps", 4, 512, 1}, {"psps", 4, 1024, 1}, {"ppss", 8, 512, 1}, {"ppps", 4, 512, 1},
+     {"pppp", 3, 256, 1}, {"dsss", 16, 512, 1}, {"psds", 8, 512, 1}, {"ppds", 4, 512, 1}, {"dsds", 8, 256, 1},
+     {"dpss", 4, 128, 1}, {"dpps", 4, 512, 1}, {"dppp", 8, 512, 3}, {"dpds", 16, 256, 1}, {"dpdp", 8, 128, 3},
+     {"ddss", 1, 256, 1}, {"ddps", 1, 512, 1}, {"ddpp", 1, 512, 1}, {"ddds", 1, 512, 1}, {"dddp", 1, 512, 2},
+     {"dddd", 1, 256, 3}},
+    {{"ssss", 4, 512, 0}, {"ssps", 4, 1024, 0}, {"psps", 16, 1024, 0}, {"ppss", 16, 512, 0}, {"ppps", 2, 512, 0},
+     {"pppp", 16, 512, 0}, {"dsss", 16, 512, 0}, {"psds", 16, 512, 0}, {"ppds", 16, 256, 0}, {"dsds", 16, 512, 0},
+     {"dpss", 8, 256, 0}, {"dpps", 2, 1024, 0}, {"dppp", 8, 512, 0}, {"dpds", 16, 256, 0}, {"dpdp", 16, 256, 0},
+     {"ddss", 2, 1024, 0}, {"ddps", 2, 1024, 0}, {"ddpp", 1, 128, 0}, {"ddds", 16, 1024, 0}, {"dddp", 4, 1024, 0},
+     {"dddd", 4, 512, 0}}};
 
-// (one row per class pair, and one per merged orientation that differs)
-static_assert(sizeof(kTileDefaults) == sizeof(kTileDefaultsMulti), "the same class pairs in both tables");
-
-const TileDefault* tile_default(const cq_ctx* c, const ClassShape& ck) {
-  auto find = [&](const TileDefault* tab, size_t n) -> const TileDefault* {
-    for (size_t i = 0; i < n; ++i)
-      if (std::strcmp(tab[i].name, ck.name) == 0) return &tab[i];
-    return nullptr;
-  };
-  return c->nmol > 1 ? find(kTileDefaultsMulti, sizeof(kTileDefaultsMulti) / sizeof(TileDefault))
-                     : find(kTileDefaults, sizeof(kTileDefaults) / sizeof(TileDefault));
+// The built-in row of a class pair's own launch, or (merged) of its part of a merged launch.
+const TileDefault* tile_default(const cq_ctx* c, const ClassShape& ck, bool merged) {
+  const bool several = c->nmol > 1;
+  for (const TileDefault& t : merged ? kMergedTiles[several] : kTiles[several ? 2 : c->pairs.size() > kOwnTilePairs])
+    if (std::strcmp(t.name, ck.name) == 0) return &t;
+  return nullptr;
 }
 
-int default_union_bound(const cq_ctx* c, const ClassShape& ck, size_t jside) {
-  if (const TileDefault* t = tile_default(c, ck)) return t->ub;
+int default_union_bound(const cq_ctx* c, const ClassShape& ck, bool merged, size_t jside) {
+  if (const TileDefault* t = tile_default(c, ck, merged)) return t->ub;
   return (int)std::min<size_t>(UNION_MAX, std::max<size_t>(64, (16 * 1024) / (jside * sizeof(double)) / 64 * 64));
 }
 
 // Chunks per work item of class pair k in an orientation: the caller's choice, else the built-in
 // table's; always a divisor of the chunk count.
-int class_chunks_per_item(const cq_ctx* c, int k, const ClassShape& ck) {
+int class_chunks_per_item(const cq_ctx* c, int k, const ClassShape& ck, bool merged) {
   const int nch = ck.nchunk;
-  const TileDefault* t = tile_default(c, ck);
+  const TileDefault* t = tile_default(c, ck, merged);
   int d = c->class_cpi[k] > 0 ? std::min(c->class_cpi[k], nch) : (!t || t->cpi == 0) ? nch : std::min(t->cpi, nch);
   while (d > 1 && nch % d != 0) --d;
   return std::max(1, d);
 }
 
-void class_tile(const cq_ctx* c, int k, const ClassShape& ck, int variant, int& mmax, int& ub) {
+void class_tile(const cq_ctx* c, int k, const ClassShape& ck, bool merged, int variant, int& mmax, int& ub) {
   const size_t jside = variant == 2 ? (size_t)ck.nc * ck.nd : (size_t)ck.na * ck.nb;
-  ub = default_union_bound(c, ck, jside);
+  ub = default_union_bound(c, ck, merged, jside);
   if (c->tile_ub[k] > 0) ub = std::max(64, std::min(c->tile_ub[k], UNION_MAX));
   const size_t budget = c->tile_lds[k] > 0 ? (size_t)c->tile_lds[k] : (size_t)48 * 1024;
   const size_t limit = std::min(budget, c->max_dyn_lds);
   // a union bound whose J slots alone overflow the device's LDS is lowered (multiples of 64)
   while (ub > 64 && group_lds(c, ck, variant, 1, ub) > c->max_dyn_lds) ub -= 64;
   mmax = 0;
-  const TileDefault* t = tile_default(c, ck);
+  const TileDefault* t = tile_default(c, ck, merged);
   const int cap = c->tile_mmax[k] > 0 ? std::min(c->tile_mmax[k], MAX_GROUP) : (t ? t->max_group : 1);
   for (int mm = cap; mm >= 1; --mm)
     if (group_lds(c, ck, variant, mm, ub) <= limit) { mmax = mm; break; }
@@ -1257,7 +1275,7 @@ void plan_tasks(cq_ctx* c) {
     if (t != 1 || !ck.grp[0][2]) return t == 2 && ck.merged == 2;
     const long long nb = c->class_start[ck.bi + 1] - c->class_start[ck.bi], nk = c->class_start[ck.ki + 1] - c->class_start[ck.ki];
     int mm2 = 0, ub2 = 64;
-    class_tile(c, k, ck, 2, mm2, ub2);
+    class_tile(c, k, ck, false, 2, mm2, ub2);
     return ck.i != ck.j && mm2 > 0 && 2 * nb <= nk;
   };
   for (int t = 0; t < 3; ++t) {
@@ -1307,8 +1325,8 @@ void plan_tasks(cq_ctx* c) {
       mc = m;
       mc.flip = bra_keyed(k, t);
       int mmax = 0, ub = 64;
-      class_tile(c, k, sh, mc.flip ? 2 : 1, mmax, ub);
-      if (!mc.flip && mmax == 0 && t < 2) class_tile(c, k, sh, 0, mmax, ub);   // K columns do not fit: HBM K atomics
+      class_tile(c, k, sh, t == 2, mc.flip ? 2 : 1, mmax, ub);
+      if (!mc.flip && mmax == 0 && t < 2) class_tile(c, k, sh, false, 0, mmax, ub);   // K columns do not fit: HBM K atomics
       if (mmax == 0 && t < 2) throw std::invalid_argument(std::string("class pair ") + ck.name + ": no tile fits the device's LDS");
       mc.mmax = mmax;
       mc.ub = ub;
@@ -2153,7 +2171,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
       MergedEntry& e = ma.e[ma.n++];
       e.k = k;
       e.blk0 = nblk;
-      e.cpi = class_chunks_per_item(c, k, ck.mrg);
+      e.cpi = class_chunks_per_item(c, k, ck.mrg, true);
       e.nblk = (int)std::max<long long>(1, std::min<long long>(persistent_grid() / 4, m.seg_cap * (ck.mrg.nchunk / e.cpi)));
       nblk += e.nblk;
       e.nres = c->batch_slots[2][k][0];
@@ -2250,7 +2268,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
       JKArgs jkk = jk;   // the LDS rows of this class pair's swept side
       jkk.lds_n = lds_rows(c, ck, kv);
       jkk.rowfn = c->d_rowfn.p + (size_t)(kv == 2 ? ck.ki : ck.bi) * c->ncart;
-      const int cpi = class_chunks_per_item(c, k, ck);
+      const int cpi = class_chunks_per_item(c, k, ck, false);
       unsigned* wq = c->d_work_q.p + ((size_t)s0 * kNumClassPairs + k) * WORK_QUEUES;
       // batches of groups, in order on this class pair's stream: a class pair in one batch
       // screens once and keeps its lists for every slot pass; a batched one clears its counters

@@ -68,3 +68,19 @@ def test_plans_that_no_launch_uses_reserve_nothing():
     print(f"[plans] context {used / 2**30:.2f} GiB, task lists {entries * 8 / 2**30:.2f} GiB, {batches} batches", flush=True)
     assert batches > 1
     assert used - 8 * entries < 8 * entries / 20
+
+
+@pytest.mark.parametrize("m,tile", [(4, (4, 256)), (24, (16, 512))])
+def test_own_launches_keep_their_tiles(m, tile):
+    """A class pair's own launch has rows of its own up to 20000 shell pairs (many small items), the
+    merged launches' rows above: (ss|ds) of (H2O)4 and (H2O)24 in cc-pVDZ, on either side of the line."""
+    L = _lib.load()
+    ls = [ctypes.c_int() for _ in range(4)]
+    ssds = None
+    for k in range(L.cq_num_class_pairs()):
+        L.cq_class_pair_info(k, *[ctypes.byref(x) for x in ls])
+        if [x.value for x in ls] == [0, 0, 2, 0]:
+            ssds = k
+    ao = AOIntegrals(_water(m, "cc-pvdz"))
+    assert (ao.nShellPair > 20000) == (m == 24)
+    assert ao.class_tile(ssds)[:2] == tile
