@@ -125,32 +125,59 @@ class AOIntegrals:
         allows them.  Tiles (max_group, union_bound) as in set_class_tile, (0, 0) being the
         built-in default.  Every (tile, variant) runs `reps` times with the class kernels
         serialised and timed by HIP events (cq_get_kernel_times + cq_get_screen_times: the
-        screening is part of the cost); the fastest is set per class pair
-        (cq_set_class_tile, cq_set_class_digestion).  With balance_streams the class pairs are
-        then placed on the four streams longest first, each on the stream with the least
-        kernel time so far (cq_set_class_stream); off by default, since the serialised times
-        do not model the streams' overlap: on (H2O)16/cc-pVDZ the balanced placement ran
-        G[D] in 4.17 ms against 4.04 ms for the built-in round robin.  Returns
+        screening is part of the cost), which gives every class pair its fastest.  Class pairs
+        of variant 2 share merged launches, which the serialised times do not show: so whole
+        contractions are timed too, with the choices per class pair and, where 2 is among the
+        variants, with variant 2 and one tile for all ((0, 0) among them: the context as
+        created), and the fastest of these is set (cq_set_class_tile, cq_set_class_digestion).
+        On (H2O)16/cc-pVDZ the choices per class pair alone ran G[D] in 3.18 ms against 2.57 ms
+        for the defaults.  With balance_streams the choices per class pair are placed on the
+        four streams longest first, each on the stream with the least kernel time so far
+        (cq_set_class_stream; their class pairs then run in launches of their own); off by
+        default, since the serialised times do not model the streams' overlap.  Returns
         {class name: (variant, tile, {(tile, variant): mean ms})}.  No reference counterpart."""
         import torch
         L = _lib.load()
         nc = L.cq_num_class_pairs()
-        tiles = list(tiles) if tiles is not None else list(self.DEFAULT_TILES)
+        tiles = [(int(g), int(u)) for g, u in (tiles if tiles is not None else self.DEFAULT_TILES)]
+        variants = [int(v) for v in variants]
         J = torch.zeros_like(X)
         K = torch.zeros_like(X)
-        times = {}
-        check(L.cq_set_launch_streams(self._h, 1), self._h)
+
+        def contract():
+            self.newTwoEContractDirect([X, X], [J, K], [COULOMB, EXCHANGE], [1.0, -0.5])
+
+        def set_tiles(chosen):
+            for k, tile in enumerate(chosen):
+                check(L.cq_set_class_tile(self._h, k, 0, *tile), self._h)
+
+        def set_launches(chosen, streams):
+            for k in range(nc):
+                check(L.cq_set_class_digestion(self._h, k, chosen[k]), self._h)
+                check(L.cq_set_class_stream(self._h, k, streams[k]), self._h)
+
+        def whole_ms():
+            contract()
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(reps):
+                contract()
+            e1.record()
+            e1.synchronize()
+            return e0.elapsed_time(e1) / reps
+
+        own = [-1] * nc   # (no stream of a class pair's own)
+        times, whole = {}, {}
         try:
             for tile in tiles:
-                for k in range(nc):
-                    check(L.cq_set_class_tile(self._h, k, 0, int(tile[0]), int(tile[1])), self._h)
+                set_tiles([tile] * nc)
+                check(L.cq_set_launch_streams(self._h, 1), self._h)
                 for v in variants:
-                    for k in range(nc):
-                        check(L.cq_set_class_digestion(self._h, k, int(v)), self._h)
-                    self.newTwoEContractDirect([X, X], [J, K], [COULOMB, EXCHANGE], [1.0, -0.5])
+                    set_launches([v] * nc, own)
+                    contract()
                     check(L.cq_set_profiling(self._h, 1), self._h)
                     for _ in range(reps):
-                        self.newTwoEContractDirect([X, X], [J, K], [COULOMB, EXCHANGE], [1.0, -0.5])
+                        contract()
                     ms = (ctypes.c_double * nc)()
                     nl = (ctypes.c_longlong * nc)()
                     sms = (ctypes.c_double * nc)()
@@ -158,26 +185,29 @@ class AOIntegrals:
                     check(L.cq_get_kernel_times(self._h, ms, nl, nc), self._h)
                     check(L.cq_get_screen_times(self._h, sms, snl, nc), self._h)
                     check(L.cq_set_profiling(self._h, 0), self._h)
-                    times[(tuple(tile), int(v))] = [(ms[k] / nl[k] if nl[k] else 0.0) +
-                                                    (sms[k] / snl[k] if snl[k] else 0.0) for k in range(nc)]
+                    times[(tile, v)] = [(ms[k] / nl[k] if nl[k] else 0.0) +
+                                        (sms[k] / snl[k] if snl[k] else 0.0) for k in range(nc)]
+                check(L.cq_set_launch_streams(self._h, 4), self._h)
+                if 2 in variants:
+                    set_launches([2] * nc, own)
+                    whole[tile] = whole_ms()
         finally:
             check(L.cq_set_launch_streams(self._h, 4), self._h)
+        best = [min(times, key=lambda tv: times[tv][k]) for k in range(nc)]   # (tile, variant)
+        streams = list(own)
+        if balance_streams:
+            load = [0.0] * 4
+            for k in sorted(range(nc), key=lambda k: -times[best[k]][k]):
+                streams[k] = min(range(4), key=lambda i: load[i])
+                load[streams[k]] += times[best[k]][k]
+        set_tiles([tile for tile, _ in best])
+        set_launches([v for _, v in best], streams)
+        if whole and min(whole.values()) < whole_ms():
+            best = [(min(whole, key=whole.get), 2)] * nc
+            set_tiles([tile for tile, _ in best])
+            set_launches([2] * nc, own)
         names = list(self.quartet_counts().keys())
-        out = {}
-        chosen_ms = []
-        for k in range(nc):
-            (tile, v) = min(times, key=lambda tv: times[tv][k])
-            check(L.cq_set_class_tile(self._h, k, 0, int(tile[0]), int(tile[1])), self._h)
-            check(L.cq_set_class_digestion(self._h, k, v), self._h)
-            out[names[k]] = (v, tile, {tv: times[tv][k] for tv in times})
-            chosen_ms.append(times[(tile, v)][k])
-        load = [0.0] * 4
-        for k in sorted(range(nc), key=lambda k: -chosen_ms[k]):
-            s = min(range(4), key=lambda i: load[i]) if balance_streams else -1
-            check(L.cq_set_class_stream(self._h, k, s), self._h)
-            if s >= 0:
-                load[s] += chosen_ms[k]
-        return out
+        return {names[k]: (v, tile, {tv: times[tv][k] for tv in times}) for k, (tile, v) in enumerate(best)}
 
     def set_class_tile(self, k: int, max_group: int = 0, union_bound: int = 0, lds_bytes: int = 0) -> None:
         """Tile of class pair k's digestion kernels (cq_set_class_tile): groups of up to

@@ -2124,9 +2124,9 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   // them all
   // merged launches (FP64, also the FP64 window of a mixed call; default settings): the class pairs
   // of a tier that run in one batch, per tier one merged launch on the tier's stream, per stream one
-  // screening launch before them.  Settings that address class pairs one by one (their variant or
-  // stream, profiling, the screening mode, one stream), class pairs in several batches and the FP32
-  // window keep a launch per class pair.  When the merged launches came in, (H2O)16/cc-pVDZ took
+  // screening launch before them.  Settings that address class pairs one by one (variant 0 or 1, a
+  // stream of their own, profiling, the screening mode, one stream), class pairs in several batches
+  // and the FP32 window keep a launch per class pair.  When the merged launches came in, (H2O)16/cc-pVDZ took
   // 3638 us with a launch per class pair and 3544 merged; smaller systems gain more
   // (choose_merge_blocks).  Mixed, threshold 1e-5: 3550 us with both windows apart, 3106 so.
   const bool can_merge = !fp32 && !profiling && c->n_streams == cq_ctx::kAux + 1 &&
@@ -2134,7 +2134,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   std::vector<char> merged(kNumClassPairs, 0);
   for (int k = 0; k < kNumClassPairs && can_merge; ++k) {
     const CPMeta& m = c->cps[2][k];
-    merged[k] = c->class_variant[k] < 0 && c->class_stream[k] < 0 && stream_of[k] >= 0 && m.ngrp > 0 &&
+    merged[k] = variant_of(k) == 2 && c->class_stream[k] < 0 && stream_of[k] >= 0 && m.ngrp > 0 &&
                 c->batch_start[2][k].size() == 2 && m.mmax >= 1 &&
                 group_lds(c, kClassKernels[k].mrg, m.flip ? 2 : 1, m.mmax, m.ub) <= c->max_dyn_lds;
   }

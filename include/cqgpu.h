@@ -154,9 +154,9 @@ int cq_set_lds_digestion(cq_ctx_t* ctx, int mode);
 
 /* Digestion variant of one class pair k (0 .. cq_num_class_pairs()-1): 0, 1 or 2 as in
  * cq_set_lds_digestion (capped by the context's mode), -1 to follow the context's mode.  A class
- * pair with a choice of its own (here or in cq_set_class_stream) has a launch of its own; the
- * others share a few merged launches, except with profiling, fewer than four streams, another
- * screening or digestion mode than the default, and in the FP32 window.  Lets
+ * pair of variant 0 or 1, or with a stream of its own (cq_set_class_stream), has a launch of its
+ * own; the others share a few merged launches, except with profiling, fewer than four streams,
+ * another screening or digestion mode than the default, and in the FP32 window.  Lets
  * a tuner pick the fastest variant per class pair from cq_get_kernel_times; results agree to
  * rounding in every variant. */
 int cq_set_class_digestion(cq_ctx_t* ctx, int k, int mode);
