@@ -96,10 +96,11 @@ static const bool kClassKernelsReady = (cq_register_all(kClassKernels), cq_merge
 // held until the process ends; every call on a device shares it, so calls that overlap on one
 // device race.  Host code never uses the array's name as an address: the device address comes
 // from hipGetSymbolAddress, resolved once per device at context creation (scratch_address).
-// A call is accepted while 5 ncart^2 doubles per density (and a flag each) fit the limit; the
-// array also holds the two further copies of each density (at most 2 ncart^2).
+// A call is accepted while 5 ncart^2 doubles per density (and a flag each) fit the limit; a density
+// takes 5 ncart^2 + 2 njel of them (DensityWork), njel <= (ncart^2 + 6 ncart) / 2: a fifth more, and 6
+// ncart doubles, at most 176 KiB over a call's densities.
 #define CQ_NOALLOC_SCRATCH_BYTES (64ull << 20)
-static __device__ __align__(256) double scratch[CQ_NOALLOC_SCRATCH_BYTES / 5 * 7 / sizeof(double) + 512];
+static __device__ __align__(256) double scratch[CQ_NOALLOC_SCRATCH_BYTES / 5 * 6 / sizeof(double) + 32768];
 
 static std::mutex g_scratch_mu;
 static std::vector<double*> g_scratch_ptr;   // by device id; null until resolved
@@ -1932,6 +1933,24 @@ struct Slot {
   int do_j = 0, do_k = 0;
 };
 
+// One density slot's part of the workspace: the density's three copies and its accumulators, those
+// in pair order (njel elements, about half a matrix) without the other half.
+struct DensityWork {
+  double *D, *Dt, *Dp, *GJ, *GJ2, *GK, *GK2;
+  DensityWork(double* p, size_t nc2, size_t njel)
+      : D(p), Dt(D + nc2), Dp(Dt + nc2), GJ(Dp + njel), GJ2(GJ + njel), GK(GJ2 + nc2), GK2(GK + nc2) {}
+  static size_t words(size_t nc2, size_t njel) { return 5 * nc2 + 2 * njel; }
+  void set(JKArgs& jk) const {
+    jk.D[0] = D;
+    jk.Dt[0] = Dt;
+    jk.Dp[0] = Dp;
+    jk.GJ[0] = GJ;
+    jk.GJ2[0] = GJ2;
+    jk.GK[0] = GK;
+    jk.GK2[0] = GK2;
+  }
+};
+
 // The contraction on device-resident X/AX (column-major, leading dimension ld).
 // With noalloc, the per-call workspace is the device's static scratch array (nothing is
 // allocated: a call whose workspace exceeds it is rejected) and no profiling events are recorded.
@@ -1964,8 +1983,8 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   const int ns = c->nshell;
   const long nc2 = (long)c->ncart * c->ncart;
   const int nslot = (int)slots.size();
-  // workspace: per slot Dc, GJ, GJ2, GK, GK2, Dt (ncart^2 each) and Dp, then one flag per slot
-  const size_t slot_words = 6 * (size_t)nc2 + c->njel;
+  // workspace: the slots one after another, then one flag per slot
+  const size_t slot_words = DensityWork::words(nc2, c->njel);
   const size_t work_words = (size_t)std::max(1, nslot) * slot_words;
   double* work = nullptr;
   int* flags = nullptr;
@@ -1997,7 +2016,10 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   zero(c->d_work_q.p, (size_t)kNumClassPairs * MAX_MATS * WORK_QUEUES * sizeof(unsigned));
   zero(c->d_ovf.p, kNumClassPairs * sizeof(unsigned));
   // (every slot's accumulators; its density copies are rewritten below)
-  for (int k = 0; k < nslot; ++k) zero(work + k * slot_words + nc2, 4 * (size_t)nc2 * sizeof(double));
+  for (int k = 0; k < nslot; ++k) {
+    const DensityWork w(work + k * slot_words, nc2, c->njel);
+    zero(w.GJ, (3 * (size_t)nc2 + c->njel) * sizeof(double));
+  }
   const int zgrid = (int)std::min<long>(1024, grid_for(std::max<long>(8 * nc2, 64 * kNumClassPairs), WG));
   hipLaunchKernelGGL(zero_kernel, dim3(zgrid), dim3(WG), 0, s, zl);
   HIPCHK(hipGetLastError());
@@ -2011,12 +2033,12 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   if (nslot == 0) return;
   // 3. Cartesian densities and symmetry flags (with the first density, the shell pairs' own norms)
   for (int k = 0; k < nslot; ++k) {
-    double* base = work + (size_t)k * slot_words;
+    const DensityWork w(work + (size_t)k * slot_words, nc2, c->njel);
     const int np = k == 0 ? (int)c->pairs.size() : 0;
     hipLaunchKernelGGL(cart_density_kernel, dim3(grid_for(std::max<long>(nc2 + c->njel + np, (long)n * n), WG)), dim3(WG), 0, s,
                        slots[k].X, n, ld, c->d_shells.p, c->d_cart2shell.p, c->ncart, c->d_tco.p, c->d_tco_off.p,
-                       c->d_nglob.p + 1 + (std::find(uniq.begin(), uniq.end(), slots[k].X) - uniq.begin()), base,
-                       base + 5 * nc2, base + 6 * nc2, c->d_jel.p, (long)c->njel, flags + k, c->d_s12.p, np,
+                       c->d_nglob.p + 1 + (std::find(uniq.begin(), uniq.end(), slots[k].X) - uniq.begin()), w.D,
+                       w.Dt, w.Dp, c->d_jel.p, (long)c->njel, flags + k, c->d_s12.p, np,
                        c->d_Nmax.p, ns, c->d_Npair.p);
     HIPCHK(hipGetLastError());
   }
@@ -2188,13 +2210,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
     JKArgs jk{};
     jk.ncart = c->ncart;
     jk.rowfn = c->d_rowfn.p;
-    jk.D[0] = work;
-    jk.GJ[0] = work + nc2;
-    jk.GJ2[0] = work + 2 * nc2;
-    jk.GK[0] = work + 3 * nc2;
-    jk.GK2[0] = work + 4 * nc2;
-    jk.Dt[0] = work + 5 * nc2;
-    jk.Dp[0] = work + 6 * nc2;
+    DensityWork(work, nc2, c->njel).set(jk);
     jk.nonsym = flags;
     jk.pblk = c->mpblk;
     jk.ublk = c->mublk;
@@ -2235,14 +2251,7 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   for (int s0 = 0; s0 < nslot; ++s0) {
     JKArgs jk{};
     jk.ncart = c->ncart;
-    double* base = work + (size_t)s0 * slot_words;
-    jk.D[0] = base;
-    jk.Dt[0] = base + 5 * nc2;
-    jk.Dp[0] = base + 6 * nc2;
-    jk.GJ[0] = base + nc2;
-    jk.GJ2[0] = base + 2 * nc2;
-    jk.GK[0] = base + 3 * nc2;
-    jk.GK2[0] = base + 4 * nc2;
+    DensityWork(work + (size_t)s0 * slot_words, nc2, c->njel).set(jk);
     jk.do_j[0] = slots[s0].do_j;
     jk.do_k[0] = slots[s0].do_k;
     jk.nonsym = flags + s0;
@@ -2331,11 +2340,11 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   for (int i = 0; i < nmat; ++i) {
     const int k = mat_slot[i];
     if (k < 0) continue;
-    double* base = work + (size_t)k * slot_words;
+    const DensityWork w(work + (size_t)k * slot_words, nc2, c->njel);
     fl.AX[fl.n] = AX[i];
     fl.coulomb[fl.n] = types[i] == CQ_COULOMB;
-    fl.A[fl.n] = base + (types[i] == CQ_COULOMB ? 1 : 3) * nc2;
-    fl.B[fl.n] = base + (types[i] == CQ_COULOMB ? 2 : 4) * nc2;
+    fl.A[fl.n] = types[i] == CQ_COULOMB ? w.GJ : w.GK;
+    fl.B[fl.n] = types[i] == CQ_COULOMB ? w.GJ2 : w.GK2;
     fl.nonsym[fl.n] = flags + k;
     fl.f[fl.n] = 0.5 * scales[i];
     ++fl.n;

@@ -84,3 +84,27 @@ def test_own_launches_keep_their_tiles(m, tile):
     ao = AOIntegrals(_water(m, "cc-pvdz"))
     assert (ao.nShellPair > 20000) == (m == 24)
     assert ao.class_tile(ssds)[:2] == tile
+
+
+def test_workspace_of_a_contraction():
+    """What the first contraction of eight densities adds to a context (the least of four equal ones: the
+    runtime's own first allocations for the kernels come on top in the first): per density three
+    matrices of accumulators, the density and its transpose, and two lists in pair order of at most half
+    a matrix each (njel <= (ncart^2 + 6 ncart) / 2 elements), and 4 MiB for the flags and the pages."""
+    import torch
+    bs = _water(40, "cc-pvdz")
+    used = []
+    for _ in range(4):
+        ao = AOIntegrals(bs)
+        ao.thresholdSchwartz = 1e-12
+        nc = ao.nCart
+        X = [torch.zeros((ao.nBasis, ao.nBasis), dtype=torch.float64, device="cuda").fill_diagonal_(1.0 + i) for i in range(8)]
+        AX = [torch.zeros_like(x) for x in X]
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        ao.newTwoEContractDirect(X, AX, [EXCHANGE] * 8, [-0.5] * 8)
+        torch.cuda.synchronize()
+        used.append(free - torch.cuda.mem_get_info()[0])
+        ao.close()
+    print(f"[plans] workspace {min(used) / 2**20:.1f} MiB, {min(used) / (8 * 8 * nc * nc):.2f} matrices a density", flush=True)
+    assert 0 < min(used) <= 8 * 8 * (6 * nc * nc + 6 * nc) + (4 << 20)
