@@ -1,8 +1,9 @@
 """GPU: the class pairs of a call in a few merged launches (the default of an FP64 call) against the
 oracle and against a launch per class pair, where the two can differ: one and two shells, class
-pairs without a partner class, the limits between the primitive-block sizes, both keyed sides, open
-shell, a non-symmetric density, class pairs of both kinds in one call, task lists in several batches,
-and several molecules; and the one-electron kernel at the edges of its 64-pair workgroups."""
+pairs without a partner class, the three sizes of primitive blocks, both keyed sides, open shell, a
+non-symmetric density, class pairs of both kinds in one call, task lists in several batches, and
+several molecules; and the one-electron kernel at the edges of its 64-pair workgroups.  (The shipped
+bases hold d as pure shells: Cartesian ones are in test_gpu_shell_forms.py.)"""
 import numpy as np
 import pytest
 
@@ -29,9 +30,9 @@ SYSTEMS = {
     "H/6-31g": (lambda: _atoms(1), "6-31g"),            # (ss|ss) alone
     "Ne/6-31g": (lambda: _atoms(10), "6-31g"),          # no d class
     "NeH/cc-pvdz": (lambda: _atoms(10, 1), "cc-pvdz"),  # every class, few pairs
-    "H2O 4/6-31g": (lambda: _water(4), "6-31g"),        # more than 300 pairs, (pp) against (ss) bra-keyed
+    "H2O 4/6-31g": (lambda: _water(4), "6-31g"),        # more than 300 pairs, (ss) the ket of (pp)
     "H2O 4/cc-pvdz": (lambda: _water(4), "cc-pvdz"),
-    "H2O 9/6-31g": (lambda: _water(9), "6-31g"),        # Cartesian order of a few hundred functions
+    "H2O 9/6-31g": (lambda: _water(9), "6-31g"),        # 117 functions, several groups a class
 }
 
 
@@ -139,3 +140,32 @@ def test_schwarz_bounds_lane_groups(name, basis):
     Q, want = AOIntegrals(bs).computeSchwartz(), oracle.OracleBasis(bs).schwarz()
     assert np.abs(Q - Q.T).max() == 0.0
     assert np.abs(Q - want).max() <= 1e-12 * max(1.0, want.max())
+
+
+@pytest.mark.parametrize("name,basis,m", [("more than 6000 pairs", "cc-pvdz", 11), ("up to 6000", "6-31g*", 8)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_merged_launches_by_primitive_blocks(name, basis, m, symmetric):
+    """On either side of the line to the largest primitive blocks (the merged launches then share the
+    orders and block counts of the launches per class pair): two densities in merged launches, a launch per
+    class pair, and with the large class pairs in several batches beside merged ones."""
+    print(f"[merged] {name} symmetric={symmetric}", flush=True)
+    L = _lib.load()
+    mol = _water(m)
+    bs = B.build_basis(basis, mol.Z, mol.coords_bohr)
+    ao = AOIntegrals(bs)
+    assert (ao.nShellPair > 6000) == (m == 11)
+    A, C = _matrices(bs.nbasis, 41, symmetric)
+    Xs, types, scales = [A, A, C], [COULOMB, EXCHANGE, EXCHANGE], [1.0, -0.5, 0.25]
+    _lib.check(L.cq_set_launch_streams(ao._h, 1), ao._h)
+    want, n = _contract(ao, Xs, types, scales)
+    _lib.check(L.cq_set_launch_streams(ao._h, 4), ao._h)
+    entries, batches = ao.task_plan()
+    assert batches == 1 and n > 0
+    for budget in (None, entries // 40):
+        if budget:
+            ao.set_task_budget(budget)
+            assert ao.task_plan()[1] > 1
+        got, k = _contract(ao, Xs, types, scales)
+        assert k == n
+        for g, w in zip(got, want):
+            assert np.abs(g - w).max() < TOL

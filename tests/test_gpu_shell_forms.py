@@ -20,6 +20,8 @@ TOL = 1e-10
 FORMS = {
     "pure s and p": lambda i, l: True,
     "every other p pure": lambda i, l: l > 1 or (l == 1 and i % 2 == 0),
+    "Cartesian d": lambda i, l: False,
+    "every other p and d pure": lambda i, l: i % 2 == 0,
 }
 
 
