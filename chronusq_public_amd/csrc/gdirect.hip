@@ -1439,10 +1439,14 @@ void plan_tasks(cq_ctx* c) {
 // np_max primitive pairs each.  Few quartets leave most of the device idle, and then the longest
 // lane task (block x block primitive quartets in series) sets the time: smaller blocks.  More
 // quartets fill the device, and every block more digests its quartet once more.
-// Measured (before the tiles of today), G[D] in us with blocks (lane, uniform) 2,8 / 4,8 / 8,32:
-//   H2O/6-31G* (55 pairs) 243 / 286 / 412, O2/cc-pVDZ UHF (78) 255 / 302 / 543,
-//   (H2O)4/cc-pVDZ (1176) 548 / 496 / 598, (H2O)11/6-31G UHF (4851) 809 / 772 / 783,
-//   C12H26/6-31G* (7750) 2354 / 2121 / 2064, (H2O)16/cc-pVDZ (18528) 4116 / 3632 / 3544.
+// Measured, G[D] in us with blocks (lane, uniform) 2,8 / 4,8 / 8,32, by pairs in the two-electron list:
+//   H2O/6-31G* (55) 214 / 237 / 340, O2/cc-pVDZ UHF (78) 286 / 317 / 455, (H2O)2/cc-pVDZ (300) 256 / 281 / 369,
+//   (H2O)3/cc-pVDZ (632) 319 / 302 / 406, (H2O)4/cc-pVDZ (1172) 565 / 563 / 589, C6H14/cc-pVDZ (2999)
+//   1466 / 1253 / 1360, (H2O)11/6-31G UHF (3634) 787 / 741 / 770, C12H26/6-31G* (5812) 1971 / 1766 / 1684,
+//   (H2O)11/cc-pVDZ (6324) 1575 / 1447 / 1622, (H2O)20/6-31G (9276) 1144 / 1056 / 1150, (H2O)16/cc-pVDZ
+//   (11990) 3643 / 3260 / 3174.
+// Between 5000 and 10000 pairs their number alone does not tell: chains prefer 8,32 there and
+// clusters 4,8, each by 5 to 11 %.
 void choose_merge_blocks(cq_ctx* c, int npair, int np_max) {
   c->mpblk = npair <= 300 ? 2 : npair <= 6000 ? 4 : PRIM_BLOCK;
   c->mublk = npair <= 6000 ? 8 : UNI_BLOCK;
@@ -2113,7 +2117,10 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   // round robin in launch order (highest angular momentum first: the latency-bound kernels
   // start early) over the class pairs that have work; the last, incomplete round runs from the
   // last stream down, so its (lowest angular momentum, longest) kernels do not all land on the
-  // streams that already hold one kernel more ((H2O)16/cc-pVDZ: 21 class pairs, 4.11 -> 4.03 ms)
+  // streams that already hold one kernel more ((H2O)16/cc-pVDZ, all 21 class pairs in launches of
+  // their own: 4.11 -> 4.03 ms).  Class pairs that merge below keep their place in this round: those
+  // left over ((H2O)64: the ones in several batches, (ss|ps) and (ss|ss) both on the last stream)
+  // dealt evenly over the streams took 75.3 ms, as dealt here 75.2.
   int stream_of[kNumClassPairs];
   {
     int nwork = 0;

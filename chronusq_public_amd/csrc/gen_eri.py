@@ -12,7 +12,7 @@ Two kernels are instantiated per class from the generated core:
   * eri_block_<cls>: writes the contracted Cartesian block (ab|cd) of each task (used for
     Schwarz bounds and for per-quartet parity tests);
   * eri_grp_<cls> / eri_grpb_<cls>: digest the block into the J/K accumulators.
-A merged kernel per tier runs several class pairs in one launch (small molecules).
+A merged kernel per tier runs several class pairs in one launch (the default of an FP64 call).
 
 The algorithm restated here replaces libint2::Engine::compute as called at
 include/aointegrals/aointegrals_contract.h:138-143; the digestion reproduces the scatter at
@@ -486,8 +486,6 @@ def gen_digest_chunk(em: Emitter, NA, NB, NC, ND, ks, persist):
         return (f"R(DIG == 2 ? row_at(D + (long)(q.{r0} + {ri}) * N, 8u * (unsigned)q.{c0} + {8 * ci}u) : "
                 f"row_at(Dt + (long)(q.{c0} + {ci}) * N, 8u * (unsigned)q.{r0} + {8 * ri}u))")
 
-    NCOL = NC + ND
-
     def kadd(G, trans, row0, ri, colkind, ci, val):
         """One K update: row (row0 + ri), column c0 + ci (colkind 'c') or d0 + ci ('d')."""
         col0 = "q.c0" if colkind == "c" else "q.d0"
@@ -568,7 +566,6 @@ def gen_digest_chunk(em: Emitter, NA, NB, NC, ND, ks, persist):
 
 
 def gen_digest_final(em: Emitter, NA, NB, NC, ND):
-    NCOL = NC + ND
     em("#pragma unroll")
     em("for (int s = 0; s < NSLOT; ++s) {")
     em.ind += 1
