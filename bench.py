@@ -329,7 +329,7 @@ def main():
     torch.cuda.synchronize()
     L = _lib.load()
     ncp = L.cq_num_class_pairs()
-    # timed region: the production configuration (class kernels over 4 streams)
+    # timed region: the production configuration (merged launches over 4 streams)
     e0 = torch.cuda.Event(enable_timing=True)
     e1 = torch.cuda.Event(enable_timing=True)
     torch.cuda.synchronize()
@@ -341,7 +341,7 @@ def main():
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     ms_per_step = e0.elapsed_time(e1) / args.steps
-    # per-kernel pass: kernels serialised on one stream, HIP events around each launch
+    # per-kernel pass: a launch per class pair, serialised on one stream, HIP events around each
     _lib.check(L.cq_set_launch_streams(ao._h, 1), ao._h)
     _lib.check(L.cq_set_profiling(ao._h, 1), ao._h)
     for _ in range(args.steps):
@@ -358,7 +358,7 @@ def main():
     _lib.check(L.cq_set_launch_streams(ao._h, 4), ao._h)
     counts = ao.quartet_counts()
     nquart = sum(counts.values())
-    # per-class digestion variants picked by the autotuner (timed once, then the same K steps)
+    # digestion variants and tiles picked by the autotuner (timed once, then the same K steps)
     autotuned = None
     if not args.no_autotune:
         autotuned = run_autotuned(bs, args, dD, dJ, dK, stream, nquart, e0, e1)
@@ -407,7 +407,10 @@ def main():
                    "all_kernels_tflops": total_flops / (sum(r["kernel_ms"] for r in per_class) * 1e-3) / 1e12,
                    "step_tflops": total_flops / (ms_per_step * 1e-3) / 1e12},
         "roofline": {"bound": "fp64-valu",
-                     "pipe": "FP64 vector ALU (no ERI kernel issues MFMA; the FP64 vector peak is 78.6 TFLOP/s)",
+                     "pipe": "FP64 vector ALU (the matrix cores only sum J over a wavefront's lanes; the FP64 vector "
+                             "and matrix peaks are both 78.6 TFLOP/s)",
+                     "note": "this kernel, classes and serial_*: a launch per class pair, serialised; the timed "
+                             "steps run the same class pairs in merged launches (step_tflops is theirs)",
                      "kernel": "eri_grp" + dom["class"], "achieved": achieved,
                      "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": achieved / FP64_PEAK_TFLOPS,
                      "traffic": traffic, "traffic_source": traffic_src,

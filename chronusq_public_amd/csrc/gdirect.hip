@@ -2155,9 +2155,9 @@ void contract_device(cq_ctx* c, int nmat, const double* const* X, double* const*
   // of a tier that run in one batch, per tier one merged launch on the tier's stream, per stream one
   // screening launch before them.  Settings that address class pairs one by one (variant 0 or 1, a
   // stream of their own, profiling, the screening mode, one stream), class pairs in several batches
-  // and the FP32 window keep a launch per class pair.  When the merged launches came in, (H2O)16/cc-pVDZ took
-  // 3638 us with a launch per class pair and 3544 merged; smaller systems gain more
-  // (choose_merge_blocks).  Mixed, threshold 1e-5: 3550 us with both windows apart, 3106 so.
+  // and the FP32 window keep a launch per class pair.  (H2O)16/cc-pVDZ takes
+  // 3530 us with a launch per class pair and 3190 merged, C12H26/6-31G* 2120 and 1770, (H2O)11/6-31G open
+  // shell 1065 and 750, one water 590 and 240.  Mixed, threshold 1e-5: 3690 us with both windows apart, 3230 so.
   const bool can_merge = !fp32 && !profiling && c->n_streams == cq_ctx::kAux + 1 &&
                          c->screen_mode == CQ_SCREEN_PER_STREAM && c->lds_mode == 2;
   std::vector<char> merged(kNumClassPairs, 0);
@@ -2814,7 +2814,8 @@ int cq_set_class_tile(cq_ctx_t* c, int k, long long lds_bytes, int max_group, in
 
 // The planned tile of class pair k in the digestion table of the given variant (0/1: ket-keyed,
 // 2: bra-keyed where the class pair has that form): largest group, union bound, number of
-// groups, and the kernel's dynamic LDS bytes.
+// groups, and the kernel's dynamic LDS bytes.  These are the launches of a class pair's own; the
+// merged table is not reported.
 int cq_get_class_tile(const cq_ctx_t* c, int k, int variant, int* max_group, int* union_bound, int* ngroups,
                       long long* lds_bytes) {
   if (!c || k < 0 || k >= kNumClassPairs || variant < 0 || variant > 2 || !max_group || !union_bound || !ngroups ||
@@ -2831,7 +2832,7 @@ int cq_get_class_tile(const cq_ctx_t* c, int k, int variant, int* max_group, int
 }
 
 // Task entries allocated over all class pairs, and the largest number of batches any class
-// pair takes (over both digestion tables).
+// pair takes (over both digestion tables; in the merged table a class pair has one batch or none).
 int cq_get_task_plan(const cq_ctx_t* c, long long* entries, int* max_batches) {
   if (!c || !entries || !max_batches) return CQ_ERR_INVALID;
   *entries = c->task_capacity;

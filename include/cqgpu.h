@@ -189,8 +189,9 @@ int cq_set_launch_streams(cq_ctx_t* ctx, int n);
  * whatever the system size.  Waits for the context's work and reallocates.  Results agree to
  * rounding for every budget. */
 int cq_set_task_budget(cq_ctx_t* ctx, long long entries);
-/* Task entries allocated over all class pairs, and the largest number of batches a class pair
- * takes. */
+/* Task entries allocated over all class pairs (each the largest of its plans), and the largest
+ * number of batches a class pair takes in a launch of its own (a class pair that needs more than
+ * one has such a launch). */
 int cq_get_task_plan(const cq_ctx_t* ctx, long long* entries, int* max_batches);
 
 /* Tile of class pair k's digestion kernels (no reference counterpart; set by the autotuner).
@@ -203,8 +204,10 @@ int cq_get_task_plan(const cq_ctx_t* ctx, long long* entries, int* max_batches);
  * class pair's built-in bound).  Waits for the context's work and re-plans.  Results agree to
  * rounding for every tile. */
 int cq_set_class_tile(cq_ctx_t* ctx, int k, long long lds_bytes, int max_group, int union_bound);
-/* The planned tile for digestion variant 0/1 (ket-keyed) or 2 (bra-keyed): largest group, union
- * bound, number of groups, dynamic LDS bytes of the kernel. */
+/* The planned tile of class pair k's own launch for digestion variant 0/1 (ket-keyed) or 2
+ * (bra-keyed): largest group, union bound, number of groups, dynamic LDS bytes of the kernel.  (The
+ * merged launches have a built-in tile of their own, which is not reported; a tile set by the
+ * caller holds for both.) */
 int cq_get_class_tile(const cq_ctx_t* ctx, int k, int variant, int* max_group, int* union_bound, int* ngroups,
                       long long* lds_bytes);
 
